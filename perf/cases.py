@@ -240,6 +240,7 @@ def prepare(case, seed):
         own = _between(case, B, case["own_lo"], case["own_hi"])
         st["k"], st["v"], slots = _pools(gen, groups * case["prefix"] + sum(own), H, D, dtype)
         lists = _cuts(slots, [case["prefix"]] * groups + own)
+        st["prefix_lists"], st["own_lists"] = lists[:groups], lists[groups:]
         st["tables"] = kernels.DecodeTables.build(lists[:groups], [g * (B // groups) for g in range(groups + 1)],
                                                   lists[groups:], _dev(), num_heads=H, head_dim=D, dtype=dtype)
         if kind == "decode":
@@ -266,7 +267,8 @@ def prepare(case, seed):
         ctx = [case["parent"] + n for n in new]
         st["k"], st["v"], slots = _pools(gen, sum(ctx), H, D, dtype)
         st["q"] = _randn(gen, (sum(new), H, D), dtype)
-        st["tables"] = kernels.PrefillTables.build(new, _cuts(slots, ctx), _dev())
+        st["new_lens"], st["contexts"] = new, _cuts(slots, ctx)
+        st["tables"] = kernels.PrefillTables.build(new, st["contexts"], _dev())
     elif kind == "ops":
         T = case["tokens"]
         st["k"], st["v"], st["new_slots"] = _pools(gen, T, H, D, dtype)
@@ -323,3 +325,106 @@ def run(st):
         kernels.discontinuous_move_tokens(st["src"], st["dst"], st["src_idx"], st["dst_idx"])
         return st["dst"]
     return kernels.sample_top_p(st["logits"], st["temperature"], st["top_p"], st["uniform"])
+
+
+# --------------------------------------------------------------------------- #
+# the same outputs in 64 bits, by plain torch
+# --------------------------------------------------------------------------- #
+def _attend64(q, keys, values, causal_from=None, scores_at_once=1 << 28):
+    """softmax(q k^T / sqrt(D)) v of `q` [n, H, D] over `keys`, `values` [m, G, D], query head h on KV head h * G // H.
+    `causal_from`: query i sees the keys 0 to causal_from + i."""
+    n, H, D = q.shape
+    out = torch.empty((n, H, D), dtype=torch.float64, device=q.device)
+    step = max(1, scores_at_once // keys.shape[0])
+    for h in range(H):
+        g = h * keys.shape[1] // H
+        kt, v = keys[:, g].double().t().contiguous(), values[:, g].double()
+        for at in range(0, n, step):
+            s = (q[at:at + step, h].double() / math.sqrt(D)) @ kt
+            if causal_from is not None:
+                last = causal_from + at + torch.arange(s.shape[0], device=s.device)
+                s.masked_fill_(torch.arange(s.shape[1], device=s.device)[None, :] > last[:, None], -math.inf)
+            out[at:at + step, h] = torch.softmax(s, dim=-1) @ v
+    return out
+
+
+def _decode64(q, k, v, prefix_lists, own_lists):
+    """Every request attends its group's prefix, then its own tokens; the groups hold equally many requests.  The requests
+    of a group share one product with the prefix, and the two parts are joined by their log-sum-exp."""
+    B, H, D = q.shape
+    G, per = k.shape[1], B // max(1, len(prefix_lists))
+    kv_head = torch.arange(H, device=q.device) * G // H
+    out = torch.empty((B, H, D), dtype=torch.float64, device=q.device)
+    q = q.double() / math.sqrt(D)
+
+    def index(slots):
+        return torch.as_tensor(slots, dtype=torch.int64, device=q.device)
+
+    prefix_lse = torch.full((B, H), -math.inf, dtype=torch.float64, device=q.device)
+    prefix_out = torch.zeros_like(out)
+    for g, slots in enumerate(prefix_lists):
+        rows = slice(g * per, (g + 1) * per)
+        keys, values = k[index(slots)], v[index(slots)]
+        for h in range(H):
+            s = q[rows, h] @ keys[:, kv_head[h]].double().t().contiguous()
+            prefix_lse[rows, h] = torch.logsumexp(s, dim=-1)
+            prefix_out[rows, h] = torch.softmax(s, dim=-1) @ values[:, kv_head[h]].double()
+    for b, slots in enumerate(own_lists):
+        keys = k[index(slots)].double()[:, kv_head]
+        s = (keys * q[b][None]).sum(-1)                                          # [n, H]
+        lse = torch.logsumexp(s, dim=0)
+        own = (torch.softmax(s, dim=0)[..., None] * v[index(slots)].double()[:, kv_head]).sum(0)
+        both = torch.logaddexp(prefix_lse[b], lse)
+        out[b] = torch.exp(prefix_lse[b] - both)[:, None] * prefix_out[b] + torch.exp(lse - both)[:, None] * own
+    return out
+
+
+def _layer64(st, attention):
+    D, eps = st["head_dim"], 1e-6
+    T, hidden = st["x"].shape
+
+    def norm(x, w):
+        return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps) * w.double()
+
+    q, k, v = (c.double().view(T, hidden // D, D) for c in torch.chunk(st["qkv"], 3, dim=-1))
+    cos, sin = st["cos_sin"][st["positions"]].double()[:, None].chunk(2, dim=-1)
+
+    def rotate(x):
+        a, b = x.chunk(2, dim=-1)
+        return torch.cat([a * cos - b * sin, b * cos + a * sin], dim=-1)
+
+    q, slots = rotate(q), st["new_slots"].long()
+    k_cache, v_cache = st["k"].double(), st["v"].double()
+    k_cache[slots], v_cache[slots] = rotate(k), v
+    out = {"normed": norm(st["x"].double(), st["w1"]), "q": q.reshape(T, hidden), "k_cache": k_cache, "v_cache": v_cache}
+    if attention:
+        out["attention"] = _decode64(q, k_cache, v_cache, st["prefix_lists"], st["own_lists"])
+    residual, gate = st["residual"].double() + st["delta"].double(), st["gate"].double()
+    out["post_norm"] = norm(residual, st["w2"])
+    out["residual"] = residual
+    out["activation"] = gate * torch.sigmoid(gate) * st["up"].double()
+    return out
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "sample":
+        return None  # whole numbers, drawn from a filter whose edge is a comparison of rounded sums
+    st = prepare(case, seed)
+    if kind in ("layer", "ops"):
+        return _layer64(st, kind == "layer")
+    if kind == "decode":
+        return _decode64(st["q"], st["k"], st["v"], st["prefix_lists"], st["own_lists"])
+    if kind in ("paged", "ragged"):
+        own = [row[:n] for row, n in zip(st["table"].long(), st["lens"].tolist())]
+        return _decode64(st["q"], st["k"], st["v"], [st["prefix_table"].long()] if kind == "paged" else [], own)
+    if kind == "prefill":
+        parts, at = [], 0
+        for n, slots in zip(st["new_lens"], st["contexts"]):
+            slots = torch.tensor(slots, dtype=torch.int64, device=_dev())
+            parts.append(_attend64(st["q"][at:at + n], st["k"][slots], st["v"][slots], causal_from=len(slots) - n))
+            at += n
+        return torch.cat(parts)
+    out = st["dst"].double()
+    out[st["dst_idx"]] = st["src"][st["src_idx"]].double()
+    return out
