@@ -423,9 +423,13 @@ int ph_prefix_post_attention(void* out, const float* prev_m, const float* prev_l
  * Query r of chunk c sees key j iff j <= r + (kv_len_c - q_len_c).
  * The new tokens' K/V must already be in the cache (append first).
  * max_kv_len: host upper bound of any chunk's context length.
- * workspace: at least ph_prefill_workspace_bytes(...) bytes, 256-byte aligned. */
+ * workspace: at least ph_prefill_workspace_min_bytes(...) bytes, 256-byte aligned.  With
+ * ph_prefill_workspace_bytes(...) every plan fits: few queries over long contexts are then cut into
+ * parts whose partial results live there. */
 size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
                                   int64_t max_kv_len);
+size_t ph_prefill_workspace_min_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
+                                      int64_t max_kv_len);
 
 int ph_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
                          int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim,

@@ -4,6 +4,7 @@
 #include "decode.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace ph {
@@ -393,6 +394,70 @@ static int run_prefix(PrefixArgs& pa, int dtype, int D, int num_groups, const in
     if (rc != PH_OK) return rc;
   }
   return PH_OK;
+}
+
+// Shape of a matrix-core prefill launch: queries per workgroup, and parts the visible tokens of every tile are cut into.
+struct PrefillPlan {
+  int tile_q, splits;
+};
+constexpr int kMaxPrefillSplits = 16;
+// most splits a launch of T query rows can take whatever its chunks: two rounds of workgroups
+static int64_t max_prefill_splits(int64_t T, int64_t H) {
+  const int64_t s = 2 * device_cus() / (cdiv(T, 256) * H);
+  return std::min<int64_t>(kMaxPrefillSplits, s);
+}
+static size_t prefill_part_bytes(int64_t T, int64_t H, int64_t D, int64_t splits) {
+  return (size_t)round_up(splits * T * H * D * 4, 256) + (size_t)round_up(splits * T * H * 2 * 4, 256);
+}
+// Estimated time of a launch (microseconds): rounds of one workgroup per compute unit, each a fixed start and end and
+// its steps, no faster than the K/V rows come from memory; a split launch adds the parts' write and fold.  The host
+// knows the query total, the chunk count and the longest context: tiles per chunk and visible lengths are averages.
+// Constants fitted to 27 shapes in bf16 (1 to 16 chunks of 16 to 4096 tokens over parents of 0 to 6000, 32 and 40
+// heads), every tile with 1 to 16 splits: the choice is within 8 % of the best form on 24 of them, 20 % on one.
+static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int tile_q, int64_t splits,
+                              int64_t cus) {
+  const double start = tile_q == 256 ? 9.0 : 8.5;
+  const double step = tile_q == 256 ? 1.46 : tile_q == 128 ? 0.96 : 1.16;  // on a lightly loaded device
+  const int64_t step_tokens = tile_q == 64 ? 128 : 64;
+  const double avg = (double)T / C, fill = avg / tile_q;
+  const double tiles = C == 1      ? (double)cdiv(T, tile_q)
+                       : fill > 1.0 ? T / (double)tile_q + 0.5 * C
+                                    : C * (1.0 + std::max(0.0, fill - 0.6));  // some chunks are longer than the average
+  const double wgs = tiles * H * splits;
+  const double rounds = std::ceil(wgs / cus - 1e-9);
+  const double step_loaded = step * (1.0 + 0.25 * std::min(1.0, wgs / (rounds * cus)));  // clock and memory under load
+  const double seen = std::max(1.0, max_kv - 0.5 * std::max(0.0, avg - tile_q));        // of an average tile
+  auto walk = [&](double tokens) { return start + std::ceil(tokens / step_tokens / splits) * step_loaded; };
+  double t = std::max(rounds * walk(seen), walk((double)max_kv));
+  const double kv_mb = (double)C * max_kv * H * D * 4 / 1e6;
+  t = std::max(t, start + kv_mb / 5.5);
+  if (splits > 1) t += 4.0 + (double)splits * T * H * D * 4 / 1e6 / 5.0;
+  return t;
+}
+
+// Query tile by the average chunk length: 256-query tiles share every K/V tile among all eight waves (least traffic,
+// deepest staging ring) but idle whole waves on short chunks, which take 128- or 64-query tiles.  That rule alone
+// holds for launches of more than four rounds of workgroups.  Below, the workgroups may not fill the device or end on
+// a short round: smaller tiles, and parts of long contexts on workgroups of their own, then go faster (bf16, one
+// chunk: 61 queries over 2048 tokens, 32 heads, 27.3 -> 18 us in 4 to 8 parts; 256 over 1256, 32 heads, 37.3 -> 19.2
+// us on 64-query tiles; 256 over 6256, 40 heads, 152 -> 58 us on 256-query tiles in 6 parts).
+static PrefillPlan plan_prefill(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, size_t workspace_bytes) {
+  const int64_t avg = T / C, cus = device_cus();
+  PrefillPlan p{avg >= 192 ? 256 : avg >= 96 ? 128 : 64, 1};
+  if (cdiv(T, p.tile_q) * H > 4 * cus || C * H > 4 * cus || C > kScanChunks) return p;
+  double best = prefill_cost_us(T, C, H, D, max_kv, p.tile_q, 1, cus);
+  const int64_t max_splits = std::min(max_prefill_splits(T, H), cdiv(max_kv, 128));
+  for (int64_t splits = 1; splits <= std::max<int64_t>(1, max_splits); ++splits) {
+    if (splits > 1 && prefill_part_bytes(T, H, D, splits) > workspace_bytes) break;
+    for (int tile_q = 256; tile_q >= 64; tile_q /= 2) {
+      const double t = prefill_cost_us(T, C, H, D, max_kv, tile_q, splits, cus);
+      if (t < 0.95 * best) {  // an estimate that is no clear gain changes nothing
+        best = t;
+        p = PrefillPlan{tile_q, (int)splits};
+      }
+    }
+  }
+  return p;
 }
 
 // Per-token (offset, length) of the prefill-as-ragged-decode formulation.
@@ -996,14 +1061,26 @@ extern "C" int ph_suffix_prev_attention(void* out, float* m_out, float* l_out, c
                       stream);
 }
 
-extern "C" size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
-                                             int64_t max_kv_len) {
+static bool prefill_on_matrix_cores(int dtype, int64_t D, int64_t H) {
+  return prefix_mfma_supported(dtype, (int)D) || (pair_heads(D, H) && prefix_mfma_supported(dtype, 128));
+}
+
+// smallest workspace a prefill call takes; with less than ph_prefill_workspace_bytes it splits fewer contexts
+extern "C" size_t ph_prefill_workspace_min_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
+                                                 int64_t max_kv_len) {
   if (num_tokens <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
+  if (prefill_on_matrix_cores(dtype, head_dim, num_heads)) return 256 + (size_t)round_up((num_tokens + 2) * 4, 256);
   const DecodePlan p = plan_decode(num_tokens, num_heads, 0, 0, max_kv_len, 0);
-  if (prefix_mfma_supported(dtype, (int)head_dim) || (pair_heads(head_dim, num_heads) && prefix_mfma_supported(dtype, 128)))
-    return 256 + (size_t)round_up((num_tokens + 2) * 4, 256);
   return (size_t)round_up(num_tokens * 8, 256) + (size_t)round_up(num_tokens * 4, 256) +
          plan_bytes(p, num_tokens, num_heads, head_dim);
+}
+
+extern "C" size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
+                                             int64_t max_kv_len) {
+  const size_t least = ph_prefill_workspace_min_bytes(num_tokens, num_heads, head_dim, dtype, max_kv_len);
+  if (least == 0 || !prefill_on_matrix_cores(dtype, head_dim, num_heads)) return least;
+  const int64_t splits = max_prefill_splits(num_tokens, num_heads);
+  return splits > 1 ? std::max(least, prefill_part_bytes(num_tokens, num_heads, head_dim, splits)) : least;
 }
 
 extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
@@ -1018,13 +1095,13 @@ extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cach
                         cache_stride_n);
   if (rc != PH_OK || num_tokens == 0) return rc;
   if (num_chunks <= 0 || max_kv_len <= 0 || max_kv_len > INT32_MAX || !q_cu || !kv_cu || !ctx_slots || ctx_slots_count <= 0) return PH_ERR_ARG;
-  if (ph_prefill_workspace_bytes(num_tokens, num_heads, head_dim, dtype, max_kv_len) > workspace_bytes || !workspace)
+  if (ph_prefill_workspace_min_bytes(num_tokens, num_heads, head_dim, dtype, max_kv_len) > workspace_bytes || !workspace)
     return PH_ERR_WORKSPACE;
   if (((uintptr_t)workspace & 255u) != 0) return PH_ERR_ALIGN;
   hipStream_t st = (hipStream_t)stream;
   const bool paired = pair_heads(D, H) && prefix_mfma_supported(dtype, 128);  // 64-wide heads as halves of head pairs
-  if (prefix_mfma_supported(dtype, D) || paired) {
-    if (num_chunks > num_tokens) return PH_ERR_ARG;  // every chunk holds at least one query (tile_cu fits the workspace)
+  if (prefill_on_matrix_cores(dtype, D, H)) {
+    if (num_chunks > num_tokens) return PH_ERR_ARG;  // every chunk holds at least one query
     PrefillArgs pa{};
     pa.q = (const uint16_t*)q;
     pa.q_stride = q_stride;
@@ -1036,12 +1113,21 @@ extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cach
     pa.q_cu = q_cu;
     pa.kv_cu = kv_cu;
     pa.ctx_slots = ctx_slots;
-    pa.tile_cu = (int32_t*)workspace;
+    pa.tile_cu = num_chunks > kScanChunks ? (int32_t*)workspace : nullptr;  // such a plan has no parts
+    pa.num_tokens = T;
     pa.num_chunks = (int)num_chunks;
     pa.H = H;
     pa.scale_log2e = scale * kLog2e;
     pa.pair = paired ? 1 : 0;
-    return launch_prefill_mfma(pa, dtype, paired ? 128 : D, num_tokens, st);
+    const PrefillPlan pp = plan_prefill(num_tokens, num_chunks, num_heads, head_dim, max_kv_len, workspace_bytes);
+    pa.n_splits = pp.splits;
+    if (pp.splits > 1) {
+      pa.opart = (float*)workspace;
+      pa.ml = (float*)((char*)workspace + round_up((int64_t)pp.splits * T * H * D * 4, 256));
+    }
+    rc = launch_prefill_mfma(pa, dtype, paired ? 128 : D, pp.tile_q, st);
+    if (rc != PH_OK || pp.splits == 1) return rc;
+    return launch_fold_parts(FoldArgs{pa.opart, pa.ml, pa.out, out_stride, pp.splits, T, H, D}, dtype, st);
   }
   int64_t* offsets = (int64_t*)workspace;
   int32_t* lens = (int32_t*)((char*)workspace + round_up(num_tokens * 8, 256));

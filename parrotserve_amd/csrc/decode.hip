@@ -203,6 +203,38 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
   }
 }
 
+// Folds the parts of a split prefill, [n_splits][rows][H] rows of D floats: a thread owns four dims of one (row, head)
+// and walks the parts, so every load and store of a wave is one contiguous run.
+template <typename E>
+__global__ __launch_bounds__(256) void fold_parts_kernel(FoldArgs a) {
+  const int dq = a.D >> 2;
+  const int64_t pairs = (int64_t)a.rows * a.H;  // (row, head) pairs of a part
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= pairs * dq) return;
+  const int64_t rh = i / dq;
+  const int d = (int)(i - rh * dq) * 4;
+  const float* op = a.opart + rh * a.D + d;
+  const float* mlp = a.ml + rh * 2;
+  float M = -INFINITY, L = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < a.n_splits; ++s) {
+    const float2 ml = *reinterpret_cast<const float2*>(mlp + s * pairs * 2);
+    const float4_t o = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(op + s * pairs * a.D));
+    const bool live = ml.y > 0.f;  // l == 0 marks an empty part (its O may be garbage)
+    const float Mn = fmaxf(M, live ? ml.x : -INFINITY);
+    const float sc = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
+    const float wgt = live ? __builtin_amdgcn_exp2f(ml.x - Mn) * ml.y : 0.f;
+    L = L * sc + wgt;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = acc[k] * sc + (live ? wgt * o[k] : 0.f);
+    M = Mn;
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int64_t row = rh / a.H;
+  const u32x2 v = {pack2<E>(acc[0] * inv, acc[1] * inv), pack2<E>(acc[2] * inv, acc[3] * inv)};
+  *reinterpret_cast<u32x2*>(a.out + row * a.out_stride + (rh - row * a.H) * a.D + d) = v;
+}
+
 // Marks parts [part0, part0+nparts) empty (l = 0) for every (request, head).
 __global__ __launch_bounds__(256) void clear_ml_kernel(float* ml, int64_t n2) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -285,6 +317,14 @@ int launch_items(const ItemArgs& a, int dtype, int D, hipStream_t st, const Kern
 }
 int launch_merge(const MergeArgs& a, int dtype, int D, hipStream_t st, const KernelEvents& ev) {
   PH_DISPATCH(launch_merge_t, dtype, D, a, st, ev);
+}
+int launch_fold_parts(const FoldArgs& a, int dtype, hipStream_t st) {
+  const int64_t threads = (int64_t)a.rows * a.H * (a.D / 4);
+  if (threads == 0) return PH_OK;
+  const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
+  if (dtype == PH_F16) hipLaunchKernelGGL((fold_parts_kernel<F16>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((fold_parts_kernel<BF16>), grid, block, 0, st, a);
+  return launch_status();
 }
 int launch_clear_ml(float* ml, int64_t entries, hipStream_t st) {
   if (entries == 0) return PH_OK;

@@ -129,6 +129,8 @@ struct PrefixArgs {
   float scale_log2e;
 };
 
+constexpr int kScanChunks = 256;  // four rounds of 64 lanes
+
 struct PrefillArgs {
   const uint16_t* q;
   int64_t q_stride;
@@ -140,20 +142,33 @@ struct PrefillArgs {
   const int32_t* q_cu;       // [C+1] device
   const int32_t* kv_cu;      // [C+1] device
   const int32_t* ctx_slots;
-  int32_t* tile_cu;          // [C+1] scratch: 64-query tiles before each chunk
-  int num_chunks;
+  int32_t* tile_cu;          // [C+1] scratch for the tiles before each chunk, null up to kScanChunks chunks
+  int num_tokens, num_chunks;
   int H;
   float scale_log2e;
   int pair;                  // 1: heads are 64 wide and run as halves of 128-wide head pairs (q, out, caches [.., H, 64])
   int tile_row0;             // first tile row of this launch (grid.y covers rows tile_row0 ..)
   int head_dim;              // 0 / 128, or 80 / 96 / 112: a short head on the 128-wide tile (set by launch_prefill_mfma)
+  int n_splits;              // > 1: every tile's visible tokens are cut into this many parts,
+  float* opart;              //      [n_splits][num_tokens][H] rows of head_dim (paired: 64) floats
+  float* ml;                 //      and (m, l) each, folded by the merge kernel
+};
+
+// The parts of a split prefill and where their fold goes (16-bit elements).
+struct FoldArgs {
+  const float* opart;  // [n_splits][rows][H] rows of D floats, normalised
+  const float* ml;     // (m, l) of each
+  uint16_t* out;
+  int64_t out_stride;
+  int n_splits, rows, H, D;
 };
 
 int launch_partial(const PartialArgs& a, int dtype, int D, hipStream_t st, const KernelEvents& ev = KernelEvents());
-// MFMA prefill: grid (head, query tile); num_tokens = total query rows (bounds the tile count).
-int launch_prefill_mfma(const PrefillArgs& a, int dtype, int D, int64_t num_tokens, hipStream_t st);
+// MFMA prefill: grid (head, query tile, split); tile_q = 64, 128 or 256 queries per workgroup.
+int launch_prefill_mfma(const PrefillArgs& a, int dtype, int D, int tile_q, hipStream_t st);
 int launch_items(const ItemArgs& a, int dtype, int D, hipStream_t st, const KernelEvents& ev = KernelEvents());
 int launch_merge(const MergeArgs& a, int dtype, int D, hipStream_t st, const KernelEvents& ev = KernelEvents());
+int launch_fold_parts(const FoldArgs& a, int dtype, hipStream_t st);
 int launch_clear_ml(float* ml, int64_t entries, hipStream_t st);
 // balanced suffix plan written on the device from the length vector (tables.hip); arrays as in ph_suffix_plan
 constexpr int kPlanMaxReqs = 8192;

@@ -1078,24 +1078,91 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
   PH_TL(11);
 }
 
+// Inclusive sum over the wave's lanes, in registers (four shifts inside a row of 16 lanes, then the row totals
+// broadcast to the rows behind).
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+
+// The query tile a workgroup takes: tile rows count from the last tile of the last chunk backwards (later tiles of a
+// chunk see more keys: the launch must not end on the longest ones).
+struct PrefillTile {
+  int cq0, n;     // the chunk's first query row and query count
+  int kv0, kvn;   // its context's place in ctx_slots
+  int tile;       // tile within the chunk
+};
+// Up to kScanChunks chunks every wave finds its tile by itself: 64 chunks at a time, lane l takes the l-th chunk from
+// the end, one round of loads and a register scan (with a pre-pass kernel and a binary search of dependent loads in
+// its place one chunk of 61 queries over 2048 tokens took 28.9 us instead of 27.1).  More chunks are searched in the
+// pre-pass's a.tile_cu.
+// false: past the last tile.
+__device__ __forceinline__ bool find_prefill_tile(const PrefillArgs& a, int row, int tile_q, PrefillTile& t) {
+  const int lane = threadIdx.x & 63;
+  if (a.tile_cu) {
+    const int ti = a.tile_cu[a.num_chunks] - 1 - row;
+    if (ti < 0) return false;
+    int lo = 0, hi = a.num_chunks;  // chunk with tile_cu[c] <= ti < tile_cu[c+1]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (a.tile_cu[mid] <= ti) lo = mid; else hi = mid;
+    }
+    t = PrefillTile{a.q_cu[lo], a.q_cu[lo + 1] - a.q_cu[lo], a.kv_cu[lo], a.kv_cu[lo + 1] - a.kv_cu[lo],
+                    ti - a.tile_cu[lo]};
+    return true;
+  }
+  for (int c0 = a.num_chunks - 1; c0 >= 0; c0 -= kWave) {
+    const int c = c0 - lane, cc = max(c, 0);
+    const int q0 = a.q_cu[cc], q1 = a.q_cu[cc + 1], k0 = a.kv_cu[cc], k1 = a.kv_cu[cc + 1];
+    const int mine = c >= 0 ? (q1 - q0 + tile_q - 1) / tile_q : 0;
+    const int upto = wave_prefix_sum(mine);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(upto > row);
+    if (hit != 0) {
+      const int l = __builtin_ctzll(hit);
+      t.cq0 = __builtin_amdgcn_readlane(q0, l);
+      t.n = __builtin_amdgcn_readlane(q1, l) - t.cq0;
+      t.kv0 = __builtin_amdgcn_readlane(k0, l);
+      t.kvn = __builtin_amdgcn_readlane(k1, l) - t.kv0;
+      t.tile = __builtin_amdgcn_readlane(upto, l) - 1 - row;
+      return true;
+    }
+    row -= __builtin_amdgcn_readlane(upto, kWave - 1);
+  }
+  return false;
+}
+
+// tile_cu[c] = number of tiles before chunk c, one wave over the chunks
+__global__ __launch_bounds__(64) void prefill_tiles_kernel(const int32_t* q_cu, int num_chunks, int32_t* tile_cu,
+                                                           int tile_q) {
+  const int lane = threadIdx.x;
+  int before = 0;
+  for (int c0 = 0; c0 < num_chunks; c0 += kWave) {
+    const int c = c0 + lane;
+    const int mine = c < num_chunks ? (q_cu[c + 1] - q_cu[c] + tile_q - 1) / tile_q : 0;
+    const int upto = wave_prefix_sum(mine);
+    if (c < num_chunks) tile_cu[c] = before + upto - mine;
+    before += __builtin_amdgcn_readlane(upto, kWave - 1);
+  }
+  if (lane == 0) tile_cu[num_chunks] = before;
+}
+
 // Prefill with parent context, eight waves: workgroup = (head, tile of 32 * (8 / TQ) queries of one chunk)
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
-template <typename E, int TQ, int SUB, bool HALF = false>
-__device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, int tile_row, char* smem) {
+// SPLIT: the tile's visible tokens are cut into a.n_splits runs, this workgroup takes run `split` and writes an
+// (O, m, l) part for the merge kernel instead of the output row.
+template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
+__device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const PrefillTile& pt, int split, char* smem) {
   constexpr int QB = 8 / TQ, NDB = 4 / TQ, QT = 32 * QB;
   // 64-wide heads: workgroup x is head x = half (x & 1) of pair x >> 1, whose K/V rows are one 128-wide row
   const int head = a.pair ? blockIdx.x >> 1 : blockIdx.x;
   const int half = a.pair ? (int)(blockIdx.x & 1) : -1;
-  // later tiles of a chunk see more keys: hand them out first so the launch does not end on the longest ones
-  const int ti = a.tile_cu[a.num_chunks] - 1 - tile_row;
-  int lo = 0, hi = a.num_chunks;  // chunk with tile_cu[c] <= ti < tile_cu[c+1]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (a.tile_cu[mid] <= ti) lo = mid; else hi = mid;
-  }
-  const int cq0 = a.q_cu[lo], n = a.q_cu[lo + 1] - cq0;
-  const int kv0 = a.kv_cu[lo], kvn = a.kv_cu[lo + 1] - kv0;
-  const int q0 = (ti - a.tile_cu[lo]) * QT;
+  const int cq0 = pt.cq0, n = pt.n, kv0 = pt.kv0, kvn = pt.kvn;
+  const int q0 = pt.tile * QT;
   const int nq = min(QT, n - q0);
   TileWork wk;
   const int hd = a.head_dim ? a.head_dim : kPD;  // 80 / 96 / 112: a short head on the 128-wide tile
@@ -1109,19 +1176,48 @@ __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, int tile_row
   wk.s0 = 0;
   wk.causal_off = kvn - n + q0;
   wk.s1 = min(kvn, wk.causal_off + nq);  // the last live query sees tokens up to causal_off + nq - 1
+  const int lane = threadIdx.x & 63, w8 = threadIdx.x >> 6, g = w8 / QB, qb = w8 % QB, h = lane >> 5, ql = lane & 31;
+  const int q = 32 * qb + ql;
+  if (SPLIT) {
+    constexpr int kRun = kTile * SUB * TQ;  // whole steps
+    const int run = ((wk.s1 + a.n_splits - 1) / a.n_splits + kRun - 1) / kRun * kRun;
+    wk.s0 = split * run;
+    if (wk.s0 >= wk.s1) {  // fewer steps than splits: mark the part empty
+      if (q < nq && g == 0 && h == 0) {
+        const int64_t pr = ((int64_t)split * a.num_tokens + cq0 + q0 + q) * a.H + blockIdx.x;
+        a.ml[pr * 2] = -INFINITY;
+        a.ml[pr * 2 + 1] = 0.f;
+      }
+      return;
+    }
+    wk.s1 = min(wk.s1, wk.s0 + run);
+  }
   float16_t of[NDB];
   float m, l;
   // the prefill loop is bound by instruction issue: the pre-scaled query saves it one multiply-add per score
   attn_tile8<E, true, TQ, NoMid, SUB, HALF, true>(wk, a.kc, a.vc, a.row_stride, head, a.scale_log2e, smem, of, m, l);
-  const int lane = threadIdx.x & 63, w8 = threadIdx.x >> 6, g = w8 / QB, qb = w8 % QB, h = lane >> 5, ql = lane & 31;
-  const int q = 32 * qb + ql;
   if (q < nq) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int64_t pr = SPLIT ? ((int64_t)split * a.num_tokens + cq0 + q0 + q) * a.H + blockIdx.x : 0;
+    if (SPLIT && h == 0 && g == 0) {
+      a.ml[pr * 2] = m;
+      a.ml[pr * 2 + 1] = l;
+    }
 #pragma unroll
     for (int nd = 0; nd < NDB; ++nd) {
       if (HALF && nd >= 2) continue;                      // accumulators 0, 1 hold this half's two blocks
       const int db = HALF ? 2 * half + nd : NDB * g + nd;  // 32-dim block of the 128-wide row
       if (a.pair && (db >> 1) != half) continue;  // the other half holds the neighbouring head's values: dropped
+      if (SPLIT) {
+        float* op = a.opart + pr * (a.pair ? 64 : hd) + (a.pair ? 32 * (db & 1) : 32 * db) + 4 * h;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float4_t v = {of[nd][4 * j] * inv, of[nd][4 * j + 1] * inv, of[nd][4 * j + 2] * inv,
+                              of[nd][4 * j + 3] * inv};
+          if (a.pair || 32 * db + 4 * h + 8 * j < hd) *reinterpret_cast<float4_t*>(op + 8 * j) = v;
+        }
+        continue;
+      }
       // paired: head 2 * pair + half, dims 32 * (db & 1) ..; else head, dims 32 * db ..
       uint16_t* op = a.out + (int64_t)(cq0 + q0 + q) * a.out_stride +
                      (a.pair ? (int)blockIdx.x * 64 + 32 * (db & 1) : head * hd + 32 * db) + 4 * h;
@@ -1137,28 +1233,17 @@ __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, int tile_row
 
 // Prefill with parent context, eight waves: workgroup = (head, tile of 32 * (8 / TQ) queries of one chunk); grid.y
 // covers the tile rows from a.tile_row0 on (more rows than a grid's y extent holds take several launches; a loop
-// over rows inside the kernel cost the common single-launch case 6 %)
+// over rows inside the kernel cost the common single-launch case 6 %), grid.z the splits
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
-template <typename E, int TQ, int SUB, bool HALF = false>
+template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
 __global__ __launch_bounds__(512) void prefill_mfma8_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   PH_TL(0);
   if ((int)blockIdx.x >= a.H) return;
-  const int row = a.tile_row0 + (int)blockIdx.y;
-  if (row >= a.tile_cu[a.num_chunks]) return;
-  prefill_tile8<E, TQ, SUB, HALF>(a, row, smem);
+  PrefillTile pt;
+  if (!find_prefill_tile(a, a.tile_row0 + (int)blockIdx.y, 32 * (8 / TQ), pt)) return;
+  prefill_tile8<E, TQ, SUB, HALF, SPLIT>(a, pt, blockIdx.z, smem);
   PH_TL(11);
-}
-
-// tile_cu[c] = number of 64-query tiles before chunk c (serial scan; chunk counts are small)
-__global__ void prefill_tiles_kernel(const int32_t* q_cu, int num_chunks, int32_t* tile_cu, int tile_q) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int acc = 0;
-  for (int c = 0; c < num_chunks; ++c) {
-    tile_cu[c] = acc;
-    acc += (q_cu[c + 1] - q_cu[c] + tile_q - 1) / tile_q;
-  }
-  tile_cu[num_chunks] = acc;
 }
 
 template <typename E, int TQ, int SUB = 1, bool PRESC = false>
@@ -1195,33 +1280,40 @@ static int launch_prefix_t(const PrefixArgs& a, int num_groups, int max_group_re
 
 constexpr int64_t kMaxGridY = 65535;  // grid extent in y and z
 
-template <typename E, int TQ, int SUB, bool HALF = false>
-static int launch_prefill_tq(const PrefillArgs& a, int64_t num_tokens, hipStream_t st) {
+template <typename E, int TQ, int SUB, bool HALF, bool SPLIT>
+static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
   constexpr int QT = 32 * (8 / TQ);  // queries per workgroup tile
-  hipLaunchKernelGGL(prefill_tiles_kernel, dim3(1), dim3(64), 0, st, a.q_cu, a.num_chunks, a.tile_cu, QT);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF>),
+  if (a.tile_cu) {
+    hipLaunchKernelGGL(prefill_tiles_kernel, dim3(1), dim3(kWave), 0, st, a.q_cu, a.num_chunks, a.tile_cu, QT);
+    const int rc = launch_status();
+    if (rc != PH_OK) return rc;
+  }
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, kTile8Lds);
   const int hx = (a.H + 7) / 8 * 8;  // keeps head == linear id mod 8 for every tile row
-  const int64_t max_tiles = num_tokens / QT + a.num_chunks;  // >= sum of ceil(n_c / QT)
+  const int64_t max_tiles = (a.num_tokens - a.num_chunks) / QT + a.num_chunks;  // >= sum of ceil(n_c / QT), n_c >= 1
   for (int64_t row0 = 0; row0 < max_tiles; row0 += kMaxGridY) {
     PrefillArgs part = a;
     part.tile_row0 = (int)row0;
     const int64_t rows = max_tiles - row0 < kMaxGridY ? max_tiles - row0 : kMaxGridY;
-    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF>), dim3(hx, (unsigned)rows), dim3(512), kTile8Lds, st,
-                       part);
+    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>), dim3(hx, (unsigned)rows, SPLIT ? a.n_splits : 1),
+                       dim3(512), kTile8Lds, st, part);
   }
   return launch_status();
 }
 
-// Query tile by the average chunk length: 256-query tiles share every K/V tile among all eight waves (least
-// traffic, deepest staging ring) but idle whole waves on short chunks, which take 128- or 64-query tiles.
+template <typename E, int TQ, int SUB, bool HALF = false>
+static int launch_prefill_sq(const PrefillArgs& a, hipStream_t st) {
+  return a.n_splits > 1 ? launch_prefill_tq<E, TQ, SUB, HALF, true>(a, st)
+                        : launch_prefill_tq<E, TQ, SUB, HALF, false>(a, st);
+}
+
 template <typename E>
-static int launch_prefill_t(const PrefillArgs& a, int64_t num_tokens, hipStream_t st) {
-  const int64_t avg = num_tokens / (a.num_chunks > 0 ? a.num_chunks : 1);
-  if (avg >= 192 && a.pair) return launch_prefill_tq<E, 1, 2, true>(a, num_tokens, st);
-  if (avg >= 192) return launch_prefill_tq<E, 1, 2>(a, num_tokens, st);  // 64-token steps (measured 4 % faster)
-  if (avg >= 96) return launch_prefill_tq<E, 2, 1>(a, num_tokens, st);
-  return launch_prefill_tq<E, 4, 1>(a, num_tokens, st);
+static int launch_prefill_t(const PrefillArgs& a, int tile_q, hipStream_t st) {
+  if (tile_q == 256 && a.pair) return launch_prefill_sq<E, 1, 2, true>(a, st);
+  if (tile_q == 256) return launch_prefill_sq<E, 1, 2>(a, st);  // 64-token steps (measured 4 % faster)
+  if (tile_q == 128) return launch_prefill_sq<E, 2, 1>(a, st);
+  return launch_prefill_sq<E, 4, 1>(a, st);
 }
 
 template <typename E, int TQ, int DS, int NQ = 1>
@@ -1297,12 +1389,12 @@ int launch_prefix_mfma(const PrefixArgs& a0, int dtype, int D, int num_groups, i
                          : launch_prefix_t<BF16>(a, num_groups, max_group_reqs, internal_ml, st, ev);
 }
 
-int launch_prefill_mfma(const PrefillArgs& a0, int dtype, int D, int64_t num_tokens, hipStream_t st) {
+int launch_prefill_mfma(const PrefillArgs& a0, int dtype, int D, int tile_q, hipStream_t st) {
   if (!prefix_mfma_supported(dtype, D)) return PH_ERR_HEAD_DIM;
-  if (num_tokens <= 0 || a0.num_chunks <= 0) return PH_OK;
+  if (a0.num_tokens <= 0 || a0.num_chunks <= 0) return PH_OK;
   PrefillArgs a = a0;
   a.head_dim = a.pair ? kPD : D;
-  return dtype == PH_F16 ? launch_prefill_t<F16>(a, num_tokens, st) : launch_prefill_t<BF16>(a, num_tokens, st);
+  return dtype == PH_F16 ? launch_prefill_t<F16>(a, tile_q, st) : launch_prefill_t<BF16>(a, tile_q, st);
 }
 
 }  // namespace ph

@@ -100,17 +100,21 @@ _captured_keys: set = set()               # (device, stream) whose current buffe
 _pinned_workspaces: List[torch.Tensor] = []  # outgrown buffers that recorded graphs still use
 
 
-def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
+def _workspace(nbytes: int, device: torch.device, least: Optional[int] = None) -> torch.Tensor:
     """Grow-only scratch buffer per (device, stream); reuse is ordered by the stream.
 
     A buffer handed out while the stream is being captured into a graph is recorded by address in that graph, so
     it is pinned for the life of the process: growing never frees it (an eager call that needs more gets a new
     buffer, the recorded graph keeps the old one), and a request made under capture that does not fit the
-    stream's buffer is refused instead of allocating inside the capture."""
+    stream's buffer is refused instead of allocating inside the capture.  ``least``: the call also works with that
+    many bytes, so under capture a buffer of at least that size is handed out as it is."""
     key = (device.index or 0, _stream())
     buf = _workspaces.get(key)
     capturing = torch.cuda.is_current_stream_capturing()
     if buf is None or buf.numel() < nbytes:
+        if capturing and buf is not None and least is not None and buf.numel() >= least:
+            _captured_keys.add(key)
+            return buf
         if capturing and buf is not None:
             raise RuntimeError(
                 f"decode workspace of {buf.numel()} bytes is too small for {nbytes} bytes and the stream is being "
@@ -941,8 +945,8 @@ def prefill_attention(query, key_cache, value_cache, tables: PrefillTables, scal
         return out
     scale = D ** -0.5 if scale is None else scale
     lib = _lib.load()
-    nbytes = lib.ph_prefill_workspace_bytes(T, H, D, _dtype_code(query), tables.max_kv_len)
-    ws = _workspace(nbytes, query.device)
+    shape = (T, H, D, _dtype_code(query), tables.max_kv_len)
+    ws = _workspace(lib.ph_prefill_workspace_bytes(*shape), query.device, lib.ph_prefill_workspace_min_bytes(*shape))
     rc = lib.ph_prefill_attention(
         _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), T, tables.num_chunks, H, D, _dtype_code(query),
         query.stride(0), out.stride(0), key_cache.stride(0), float(scale), _ptr(tables.q_cu), _ptr(tables.kv_cu),

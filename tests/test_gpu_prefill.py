@@ -186,6 +186,55 @@ def test_prefill_short_heads_on_the_wide_tile(dev, D, dtype):
         torch.testing.assert_close(out.float(), ref.float(), **TOL[dtype])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("q_lens,parent,H,D", [
+    ([61], 1987, 4, 128),      # many parts of one 64-query tile
+    ([1], 1100, 3, 128),       # nine steps: the last of several parts is empty
+    ([16, 5], 900, 5, 128),    # two chunks of different visible lengths
+    ([33], 1500, 2, 96),       # short heads
+    ([40, 7], 800, 4, 64),     # head pairs
+    ([700], 5000, 2, 64),      # head pairs on more than one tile, parts beyond the slot window's length
+    ([300], 6100, 9, 128),     # several tiles, the last one partly filled
+])
+def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, dtype):
+    """Few queries over long contexts: every tile's visible tokens are cut into parts folded afterwards.  A call with
+    only the smallest workspace takes the same chunks in one part per tile."""
+    from parrotserve_amd import _lib, kernels, synth
+
+    case = synth.make_prefill_case("parts", 70 + parent + H, dtype, q_lens, parent, H, D, 1 << 13)
+    out, ref = run_prefill_case(case, dev)
+    torch.testing.assert_close(out.float(), ref.float(), **TOL[dtype])
+
+    lib, T = _lib.load(), sum(q_lens)
+    shape = (T, H, D, _lib.PH_F16 if dtype == torch.float16 else _lib.PH_BF16, parent + max(q_lens))
+    least = lib.ph_prefill_workspace_min_bytes(*shape)
+    assert lib.ph_prefill_workspace_bytes(*shape) > least
+    kc, vc = synth.pool_to_device(torch.cat([case.k_rows, case.k_new]), torch.cat([case.v_rows, case.v_new]),
+                                  case.used_slots, case.pool_slots, dev)
+    q = case.q.to(dev)
+    ctx = [case.used_slots[torch.cat([p, n])].tolist() for p, n in zip(case.parent_lists, case.new_lists)]
+    tabs = kernels.PrefillTables.build(q_lens, ctx, dev)
+    whole, small = kernels.prefill_attention(q, kc, vc, tabs), torch.empty_like(q)
+    ws = torch.empty(least, dtype=torch.uint8, device=dev)
+    args = (q.data_ptr(), kc.data_ptr(), vc.data_ptr(), T, len(q_lens), H, D, shape[3], H * D, H * D, H * D, D ** -0.5,
+            tabs.q_cu.data_ptr(), tabs.kv_cu.data_ptr(), tabs.ctx_slots.data_ptr(), tabs.ctx_slots.numel(), shape[4])
+    assert lib.ph_prefill_attention(small.data_ptr(), *args, ws.data_ptr(), least, kernels._stream()) == 0
+    torch.testing.assert_close(whole.float(), small.float(), **TOL[dtype])
+    assert lib.ph_prefill_attention(small.data_ptr(), *args, ws.data_ptr(), least - 1, kernels._stream()) == \
+        _lib.PH_ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("chunks", [64, 65, 130, 256, 257])
+def test_prefill_chunk_counts_around_the_tile_search(dev, chunks):
+    """Chunk counts at the edges of the in-kernel tile search (64 chunks a round, a pre-pass beyond 256)."""
+    from parrotserve_amd import synth
+
+    q_lens = [1 + (7 * i) % 5 + (66 if i % 50 == 3 else 0) for i in range(chunks)]
+    case = synth.make_prefill_case("many", 40 + chunks, torch.bfloat16, q_lens, 9, 2, 128, 1 << 13)
+    out, ref = run_prefill_case(case, dev)
+    torch.testing.assert_close(out.float(), ref.float(), **TOL[torch.bfloat16])
+
+
 def test_more_tile_rows_than_the_grid_holds(dev):
     """70,000 one-token chunks without parents: more tile rows than a grid's y extent (65,535), so workgroups stride
     over them.  A query that sees exactly one key returns that key's value row."""
