@@ -7,17 +7,17 @@
 // The reference sorts every row twice (sort, then arg-sort of the permutation) to apply the filter.  Here the
 // filter is a threshold: with e_i = exp(x_i - max) and G(t) = sum of e_j over e_j > t, token i stays iff
 // G(e_i) + (its rank among equal values) * e_i <= top_p * sum(e).  G is monotone, so the smallest surviving value
-// is found by bisection over the ordered bit patterns of the element type (16 steps for bf16, 19 for fp16, 32
-// for fp32), each step a compare-and-add over the row's e values (the exponential is taken once per token) and
-// one block reduction.  Equal values are ranked by ascending token id.
+// is found by a search over ordered bit patterns.  Equal values are ranked by ascending token id.
 // The draw is the inverse-CDF draw over ascending token ids from a uniform number the caller passes, so the
 // result is a function of the inputs (the reference draws through torch.multinomial's own random stream).
 //
 // One workgroup of 1024 lanes per row.  Two kernels, same arithmetic:
-//   sample_rows_kernel   rows on the 16-byte grid of up to 57,344 tokens: the row lives in registers;
+//   sample_rows_kernel   rows on the 16-byte grid of up to 57,344 tokens: the row lives in registers, the cut
+//                        comes from histograms of the mass over the bit patterns of e;
 //   sample_top_p_kernel  any other row: e values in LDS up to 36 K tokens, longer rows are re-read and
-//                        re-exponentiated in every pass (they sit in L2; slower).
-// Sums are taken in a fixed order (per-lane partial sums, a wave tree, then the sixteen wave sums in
+//                        re-exponentiated in every pass (they sit in L2; slower); the cut comes from a bisection
+//                        over the patterns of the element type, a compare-and-add over the row per bit.
+// Histogram sums are whole numbers (atomic order does not matter), float sums are taken in a fixed order (per-lane partial sums, a wave tree, then the sixteen wave sums in
 // sequence): the same tokens on every run.
 #include "common.hpp"
 
@@ -255,9 +255,66 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(const SampAr
   }
 }
 
+// x / T rounded to nearest for many x and one T: r = 1 / T rounded to nearest, one Newton correction of x * r, exact
+// while nothing leaves the normal range; 3 instructions in place of a division's 10.
+__device__ __forceinline__ bool quotient_by_reciprocal(float T) { return T >= 0x1p-40f && T <= 0x1p40f; }
+__device__ __forceinline__ float div_by(float x, float T, float r) {
+  const float q = x * r;
+  return __builtin_fabsf(q) < INFINITY ? __builtin_fmaf(__builtin_fmaf(-q, T, x), r, q) : q;
+}
+
+// Histograms of the mass over the bit pattern of e: 32 bins per power of two, then 9 bits inside the bin the mass
+// crosses its target in, then the last 9 bits.  Values of one coarse bin differ in the low 18 bits of their mantissas
+// only, so a bin takes the tokens' count (from bit 40 up) and the sum of those bits: whole numbers, one add per token.
+// Masses of different bins are compared in units of 2^-46 (a row's mass stays below 2^62), inside a bin in mantissas.
+typedef unsigned long long mass_t;
+constexpr int kHistShift = 18, kHistFine = 9, kHistCount = 40;
+constexpr int kHistBins = 4096;  // up to the bin of e == 1 and beyond (any pattern is masked into them)
+static_assert((0x3f800000 >> kHistShift) < kHistBins && kHistBins == 4 * kSampThreads, "four bins per lane");
+constexpr uint32_t kHistLeast = 0x21800000u;  // 2^-60: less is no mass
+__device__ __forceinline__ uint32_t mantissa(uint32_t bits) { return (bits & 0x7fffffu) | 0x800000u; }
+__device__ __forceinline__ mass_t hist_entry(uint32_t bits) {
+  return ((mass_t)1 << kHistCount) | (bits & ((1u << kHistShift) - 1));
+}
+// Sum of the mantissas of a coarse bin.  (The count times the leading bits as a whole, a product of two 24-bit numbers,
+// is miscompiled by this toolchain: it loses the mask of the leading bits.)
+__device__ __forceinline__ mass_t hist_mantissas(mass_t entry, uint32_t bin) {
+  const uint32_t count = (uint32_t)(entry >> kHistCount);
+  return ((mass_t)count << 23) + ((mass_t)(count * (bin & ((1u << (23 - kHistShift)) - 1))) << kHistShift) +
+         (entry & (((mass_t)1 << kHistCount) - 1));
+}
+__device__ __forceinline__ int mass_shift(uint32_t bin) {  // mantissas of a coarse bin << this = units of 2^-46
+  return (int)(bin >> (23 - kHistShift)) - (127 - 23);
+}
+__device__ __forceinline__ mass_t* hist_slot(mass_t* coarse, uint32_t bits) {
+  return reinterpret_cast<mass_t*>(reinterpret_cast<char*>(coarse) +
+                                   ((bits >> (kHistShift - 3)) & ((kHistBins - 1) * sizeof(mass_t))));
+}
+__device__ __forceinline__ mass_t wave_prefix_mass(mass_t v, int lane) {
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const mass_t up = __shfl_up(v, d, kWave);
+    if (lane >= d) v += up;
+  }
+  return v;
+}
+
+struct SampHist {
+  mass_t coarse[kHistBins];
+  mass_t fine[2][1 << kHistFine];
+  mass_t wave_mass[kSampWaves];
+  mass_t goal;     // what the bins still in question may hold above the cut, in mantissas
+  uint32_t bin;    // the bin the mass crosses the target in
+  uint32_t thr;    // bit pattern of the smallest surviving e ...
+  int n_equal;     // ... how many tokens of that value survive
+  int equal;       // ... and how many there are
+};
+
 // Rows that fit the register file: 16-byte aligned rows of up to 1024 * kSampRegFloats tokens.  Lane t owns the
 // 16-byte chunks t, t + 1024, t + 2048, ... of the row (K "rounds" of 1024 chunks); the row is read once, the
-// exponentials are taken once, and every later pass is compares and adds on registers.  Token-id order is
+// exponentials are taken once, and every later pass is compares and adds on registers.  Bound by vector issue on one
+// compute unit per row: the cut by three histogram levels instead of a bisection of 16 to 32 compare-and-add passes
+// with a reduction each took 64 rows of 32,000 fp16 logits from 37.7 to 24.4 us.  Token-id order is
 // (round, lane, position in the chunk), so the two places that need it -- ranking equal values at the cut and
 // the cumulative sum of the draw -- take one batched reduction over the rounds to find the round in which the
 // count / the sum crosses, and one scan over the lanes inside that round.
@@ -269,6 +326,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   constexpr int K = kSampRegFloats / N;     // chunks per lane
   constexpr int SH = key_shift<E>();
   __shared__ SampShared sh;
+  __shared__ SampHist hist;
   __shared__ float fred[K][kSampWaves];
   __shared__ int ired[K][kSampWaves];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -298,6 +356,13 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
     return s;
   };
 
+  const bool filter = p < 1.f;
+  if (filter) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) hist.coarse[t + i * kSampThreads] = 0;
+    if (t < 2 << kHistFine) hist.fine[t >> kHistFine][t & ((1 << kHistFine) - 1)] = 0;
+  }
+
   float e[K][N];
   const int chunks = (V + N - 1) / N;
   const int rounds = (chunks + kSampThreads - 1) / kSampThreads;  // rounds that hold tokens; the rest stay zero
@@ -317,15 +382,27 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
       }
     }
   }
+  if (T != 1.f) {
+    const bool by_r = quotient_by_reciprocal(T);
+    const float r = __fdiv_rn(1.f, T);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) break;
+      if (by_r) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) e[k][j] = Logit<E>::round(div_by(e[k][j], T, r));
+      } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) e[k][j] = Logit<E>::round(__fdiv_rn(e[k][j], T));
+      }
+    }
+  }
   float m = -INFINITY;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     if (k >= rounds) break;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      if (T != 1.f) e[k][j] = Logit<E>::round(__fdiv_rn(e[k][j], T));
-      m = fmaxf(m, e[k][j]);
-    }
+    for (int j = 0; j < N; ++j) m = fmaxf(m, e[k][j]);
   }
   m = group_max<64>(m);
   if (lane == 0) sh.red[par][w] = m;
@@ -345,36 +422,159 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
       z += e[k][j];
     }
   }
+  if (filter) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) break;
+      // a row of few distinct values would send a whole wave to one address, one lane after the other: where all lanes
+      // hold the same value, one of them adds for all
+      const float e0 = e[k][0];
+      const bool same = __builtin_amdgcn_ballot_w64(e0 != __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                                                                __builtin_bit_cast(int, e0)))) == 0;
+      if (same) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const uint32_t v = __builtin_bit_cast(uint32_t, e[k][j]);
+          const bool all = __builtin_amdgcn_ballot_w64(v != (uint32_t)__builtin_amdgcn_readfirstlane((int)v)) == 0;
+          if (v >= kHistLeast && (!all || lane == 0))
+            atomicAdd(hist_slot(hist.coarse, v), hist_entry(v) << (all ? 6 : 0));
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const uint32_t v = __builtin_bit_cast(uint32_t, e[k][j]);
+          if (v >= kHistLeast) atomicAdd(hist_slot(hist.coarse, v), hist_entry(v));
+        }
+      }
+    }
+  }
   z = block_sum(z);
 
-  if (p < 1.f) {  // the filter: zero the e of every token that does not survive
-    const float target = fmaxf(p, 0.f) * z;
-    uint32_t lo = to_key<SH>(-INFINITY), hi = to_key<SH>(m);
-    float g_hi = 0.f;
-    while (lo < hi) {  // lo, hi and g are the same in every lane
-      const uint32_t mid = lo + ((hi - lo) >> 1);
-      const float cut = expf(from_key<SH>(mid) - m);
-      float g = 0.f;
+  if (filter) {  // zero the e of every token that does not survive
+    float thr;
+    int n_equal = INT_MAX, equal = INT_MAX;  // equal: tokens of value thr, or more
+    if (z >= 1.f && z < INFINITY) {          // the most likely token has e == 1 and no e is NaN: every e is in [0, 1]
+      // the value at which the mass of the values from the top down passes the target
+      mass_t four[4], mine = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int bin = kHistBins - 1 - (4 * t + i);  // from the top down
+        const mass_t sum = hist_mantissas(hist.coarse[bin], bin);
+        const int up = mass_shift(bin);
+        four[i] = up >= 0 ? sum << up : up > -64 ? sum >> -up : 0;
+        mine += four[i];
+      }
+      const mass_t inc = wave_prefix_mass(mine, lane);
+      if (lane == kWave - 1) hist.wave_mass[w] = inc;
+      __syncthreads();
+      mass_t before = inc - mine, total = 0;
+#pragma unroll
+      for (int i = 0; i < kSampWaves; ++i) {
+        if (i == w) before += total;
+        total += hist.wave_mass[i];
+      }
+      const mass_t target = (mass_t)((double)fmaxf(p, 0.f) * (double)total);
+      if (before <= target && target < before + mine) {  // one lane of the workgroup
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (before <= target && target < before + four[i]) {
+            const int bin = kHistBins - 1 - (4 * t + i), up = mass_shift(bin);
+            hist.bin = bin;
+            hist.goal = up >= 0 ? (target - before) >> up : (target - before) << -up;
+          }
+          before += four[i];
+        }
+      }
+      __syncthreads();
+      uint32_t top = hist.bin;  // the leading bits found so far
+#pragma unroll
+      for (int level = 0; level < 2; ++level) {
+        const int low = level == 0 ? kHistFine : 0;  // bits below this level's
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (k >= rounds) break;
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const uint32_t b = __builtin_bit_cast(uint32_t, e[k][j]);
+            if (b >> (low + kHistFine) == top)
+              atomicAdd(&hist.fine[level][(b >> low) & ((1 << kHistFine) - 1)], (mass_t)mantissa(b));
+          }
+        }
+        __syncthreads();
+        if (w == 0) {  // eight bins per lane
+          constexpr int kPer = (1 << kHistFine) / kWave;
+          mass_t bins[kPer], sum = 0;
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) {
+            bins[i] = hist.fine[level][(1 << kHistFine) - 1 - (kPer * lane + i)];
+            sum += bins[i];
+          }
+          const mass_t goal = hist.goal;
+          mass_t at = wave_prefix_mass(sum, lane) - sum;
+          if (at <= goal && goal < at + sum) {
+            mass_t in_bin = 0;
+            int bin = 0;
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+              if (in_bin == 0 && goal < at + bins[i]) {
+                in_bin = bins[i];
+                bin = (1 << kHistFine) - 1 - (kPer * lane + i);
+              }
+              if (in_bin == 0) at += bins[i];
+            }
+            hist.bin = bin;
+            hist.goal = goal - at;
+            if (level == 1) {
+              const uint32_t b = (top << kHistFine) | bin;
+              hist.thr = b;
+              hist.n_equal = (int)((goal - at) / mantissa(b)) + 1;
+              hist.equal = (int)(in_bin / mantissa(b));
+            }
+          }
+        }
+        __syncthreads();
+        if (level == 0) top = (top << kHistFine) | hist.bin;
+      }
+      const uint32_t tb = hist.thr;  // a copy: the cast is applied to a plain scalar
+      thr = __builtin_bit_cast(float, tb);
+      n_equal = hist.n_equal;
+      equal = hist.equal;
+    } else {  // NaN or infinite logits: bisection over the element type's patterns
+      const float target = fmaxf(p, 0.f) * z;
+      uint32_t lo = to_key<SH>(-INFINITY), hi = to_key<SH>(m);
+      float g_hi = 0.f;
+      while (lo < hi) {  // lo, hi and g are the same in every lane
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        const float cut = expf(from_key<SH>(mid) - m);
+        float g = 0.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (k >= rounds) break;
+#pragma unroll
+          for (int j = 0; j < N; ++j) g += e[k][j] > cut ? e[k][j] : 0.f;
+        }
+        g = block_sum(g);
+        if (g <= target) {
+          hi = mid;
+          g_hi = g;
+        } else {
+          lo = mid + 1;
+        }
+      }
+      thr = expf(from_key<SH>(hi) - m);
+      if (thr > 0.f) {
+        const float r = floorf((target - g_hi) / thr);
+        n_equal = r >= 2.0e9f ? INT_MAX : max((int)r + 1, 1);
+      }
+    }
+    if (equal <= n_equal) {  // every token of value thr survives
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         if (k >= rounds) break;
 #pragma unroll
-        for (int j = 0; j < N; ++j) g += e[k][j] > cut ? e[k][j] : 0.f;
+        for (int j = 0; j < N; ++j) e[k][j] = e[k][j] >= thr ? e[k][j] : 0.f;
       }
-      g = block_sum(g);
-      if (g <= target) {
-        hi = mid;
-        g_hi = g;
-      } else {
-        lo = mid + 1;
-      }
-    }
-    const float thr = expf(from_key<SH>(hi) - m);
-    int n_equal = INT_MAX;
-    if (thr > 0.f) {
-      const float r = floorf((target - g_hi) / thr);
-      n_equal = r >= 2.0e9f ? INT_MAX : max((int)r + 1, 1);
-    }
+    } else {
     // tokens equal to thr, per round; they survive in id order until n_equal of them have
     int cnt[K], tot[K];
 #pragma unroll
@@ -431,6 +631,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
         e[k][j] = keep ? v : 0.f;
       }
     }
+    }
   }
 
   // the draw: first token, in id order, at which the running sum of e passes uniform * (sum of e)
@@ -480,34 +681,40 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   float running = before_kd;
   for (int i = 0; i < w; ++i) running += sh.fpart[i];
   running += finc - mine;
-  int found = INT_MAX, found_after = INT_MAX, last = -1;
+  int found = INT_MAX;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    if (k >= rounds) break;
+    if (k != kd) continue;  // same in every lane
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const float v = e[k][j];
-      const int i = (t + k * kSampThreads) * N + j;
-      if (v > 0.f) {
-        last = i;
-        if (k > kd && found_after == INT_MAX) found_after = i;
-        if (k == kd) {
-          running += v;
-          if (running > goal && found == INT_MAX) found = i;
-        }
-      }
+      running += v;
+      if (v > 0.f && running > goal && found == INT_MAX) found = (t + k * kSampThreads) * N + j;
     }
   }
   if (found != INT_MAX) atomicMin(&sh.found, found);
-  if (found_after != INT_MAX) atomicMin(&sh.found_after, found_after);
-  if (last >= 0) atomicMax(&sh.last, last);
   __syncthreads();
-  if (t == 0) {
+  if (sh.found == INT_MAX) {  // same in every lane
     // rounding can leave the goal a hair above the sums of the round it was placed in: then the next surviving
     // token, or the last one of the row
-    const int id = sh.found != INT_MAX ? sh.found : sh.found_after != INT_MAX ? sh.found_after : max(sh.last, 0);
-    a.out[row] = id;
+    int found_after = INT_MAX, last = -1;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) break;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const int i = (t + k * kSampThreads) * N + j;
+        if (e[k][j] > 0.f) {
+          last = i;
+          if (k > kd && found_after == INT_MAX) found_after = i;
+        }
+      }
+    }
+    if (found_after != INT_MAX) atomicMin(&sh.found_after, found_after);
+    if (last >= 0) atomicMax(&sh.last, last);
+    __syncthreads();
   }
+  if (t == 0) a.out[row] = sh.found != INT_MAX ? sh.found : sh.found_after != INT_MAX ? sh.found_after : max(sh.last, 0);
 }
 
 template <typename E>

@@ -213,3 +213,50 @@ def test_reference_draw_mode_of_the_sampler_module():
     # (the torch path rounds its probabilities and their running sums to fp16, which can move a cut by a token)
     assert same_support.float().mean() >= 0.75
     assert torch.equal(ids[same_support], want[same_support])
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+def test_histogram_cut_on_unusual_rows(dtype):
+    """Rows at the edges of the mass histograms: one value everywhere (whole waves on one bin, ranks decide), almost
+    everything masked, values that span far more than the histogram's least mass, temperatures outside the range of the
+    reciprocal form, a cut between two neighbouring values of the element type."""
+    g = torch.Generator().manual_seed(31)
+    V = 4000
+    rows, temps, tops = [], [], []
+
+    def add(row, temp, top):
+        rows.append(row), temps.append(temp), tops.append(top)
+
+    add(torch.zeros(V), 1.0, 0.37013)
+    add(torch.full((V,), -3.5), 0.7, 0.90009)
+    masked = torch.full((V,), -float("inf"))
+    masked[::997] = torch.tensor([1.0, 2.0, 2.0, 0.5, 1.5])
+    add(masked, 0.9, 0.8)
+    add(torch.randn(V, generator=g) * 60, 1.0, 0.97)
+    add(torch.randn(V, generator=g) * 1e-3, 1.0, 0.6)
+    add(torch.where(torch.arange(V) % 2 == 0, 8.0, 8.0078125), 1.0, 0.7003)
+    add(torch.randn(V, generator=g) * 4, 1.0, 0.9999)
+    if dtype != "f16":
+        add(torch.randn(V, generator=g) * 1e-13, 2.0 ** -42, 0.9)
+        add(torch.randn(V, generator=g) * 1e13, 2.0 ** 42, 0.9)
+    x = torch.stack(rows).to(DT[dtype])
+    _check(x, torch.tensor(temps), torch.tensor(tops), torch.rand(len(rows), generator=g), dtype, min_compared=0.7)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+def test_rows_without_a_finite_mass_take_the_general_rule(dtype):
+    """NaN, +inf and nothing but -inf: the same token as from the kernel for rows off the 16-byte grid."""
+    g = torch.Generator().manual_seed(32)
+    V = 2000
+    x = torch.randn(8, V, generator=g) * 3
+    x[0, 17] = float("nan")
+    x[1, 5] = x[1, 1900] = float("inf")
+    x[2] = -float("inf")
+    x[3, 11], x[3, 12] = float("nan"), float("inf")
+    x[4, 100:] = -float("inf")
+    x = x.to(DT[dtype]).cuda()
+    temps, tops = torch.tensor([1.0, 0.7] * 4).cuda(), torch.tensor([0.9, 0.5, 1.0, 0.3] * 2).cuda()
+    u = torch.rand(8, generator=g).cuda()
+    buf = torch.zeros(8, V + 8, dtype=x.dtype, device="cuda")
+    buf[:, 1:V + 1] = x
+    assert torch.equal(kernels.sample_top_p(x, temps, tops, u), kernels.sample_top_p(buf[:, 1:V + 1], temps, tops, u))
