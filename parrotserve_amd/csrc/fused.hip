@@ -23,55 +23,98 @@ __device__ __forceinline__ float block_sum4(float v, float* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// One workgroup per row; ITERS 16-byte chunks per thread stay in registers between the sum and the write.
-template <typename E, int ITERS, bool ROUND_FIRST>
+// One workgroup per ROWS consecutive rows; ITERS 16-byte chunks per thread and row stay in registers between the sum
+// and the write.  Bound by HBM (four passes over the rows).  Every load of the ROWS rows is requested before the first
+// store: x and residual may not alias, but the compiler cannot know that two chunks of the residual do not, and kept
+// each chunk's loads behind the store of the one before.  Launches of many rows read both inputs past the caches.
+// Measured with inputs out of the caches, one row per workgroup with plain interleaved loads against three with
+// non-temporal loads ahead: 9404 rows of 5120 bf16 72.7 -> 63.2 us (1 row: 61.1, 2 rows: 60.7), 9404 of 4096 fp16
+// 50.1 -> 49.5, 3000 of 4096 fp16 18.7 -> 17.4 (19.5, 18.9), but 2500 of 5120 bf16 20.3 -> 21.3 us.  Plain loads
+// ahead with one row take what the interleaved ones took (71.2 and 18.7 us).
+template <typename E, int ITERS, bool ROUND_FIRST, int ROWS>
 __global__ __launch_bounds__(kFusedThreads) void add_rms_norm_vec(uint16_t* __restrict__ out, uint16_t* residual,
                                                                  const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ w, float eps, int n,
-                                                                 int64_t x_stride, int64_t r_stride,
+                                                                 int64_t rows, int64_t x_stride, int64_t r_stride,
                                                                  int64_t out_stride) {
-  __shared__ float red[4];
-  const int64_t row = blockIdx.x;
-  const uint16_t* xr = x + row * x_stride;
-  uint16_t* rr = residual + row * r_stride;
-  uint16_t* orow = out + row * out_stride;
+  __shared__ float red[ROWS][4];
+  const int64_t row0 = (int64_t)blockIdx.x * ROWS;
   const int chunks = n >> 3;
-  u32x4 v[ITERS];
-  float ss = 0.f;
+  u32x4 v[ROWS][ITERS], b[ROWS][ITERS], wv[ITERS];
 #pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    const int c = threadIdx.x + i * kFusedThreads;
-    if (c < chunks) {
-      const u32x4 a = ld16(xr + c * 8), b = ld16(rr + c * 8);
+  for (int r = 0; r < ROWS; ++r) {
+    const int64_t row = row0 + r < rows ? row0 + r : row0;  // a row past the end: row0's loads again, nothing stored
+    const uint16_t* xr = x + row * x_stride;
+    const uint16_t* rr = residual + row * r_stride;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // the sum is stored (rounded) as the new residual, and the norm runs on the stored value
-        const uint32_t s = pack2<E>(Elem<E>::lo(a[j]) + Elem<E>::lo(b[j]), Elem<E>::hi(a[j]) + Elem<E>::hi(b[j]));
-        v[i][j] = s;
-        const float lo = Elem<E>::lo(s), hi = Elem<E>::hi(s);
-        ss += lo * lo + hi * hi;
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = threadIdx.x + i * kFusedThreads;
+      if (c < chunks) {
+        v[r][i] = ROWS > 1 ? ld16_nt(xr + c * 8) : ld16(xr + c * 8);
+        b[r][i] = ROWS > 1 ? ld16_nt(rr + c * 8) : ld16(rr + c * 8);
       }
-      st16(rr + c * 8, v[i]);
     }
   }
-  ss = block_sum4(ss, red);
-  const float rstd = rsqrtf(ss / (float)n + eps);
+  if (ROWS > 1) {
 #pragma unroll
-  for (int i = 0; i < ITERS; ++i) {
-    const int c = threadIdx.x + i * kFusedThreads;
-    if (c < chunks) {
-      const u32x4 wv = ld16(w + c * 8);
-      u32x4 o;
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = threadIdx.x + i * kFusedThreads;
+      if (c < chunks) wv[i] = ld16(w + c * 8);
+    }
+  }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float a = Elem<E>::lo(v[i][j]) * rstd, b = Elem<E>::hi(v[i][j]) * rstd;
-        if (ROUND_FIRST) {
-          a = rnd<E>(a);
-          b = rnd<E>(b);
+  for (int r = 0; r < ROWS; ++r) {
+    const bool live = row0 + r < rows;
+    uint16_t* rr = residual + (row0 + r) * r_stride;
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = threadIdx.x + i * kFusedThreads;
+      if (c < chunks) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // the sum is stored (rounded) as the new residual, and the norm runs on the stored value
+          const uint32_t xw = v[r][i][j], bw = b[r][i][j];
+          const uint32_t s = pack2<E>(Elem<E>::lo(xw) + Elem<E>::lo(bw), Elem<E>::hi(xw) + Elem<E>::hi(bw));
+          v[r][i][j] = s;
+          const float lo = Elem<E>::lo(s), hi = Elem<E>::hi(s);
+          ss += lo * lo + hi * hi;
         }
-        o[j] = pack2<E>(a * Elem<E>::lo(wv[j]), b * Elem<E>::hi(wv[j]));
+        if (live) st16(rr + c * 8, v[r][i]);
       }
-      st16(orow + c * 8, o);
+    }
+    ss = group_sum<64>(ss);
+    if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = ss;
+  }
+  __syncthreads();
+  if (ROWS == 1) {
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = threadIdx.x + i * kFusedThreads;
+      if (c < chunks) wv[i] = ld16(w + c * 8);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    if (row0 + r >= rows) break;
+    const float rstd = rsqrtf((red[r][0] + red[r][1] + red[r][2] + red[r][3]) / (float)n + eps);
+    uint16_t* orow = out + (row0 + r) * out_stride;
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = threadIdx.x + i * kFusedThreads;
+      if (c < chunks) {
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float lo = Elem<E>::lo(v[r][i][j]) * rstd, hi = Elem<E>::hi(v[r][i][j]) * rstd;
+          if (ROUND_FIRST) {
+            lo = rnd<E>(lo);
+            hi = rnd<E>(hi);
+          }
+          o[j] = pack2<E>(lo * Elem<E>::lo(wv[i][j]), hi * Elem<E>::hi(wv[i][j]));
+        }
+        st16(orow + c * 8, o);
+      }
     }
   }
 }
@@ -116,13 +159,26 @@ static int launch_add_rms(void* out, void* residual, const void* x, const void* 
   dim3 grid((unsigned)rows), block(kFusedThreads);
   if (vec) {
     const int iters = (int)((n / 8 + kFusedThreads - 1) / kFusedThreads);
-#define PH_ARMS(I) \
-  hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, xs, rs, os)
+    // Three rows per workgroup from ten workgroups per compute unit on: with three or four each, the units that get one
+    // more than the others are what the launch waits for (2500 rows of 5120: 20.3 us with one row, 21.3 with three).
+    const bool multi = rows >= 8192 && iters <= 4;
+    const dim3 vgrid((unsigned)(multi ? (rows + 2) / 3 : rows));
+#define PH_ARMS(I)                                                                                            \
+  do {                                                                                                        \
+    if (multi)                                                                                                \
+      hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF, 3>), vgrid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, \
+                         xs, rs, os);                                                                         \
+    else                                                                                                      \
+      hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF, 1>), vgrid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, \
+                         xs, rs, os);                                                                         \
+  } while (0)
     if (iters <= 1) PH_ARMS(1);
     else if (iters <= 2) PH_ARMS(2);
     else if (iters <= 3) PH_ARMS(3);
     else if (iters <= 4) PH_ARMS(4);
-    else PH_ARMS(8);
+    else
+      hipLaunchKernelGGL((add_rms_norm_vec<E, 8, RF, 1>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, xs, rs,
+                         os);
 #undef PH_ARMS
   } else {
     hipLaunchKernelGGL((add_rms_norm_generic<E, RF>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, xs, rs, os);
@@ -137,21 +193,44 @@ __device__ __forceinline__ float silu_mul_one(float g, float u) {
   return s * u;
 }
 
-template <typename E>
+// UN 16-byte chunks per thread, a workgroup's chunks consecutive over the rows, all loads before the first exponential
+// and past the caches (gate and up are read once).  Bound by HBM, with the exponential and the division close behind:
+// index arithmetic in 64 bits and a second trip around the loop cost as much as the loads' policy.  13,824 wide bf16,
+// 9404 rows: 146.9 us with 64-bit indexes, plain loads and a capped grid, 136.5 with 32-bit indexes and no cap, 127.8
+// with non-temporal loads too, 125.7 with two chunks per thread; 11,008 wide fp16, 9404 rows 113.3 -> 95.1, 3000 rows
+// 33.9 -> 33.4 us.
+template <typename E, typename IDX, int UN>
 __global__ __launch_bounds__(256) void silu_mul_vec(uint16_t* __restrict__ out, const uint16_t* __restrict__ gate,
-                                                    const uint16_t* __restrict__ up, int64_t rows, int chunks,
+                                                    const uint16_t* __restrict__ up, IDX total, IDX chunks,
                                                     int64_t g_stride, int64_t u_stride, int64_t o_stride) {
-  const int64_t total = rows * chunks;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t r = i / chunks;
-    const int c = (int)(i - r * chunks) * 8;
-    const u32x4 g = ld16(gate + r * g_stride + c), u = ld16(up + r * u_stride + c);
-    u32x4 o;
+  for (IDX i0 = (IDX)blockIdx.x * (256 * UN) + threadIdx.x; i0 < total; i0 += (IDX)gridDim.x * (256 * UN)) {
+    u32x4 g[UN], u[UN];
+    uint16_t* dst[UN];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] = pack2<E>(silu_mul_one<E>(Elem<E>::lo(g[j]), Elem<E>::lo(u[j])),
-                      silu_mul_one<E>(Elem<E>::hi(g[j]), Elem<E>::hi(u[j])));
-    st16(out + r * o_stride + c, o);
+    for (int k = 0; k < UN; ++k) {
+      const IDX i = i0 + k * 256;
+      if (i < total) {
+        const IDX r = i / chunks;
+        const int64_t c = (int64_t)(i - r * chunks) * 8;
+        const uint16_t *gp = gate + (int64_t)r * g_stride + c, *upp = up + (int64_t)r * u_stride + c;
+        g[k] = ld16_nt(gp);
+        u[k] = ld16_nt(upp);
+        dst[k] = out + (int64_t)r * o_stride + c;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < UN; ++k) {
+      if (i0 + k * 256 < total) {
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t gw = g[k][j], uw = u[k][j];
+          o[j] = pack2<E>(silu_mul_one<E>(Elem<E>::lo(gw), Elem<E>::lo(uw)),
+                          silu_mul_one<E>(Elem<E>::hi(gw), Elem<E>::hi(uw)));
+        }
+        st16(dst[k], o);
+      }
+    }
   }
 }
 
@@ -173,16 +252,22 @@ static int launch_silu_mul(void* out, const void* gate, const void* up, int64_t 
                            int64_t us, int64_t os, hipStream_t st) {
   const bool vec = d % 8 == 0 && gs % 8 == 0 && us % 8 == 0 && os % 8 == 0 && aligned16(out) && aligned16(gate) &&
                    aligned16(up);
-  const int64_t work = vec ? rows * (d / 8) : rows * d;
-  int64_t blocks = (work + 255) / 256;
-  if (blocks > 256 * 64) blocks = 256 * 64;
-  dim3 grid((unsigned)blocks), block(256);
-  if (vec)
-    hipLaunchKernelGGL((silu_mul_vec<E>), grid, block, 0, st, (uint16_t*)out, (const uint16_t*)gate,
-                       (const uint16_t*)up, rows, (int)(d / 8), gs, us, os);
-  else
-    hipLaunchKernelGGL((silu_mul_generic<E>), grid, block, 0, st, (uint16_t*)out, (const uint16_t*)gate,
-                       (const uint16_t*)up, rows, (int)d, gs, us, os);
+  const dim3 block(256);
+  if (vec) {
+    const int64_t chunks = d / 8, total = rows * chunks;
+#define PH_SILU(IDX, UN, BLOCKS)                                                                                 \
+  hipLaunchKernelGGL((silu_mul_vec<E, IDX, UN>), dim3((unsigned)(BLOCKS)), block, 0, st, (uint16_t*)out,           \
+                     (const uint16_t*)gate, (const uint16_t*)up, (IDX)total, (IDX)chunks, gs, us, os)
+    if (total < 256 * 512) PH_SILU(uint32_t, 1, (total + 255) / 256);  // two workgroups a unit: as many as there can be
+    else if (total < (int64_t)1 << 30) PH_SILU(uint32_t, 2, (total + 511) / 512);  // no index passes 2^32
+    else PH_SILU(int64_t, 2, 256 * 64);
+#undef PH_SILU
+  } else {
+    int64_t blocks = (rows * d + 255) / 256;
+    if (blocks > 256 * 64) blocks = 256 * 64;
+    hipLaunchKernelGGL((silu_mul_generic<E>), dim3((unsigned)blocks), block, 0, st, (uint16_t*)out,
+                       (const uint16_t*)gate, (const uint16_t*)up, rows, (int)d, gs, us, os);
+  }
   return launch_status();
 }
 

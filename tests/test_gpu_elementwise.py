@@ -346,6 +346,26 @@ def test_fused_add_rms_norm(dev, dtype, rows, n):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [8191, 8192, 8193, 8194])
+@pytest.mark.parametrize("n", [8, 2056, 8192, 8200])
+def test_fused_add_rms_norm_rows_per_workgroup(dev, dtype, rows, n):
+    """Around the row count at which a workgroup takes three rows, whole and partial last workgroups, row widths of one
+    chunk to more than four per thread, strided inputs: the sum is a rounded add (exact), the norm equals the norm
+    kernel on the stored sum, and the rows behind the last stay as they were."""
+    from parrotserve_amd import kernels
+
+    g = torch.Generator().manual_seed(18)
+    x = torch.randn(rows, n + 8, generator=g).to(dtype).to(dev)[:, :n]
+    buf = torch.randn(rows + 2, n + 16, generator=g).to(dtype).to(dev)
+    w = (torch.rand(n, generator=g) + 0.5).to(dtype).to(dev)
+    want = buf.clone()
+    want[:rows, :n] = x + buf[:rows, :n]
+    y = kernels.fused_add_rms_norm(x, buf[:rows, :n], w, 1e-6)
+    assert torch.equal(_bits(buf), _bits(want))
+    assert torch.equal(_bits(y), _bits(kernels.vllm_rms_norm(want[:rows, :n], w, 1e-6)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,d", [(128, 13824), (9, 11008), (3, 100), (1, 7)])
 def test_silu_mul(dev, dtype, rows, d):
     from oracle.ref_ops import ref_silu_mul
@@ -362,6 +382,24 @@ def test_silu_mul(dev, dtype, rows, d):
     assert torch.equal(_bits(out2.cpu()), _bits(out.cpu()))
     sep = kernels.silu_mul(dgu[:, :d].contiguous(), dgu[:, d:].contiguous())
     assert torch.equal(_bits(sep.cpu()), _bits(out.cpu()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,d", [(1, 8 * 131071), (1, 8 * 131072), (129, 8 * 1017), (8193, 136)])
+def test_silu_mul_chunks_per_thread(dev, dtype, rows, d):
+    """Around the size at which a thread takes two chunks, with a partial last workgroup: bit for bit what rows small
+    enough for one chunk per thread give."""
+    from parrotserve_amd import kernels
+
+    g = torch.Generator().manual_seed(19)
+    gu = (torch.randn(rows, 2 * d, generator=g) * 2).to(dtype).to(dev)
+    gate, up = gu[:, :d], gu[:, d:]
+    buf = torch.zeros(rows * d + 8, dtype=dtype, device=dev)
+    out = kernels.silu_mul(gate, up, buf[:rows * d].view(rows, d))
+    gf, uf = gate.reshape(-1), up.reshape(-1)
+    parts = [kernels.silu_mul(gf[None, i:i + 65536], uf[None, i:i + 65536])[0] for i in range(0, rows * d, 65536)]
+    assert torch.equal(_bits(out).view(-1), _bits(torch.cat(parts)))
+    assert not buf[rows * d:].any()
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
