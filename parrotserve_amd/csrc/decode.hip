@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void fold_parts_kernel(FoldArgs a) {
   for (int s = 0; s < a.n_splits; ++s) {
     const float2 ml = *reinterpret_cast<const float2*>(mlp + s * pairs * 2);
     const float4_t o = __builtin_nontemporal_load(reinterpret_cast<const float4_t*>(op + s * pairs * a.D));
-    const bool live = ml.y > 0.f;  // l == 0 marks an empty part (its O may be garbage)
+    const bool live = ml.y != 0.f;  // l == 0 marks an empty part (its O may be garbage); a NaN stays in the result
     const float Mn = fmaxf(M, live ? ml.x : -INFINITY);
     const float sc = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
     const float wgt = live ? __builtin_amdgcn_exp2f(ml.x - Mn) * ml.y : 0.f;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void fold_parts_kernel(FoldArgs a) {
     for (int k = 0; k < 4; ++k) acc[k] = acc[k] * sc + (live ? wgt * o[k] : 0.f);
     M = Mn;
   }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = L != 0.f ? 1.f / L : 0.f;
   const int64_t row = rh / a.H;
   const u32x2 v = {pack2<E>(acc[0] * inv, acc[1] * inv), pack2<E>(acc[2] * inv, acc[3] * inv)};
   *reinterpret_cast<u32x2*>(a.out + row * a.out_stride + (rh - row * a.H) * a.D + d) = v;

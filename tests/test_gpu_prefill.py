@@ -224,6 +224,40 @@ def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, dtype):
         _lib.PH_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bad", ["key nan", "key inf", "query nan", "query inf", "value nan"])
+@pytest.mark.parametrize("T,parent,D", [
+    (61, 1987, 128),   # parts of one 64-query tile
+    (300, 3000, 128),  # parts of several tiles
+    (33, 1500, 96),    # short heads
+    (33, 500, 128),    # few parts
+])
+def test_prefill_in_parts_keeps_non_finite_values(dev, T, parent, D, bad, dtype):
+    """A non-finite key, value or query in a prefill in parts: NaN wherever the same attention in plain fp32 has it,
+    the other heads and queries as without it."""
+    from parrotserve_amd import kernels
+
+    H, head, n = 4, 1, parent + T
+    g = torch.Generator().manual_seed(77 + T)
+    q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (T, n, n))
+    what, value = bad.split()
+    {"key": k, "value": v, "query": q}[what][T // 2 if what == "query" else parent // 2, head, 5] = float(value)
+    qf, kf, vf = (x.float().transpose(0, 1).contiguous() for x in (q, k, v))
+    s = (qf @ kf.transpose(1, 2).contiguous()) * D ** -0.5
+    s.masked_fill_(torch.arange(n)[None, None, :] > parent + torch.arange(T)[None, :, None], -float("inf"))
+    ref = (torch.softmax(s, dim=-1) @ vf).transpose(0, 1)
+    assert ref.isnan().any() and not ref[:, 0].isnan().any()
+
+    tables = kernels.PrefillTables.build([T], [list(range(n))], dev)
+    out = kernels.prefill_attention(q.to(dev), k.to(dev), v.to(dev), tables).cpu().float()
+    assert out[ref.isnan()].isnan().all()
+    others = torch.arange(H) != head
+    torch.testing.assert_close(out[:, others], ref[:, others], **TOL[dtype])
+    if what == "query":
+        queries = torch.arange(T) != T // 2
+        torch.testing.assert_close(out[queries], ref[queries], **TOL[dtype])
+
+
 @pytest.mark.parametrize("chunks", [64, 65, 130, 256, 257])
 def test_prefill_chunk_counts_around_the_tile_search(dev, chunks):
     """Chunk counts at the edges of the in-kernel tile search (64 chunks a round, a pre-pass beyond 256)."""
