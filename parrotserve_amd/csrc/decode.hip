@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
 
   if (a.prev_m && w == 0) {  // a partial already sitting in out / prev_m / prev_l
     const float lp = a.prev_l[(int64_t)b * a.H + head];
-    if (lp > 0.f) {
+    if (lp != 0.f) {
       float ov[8];
       load8f<E>(a.out, (int64_t)b * a.out_stride + (int64_t)head * D + dl, ov);
       M = a.prev_m[(int64_t)b * a.H + head];
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     const float2 mlp = *reinterpret_cast<const float2*>(mlrow);
     const float4_t o0 = *reinterpret_cast<const float4_t*>(op);
     const float4_t o1 = *reinterpret_cast<const float4_t*>(op + 4);
-    const bool live = mlp.y > 0.f;  // l == 0 marks an empty part (its O may be garbage)
+    const bool live = mlp.y != 0.f;  // l == 0 marks an empty part (its O may be garbage); a NaN stays in the result
     const float mp = live ? mlp.x : -INFINITY;
     const float Mn = fmaxf(M, mp);
     const float sc = (M == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     M = Mn;
   }
   if (!head_ok || !HeadLanes<D>::active(lane)) return;
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = L != 0.f ? 1.f / L : 0.f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) acc[k] *= inv;
   store8f<E>(a.out, (int64_t)b * a.out_stride + (int64_t)head * D + dl, acc);

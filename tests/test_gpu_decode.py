@@ -575,6 +575,41 @@ def test_timed_call_is_the_same_call_with_timestamps(dev):
         torch.testing.assert_close(timed.cpu().float(), ref.float(), **TOL[torch.float16])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bad", ["prefix key", "own key", "own value", "query"])
+@pytest.mark.parametrize("H,D,P,own", [(8, 128, 1000, 40), (8, 64, 700, 40), (3, 256, 300, 40), (8, 128, 0, 900)])
+def test_nan_inputs_stay_in_the_result(dev, H, D, P, own, bad, dtype):
+    """A NaN in one key, value or query: NaN wherever the same attention in plain fp32 has it, the requests that do not
+    see it as without it."""
+    from parrotserve_amd import kernels
+
+    if P == 0 and bad == "prefix key":
+        pytest.skip("no prefix")
+    B, head, b = 6, 1, 3
+    g = torch.Generator().manual_seed(91 + P + D)
+    q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (B, P + B * own, P + B * own))
+    {"prefix key": k, "own key": k, "own value": v, "query": q}[bad][
+        {"prefix key": P // 2, "query": b}.get(bad, P + b * own + own // 2), head, 5] = float("nan")
+    lists = [list(range(P + i * own, P + (i + 1) * own)) for i in range(B)]
+    rows = []
+    for i in range(B):
+        ix = list(range(P)) + lists[i]
+        kf, vf = k[ix].float().transpose(0, 1).contiguous(), v[ix].float().transpose(0, 1).contiguous()
+        s = (kf * q[i].float()[:, None]).sum(-1) * D ** -0.5
+        rows.append((torch.softmax(s, dim=-1)[:, None] @ vf)[:, 0])
+    ref = torch.stack(rows)
+    assert ref.isnan().any()
+
+    tables = kernels.DecodeTables.build([list(range(P))] if P else [], [0, B] if P else [0], lists, dev, num_heads=H,
+                                        head_dim=D, dtype=dtype)
+    out = kernels.decode_attention(q.to(dev), k.to(dev), v.to(dev), tables).cpu().float()
+    assert out[ref.isnan()].isnan().all()
+    tol = TOL.get(dtype, dict(atol=1e-4, rtol=1e-4))
+    if bad != "prefix key":
+        torch.testing.assert_close(out[torch.arange(B) != b], ref[torch.arange(B) != b], **tol)
+    torch.testing.assert_close(out[:, 2:], ref[:, 2:], **tol)  # heads 0 and 1 may share a row of the wide tile
+
+
 @pytest.mark.parametrize("balanced", [True, False])
 def test_lengths_beyond_the_table_are_clamped(dev, balanced):
     """A context length larger than the table's width must not walk into the next request's row (or past the
