@@ -430,6 +430,12 @@ size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_heads, int64_t
                                   int64_t max_kv_len);
 size_t ph_prefill_workspace_min_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
                                       int64_t max_kv_len);
+/* How a ph_prefill_attention call of these sizes with such a workspace is launched: queries per
+ * workgroup (64, 128 or 256; 1 where every token is a row of its own) and parts every context is
+ * cut into.  Host-only, no launch. */
+int ph_prefill_plan(int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim, int dtype,
+                    int64_t max_kv_len, int64_t ctx_slots_count, size_t workspace_bytes,
+                    int32_t* tile_queries, int32_t* parts);
 
 int ph_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
                          int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim,

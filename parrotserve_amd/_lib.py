@@ -52,6 +52,7 @@ SIGNATURES: Dict[str, Tuple[object, List[object]]] = {
     "ph_top_p_probs": (I, [P, L, P, P, P, L, L, L, I, P]),
     "ph_prefill_workspace_bytes": (Z, [L, L, L, I, L]),
     "ph_prefill_workspace_min_bytes": (Z, [L, L, L, I, L]),
+    "ph_prefill_plan": (I, [L, L, L, L, I, L, L, Z, P, P]),
     "ph_prefill_attention": (I, [P, P, P, P, L, L, L, L, I, L, L, L, F, P, P, P, L, L, P, Z, P]),
 }
 

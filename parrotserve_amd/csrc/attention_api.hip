@@ -411,11 +411,12 @@ static size_t prefill_part_bytes(int64_t T, int64_t H, int64_t D, int64_t splits
 }
 // Estimated time of a launch (microseconds): rounds of one workgroup per compute unit, each a fixed start and end and
 // its steps, no faster than the K/V rows come from memory; a split launch adds the parts' write and fold.  The host
-// knows the query total, the chunk count and the longest context: tiles per chunk and visible lengths are averages.
+// knows the query total, the chunk count, the longest context and the sum of all contexts (kv_rows): tiles per chunk
+// and visible lengths are averages, and the longest context bounds the launch from below.
 // Constants fitted to 27 shapes in bf16 (1 to 16 chunks of 16 to 4096 tokens over parents of 0 to 6000, 32 and 40
 // heads), every tile with 1 to 16 splits: the choice is within 8 % of the best form on 24 of them, 20 % on one.
-static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int tile_q, int64_t splits,
-                              int64_t cus) {
+static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int64_t kv_rows, int tile_q,
+                              int64_t splits, int64_t cus) {
   const double start = tile_q == 256 ? 9.0 : 8.5;
   const double step = tile_q == 256 ? 1.46 : tile_q == 128 ? 0.96 : 1.16;  // on a lightly loaded device
   const int64_t step_tokens = tile_q == 64 ? 128 : 64;
@@ -426,10 +427,10 @@ static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_
   const double wgs = tiles * H * splits;
   const double rounds = std::ceil(wgs / cus - 1e-9);
   const double step_loaded = step * (1.0 + 0.25 * std::min(1.0, wgs / (rounds * cus)));  // clock and memory under load
-  const double seen = std::max(1.0, max_kv - 0.5 * std::max(0.0, avg - tile_q));        // of an average tile
+  const double seen = std::max(1.0, (double)kv_rows / C - 0.5 * std::max(0.0, avg - tile_q));  // of an average tile
   auto walk = [&](double tokens) { return start + std::ceil(tokens / step_tokens / splits) * step_loaded; };
   double t = std::max(rounds * walk(seen), walk((double)max_kv));
-  const double kv_mb = (double)C * max_kv * H * D * 4 / 1e6;
+  const double kv_mb = (double)kv_rows * H * D * 4 / 1e6;
   t = std::max(t, start + kv_mb / 5.5);
   if (splits > 1) t += 4.0 + (double)splits * T * H * D * 4 / 1e6 / 5.0;
   return t;
@@ -441,16 +442,18 @@ static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_
 // a short round: smaller tiles, and parts of long contexts on workgroups of their own, then go faster (bf16, one
 // chunk: 61 queries over 2048 tokens, 32 heads, 27.3 -> 18 us in 4 to 8 parts; 256 over 1256, 32 heads, 37.3 -> 19.2
 // us on 64-query tiles; 256 over 6256, 40 heads, 152 -> 58 us on 256-query tiles in 6 parts).
-static PrefillPlan plan_prefill(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, size_t workspace_bytes) {
+static PrefillPlan plan_prefill(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int64_t ctx_slots_count,
+                                size_t workspace_bytes) {
   const int64_t avg = T / C, cus = device_cus();
   PrefillPlan p{avg >= 192 ? 256 : avg >= 96 ? 128 : 64, 1};
   if (cdiv(T, p.tile_q) * H > 4 * cus || C * H > 4 * cus || C > kScanChunks) return p;
-  double best = prefill_cost_us(T, C, H, D, max_kv, p.tile_q, 1, cus);
+  const int64_t kv_rows = std::min(ctx_slots_count, C * max_kv);  // the slot list may be longer than the contexts
+  double best = prefill_cost_us(T, C, H, D, max_kv, kv_rows, p.tile_q, 1, cus);
   const int64_t max_splits = std::min(max_prefill_splits(T, H), cdiv(max_kv, 128));
   for (int64_t splits = 1; splits <= std::max<int64_t>(1, max_splits); ++splits) {
     if (splits > 1 && prefill_part_bytes(T, H, D, splits) > workspace_bytes) break;
     for (int tile_q = 256; tile_q >= 64; tile_q /= 2) {
-      const double t = prefill_cost_us(T, C, H, D, max_kv, tile_q, splits, cus);
+      const double t = prefill_cost_us(T, C, H, D, max_kv, kv_rows, tile_q, splits, cus);
       if (t < 0.95 * best) {  // an estimate that is no clear gain changes nothing
         best = t;
         p = PrefillPlan{tile_q, (int)splits};
@@ -1083,6 +1086,21 @@ extern "C" size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_hea
   return splits > 1 ? std::max(least, prefill_part_bytes(num_tokens, num_heads, head_dim, splits)) : least;
 }
 
+extern "C" int ph_prefill_plan(int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim, int dtype,
+                               int64_t max_kv_len, int64_t ctx_slots_count, size_t workspace_bytes,
+                               int32_t* tile_queries, int32_t* parts) {
+  if (num_tokens <= 0 || num_chunks <= 0 || num_chunks > num_tokens || num_heads <= 0 || head_dim <= 0 ||
+      max_kv_len <= 0 || max_kv_len > INT32_MAX || ctx_slots_count <= 0 || !tile_queries || !parts)
+    return PH_ERR_ARG;
+  const PrefillPlan p = prefill_on_matrix_cores(dtype, head_dim, num_heads)
+                            ? plan_prefill(num_tokens, num_chunks, num_heads, head_dim, max_kv_len, ctx_slots_count,
+                                           workspace_bytes)
+                            : PrefillPlan{1, 1};
+  *tile_queries = p.tile_q;
+  *parts = p.splits;
+  return PH_OK;
+}
+
 extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
                                     int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim,
                                     int dtype, int64_t q_stride, int64_t out_stride, int64_t cache_stride_n,
@@ -1119,7 +1137,8 @@ extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cach
     pa.H = H;
     pa.scale_log2e = scale * kLog2e;
     pa.pair = paired ? 1 : 0;
-    const PrefillPlan pp = plan_prefill(num_tokens, num_chunks, num_heads, head_dim, max_kv_len, workspace_bytes);
+    const PrefillPlan pp =
+        plan_prefill(num_tokens, num_chunks, num_heads, head_dim, max_kv_len, ctx_slots_count, workspace_bytes);
     pa.n_splits = pp.splits;
     if (pp.splits > 1) {
       pa.opart = (float*)workspace;

@@ -1,5 +1,6 @@
 """The C-ABI library loads and exports every symbol include/parrot_hip.h declares
 (no compute calls: this runs without a GPU)."""
+import ctypes
 import os
 import re
 
@@ -73,6 +74,28 @@ def test_how_the_planner_divides_a_256_unit_device():
     assert lanes(64, 32, 128, f16, 1, 4096, 512, 4) > 2 * lanes(64, 32, 128, f16, 1, 4096, 512, 1)
     assert lanes(64, 32, 128, f16, 1, 4096, 60, 4) <= 256
     assert lanes(64, 32, 128, f16, 0, 0, 512, 2) == 256
+
+
+def _prefill_plan(q_lens, ctx_lens, heads, dim=128, workspace=1 << 40, spare_slots=0):
+    from parrotserve_amd import _lib
+
+    tile, parts = ctypes.c_int32(), ctypes.c_int32()
+    assert _lib.load().ph_prefill_plan(sum(q_lens), len(q_lens), heads, dim, _lib.PH_BF16, max(ctx_lens),
+                                       sum(ctx_lens) + spare_slots, workspace, ctypes.byref(tile),
+                                       ctypes.byref(parts)) == _lib.PH_OK
+    return tile.value, parts.value
+
+
+def test_how_a_prefill_over_contexts_of_different_lengths_is_planned():
+    """The planner prices the contexts it is given, not every chunk as long as the longest: one long context among short
+    ones is cut into parts, and a launch that ends on its longest context keeps the tile that fits its chunks."""
+    assert _prefill_plan([16] * 4, [8192, 64, 64, 64], 32) == (64, 4)
+    assert _prefill_plan([16] * 8, [6000] + [100] * 7, 32) == (64, 3)
+    assert _prefill_plan([64] * 4, [4096, 512, 512, 512], 32) == (64, 2)
+    assert _prefill_plan([61] * 6, [100, 200, 400, 800, 1600, 3200], 32) == (64, 1)
+    assert _prefill_plan([2, 303, 46, 2, 25], [2, 369, 235, 2, 2172], 32) == (64, 1)
+    # a slot list with room behind the contexts is priced no higher than contexts all as long as the longest
+    assert _prefill_plan([16] * 4, [8192] * 4, 32) == _prefill_plan([16] * 4, [8192] * 4, 32, spare_slots=1 << 20)
 
 
 def test_argument_validation_needs_no_gpu():

@@ -258,6 +258,34 @@ def test_prefill_in_parts_keeps_non_finite_values(dev, T, parent, D, bad, dtype)
         torch.testing.assert_close(out[queries], ref[queries], **TOL[dtype])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("q_lens,ctx_lens,D", [
+    ([16] * 4, [8192, 64, 64, 64], 128),                      # parts made for one long context: the others fill one
+    ([64, 3, 64, 1], [512, 4100, 64, 1], 128),                # the long one in the middle, a chunk of one token
+    ([61] * 6, [100, 200, 400, 800, 1600, 3200], 96),
+    ([256, 40], [6256, 40], 64),
+])
+def test_prefill_contexts_of_different_lengths(dev, q_lens, ctx_lens, D, dtype):
+    """Chunks over contexts of very different lengths in one launch against plain fp32 attention."""
+    from parrotserve_amd import kernels
+
+    H = 8
+    g = torch.Generator().manual_seed(5 + sum(ctx_lens))
+    n = sum(ctx_lens)
+    q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (sum(q_lens), n, n))
+    slots, ref, lists, at = torch.randperm(n, generator=g), [], [], 0
+    for new, length in zip(q_lens, ctx_lens):
+        lists.append(slots[sum(ctx_lens[:len(lists)]):][:length])
+        qf, kf, vf = (x.float().transpose(0, 1).contiguous() for x in (q[at:at + new], k[lists[-1]], v[lists[-1]]))
+        s = (qf @ kf.transpose(1, 2).contiguous()) * D ** -0.5
+        s.masked_fill_(torch.arange(length)[None, None, :] > length - new + torch.arange(new)[None, :, None], -float("inf"))
+        ref.append((torch.softmax(s, dim=-1) @ vf).transpose(0, 1))
+        at += new
+    tables = kernels.PrefillTables.build(q_lens, [x.tolist() for x in lists], dev)
+    out = kernels.prefill_attention(q.to(dev), k.to(dev), v.to(dev), tables)
+    torch.testing.assert_close(out.cpu().float(), torch.cat(ref), **TOL[dtype])
+
+
 @pytest.mark.parametrize("chunks", [64, 65, 130, 256, 257])
 def test_prefill_chunk_counts_around_the_tile_search(dev, chunks):
     """Chunk counts at the edges of the in-kernel tile search (64 chunks a round, a pre-pass beyond 256)."""
