@@ -98,6 +98,16 @@ def test_how_a_prefill_over_contexts_of_different_lengths_is_planned():
     assert _prefill_plan([16] * 4, [8192] * 4, 32) == _prefill_plan([16] * 4, [8192] * 4, 32, spare_slots=1 << 20)
 
 
+def test_parts_have_to_promise_more_than_another_tile():
+    """Parts are taken for a clear estimated gain only: a chunk of 1024 queries over 3024 tokens of 40 heads, whose parts
+    were estimated 6 % faster and measured 11 % slower, keeps one part; the short chunks that parts are for get them."""
+    assert _prefill_plan([1024], [3024], 40) == (256, 1)
+    assert _prefill_plan([61], [2048], 32) == (64, 4)
+    assert _prefill_plan([1], [2001], 32) == (64, 4)
+    assert _prefill_plan([256], [6256], 40) == (256, 6)
+    assert _prefill_plan([1024], [7024], 32) == (256, 2)
+
+
 def test_argument_validation_needs_no_gpu():
     """Bad arguments are rejected before any launch."""
     from parrotserve_amd import _lib
