@@ -424,8 +424,9 @@ int ph_prefix_post_attention(void* out, const float* prev_m, const float* prev_l
  * The new tokens' K/V must already be in the cache (append first).
  * max_kv_len: host upper bound of any chunk's context length.
  * workspace: at least ph_prefill_workspace_min_bytes(...) bytes, 256-byte aligned.  With
- * ph_prefill_workspace_bytes(...) every plan fits: few queries over long contexts are then cut into
- * parts whose partial results live there. */
+ * ph_prefill_workspace_bytes(...) every plan of calls up to these sizes fits: few queries over long
+ * contexts are then cut into parts whose partial results live there.  Neither size falls as
+ * num_tokens or max_kv_len grows. */
 size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,
                                   int64_t max_kv_len);
 size_t ph_prefill_workspace_min_bytes(int64_t num_tokens, int64_t num_heads, int64_t head_dim, int dtype,

@@ -401,13 +401,27 @@ struct PrefillPlan {
   int tile_q, splits;
 };
 constexpr int kMaxPrefillSplits = 16;
-// most splits a launch of T query rows can take whatever its chunks: two rounds of workgroups
-static int64_t max_prefill_splits(int64_t T, int64_t H) {
-  const int64_t s = 2 * device_cus() / (cdiv(T, 256) * H);
-  return std::min<int64_t>(kMaxPrefillSplits, s);
+// most splits a launch of T query rows can take whatever its chunks: one round of workgroups, at least a step of the
+// 64-query tile (128 tokens) each.  (Two rounds were no faster: 23 shapes of 512 to 8192 queries over 6000 to 20,000
+// tokens took 0.90 to 1.09 of their time with one, half of them more, and twice the workspace.)
+static int64_t max_prefill_splits(int64_t T, int64_t H, int64_t max_kv) {
+  const int64_t s = device_cus() / (cdiv(T, 256) * H);
+  return std::min({(int64_t)kMaxPrefillSplits, s, cdiv(max_kv, 128)});
 }
 static size_t prefill_part_bytes(int64_t T, int64_t H, int64_t D, int64_t splits) {
   return (size_t)round_up(splits * T * H * D * 4, 256) + (size_t)round_up(splits * T * H * 2 * 4, 256);
+}
+// Room for the parts of any launch of up to T query rows: shorter calls take more parts, so a workspace sized for the
+// longest call has to hold what the shorter ones cut (at most 65,536 rows: 34 MB for 128-wide heads).
+static size_t prefill_parts_room(int64_t T, int64_t H, int64_t D, int64_t max_kv) {
+  size_t most = 0;
+  for (int64_t t = 256;; t += 256) {
+    const int64_t rows = std::min(t, T), splits = max_prefill_splits(rows, H, max_kv);
+    if (splits <= 1) break;
+    most = std::max(most, prefill_part_bytes(rows, H, D, splits));
+    if (rows == T) break;
+  }
+  return most;
 }
 // Estimated time of a launch (microseconds): rounds of one workgroup per compute unit, each a fixed start and end and
 // its steps, no faster than the K/V rows come from memory; a split launch adds the parts' write and fold.  The host
@@ -449,7 +463,7 @@ static PrefillPlan plan_prefill(int64_t T, int64_t C, int64_t H, int64_t D, int6
   if (cdiv(T, p.tile_q) * H > 4 * cus || C * H > 4 * cus || C > kScanChunks) return p;
   const int64_t kv_rows = std::min(ctx_slots_count, C * max_kv);  // the slot list may be longer than the contexts
   double best = prefill_cost_us(T, C, H, D, max_kv, kv_rows, p.tile_q, 1, cus);
-  const int64_t max_splits = std::min(max_prefill_splits(T, H), cdiv(max_kv, 128));
+  const int64_t max_splits = max_prefill_splits(T, H, max_kv);
   for (int64_t splits = 1; splits <= std::max<int64_t>(1, max_splits); ++splits) {
     if (splits > 1 && prefill_part_bytes(T, H, D, splits) > workspace_bytes) break;
     for (int tile_q = 256; tile_q >= 64; tile_q /= 2) {
@@ -1085,8 +1099,7 @@ extern "C" size_t ph_prefill_workspace_bytes(int64_t num_tokens, int64_t num_hea
                                              int64_t max_kv_len) {
   const size_t least = ph_prefill_workspace_min_bytes(num_tokens, num_heads, head_dim, dtype, max_kv_len);
   if (least == 0 || !prefill_on_matrix_cores(dtype, head_dim, num_heads)) return least;
-  const int64_t splits = max_prefill_splits(num_tokens, num_heads);
-  return splits > 1 ? std::max(least, prefill_part_bytes(num_tokens, num_heads, head_dim, splits)) : least;
+  return std::max(least, prefill_parts_room(num_tokens, num_heads, head_dim, max_kv_len));
 }
 
 extern "C" int ph_prefill_plan(int64_t num_tokens, int64_t num_chunks, int64_t num_heads, int64_t head_dim, int dtype,

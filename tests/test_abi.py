@@ -108,6 +108,29 @@ def test_parts_have_to_promise_more_than_another_tile():
     assert _prefill_plan([1024], [7024], 32) == (256, 2)
 
 
+@pytest.mark.parametrize("heads,dim", [(32, 128), (40, 128), (4, 128), (32, 64), (12, 96)])
+def test_a_prefill_workspace_for_the_largest_call_serves_the_smaller_ones(heads, dim):
+    """The workspace protocol is one allocation for the largest call: sizes do not fall as the call grows, and every
+    smaller call is planned in it as it is in a workspace without limit."""
+    from parrotserve_amd import _lib
+
+    lib = _lib.load()
+    tokens, contexts = [1, 61, 255, 256, 257, 500, 1024, 2048, 2049, 9404], [130, 700, 2048, 6256, 20000]
+    size = lambda t, kv: lib.ph_prefill_workspace_bytes(t, heads, dim, _lib.PH_BF16, kv)
+    for kv in contexts:
+        sizes = [size(t, kv) for t in tokens]
+        assert sizes == sorted(sizes)
+        assert all(n >= lib.ph_prefill_workspace_min_bytes(t, heads, dim, _lib.PH_BF16, kv) for t, n in zip(tokens, sizes))
+    for t in tokens:
+        assert [size(t, kv) for kv in contexts] == sorted(size(t, kv) for kv in contexts)
+        for kv in contexts:
+            if kv >= t:
+                assert _prefill_plan([t], [kv], heads, dim, size(9404, 20000)) == _prefill_plan([t], [kv], heads, dim)
+    # no more than the parts that so short a context can be cut into
+    rows = 2 * 256 * heads
+    assert size(256, 256) <= rows * (dim + 2) * 4 + 1024
+
+
 def test_argument_validation_needs_no_gpu():
     """Bad arguments are rejected before any launch."""
     from parrotserve_amd import _lib
