@@ -401,11 +401,13 @@ struct PrefillPlan {
   int tile_q, splits;
 };
 constexpr int kMaxPrefillSplits = 16;
+// compute units a prefill launch can reach: head h runs on XCD h mod 8, so the busiest chiplet sets the pace
+static int64_t prefill_cus(int64_t H) { return std::max<int64_t>(1, device_cus() * H / round_up(H, 8)); }
 // most splits a launch of T query rows can take whatever its chunks: one round of workgroups, at least a step of the
 // 64-query tile (128 tokens) each.  (Two rounds were no faster: 23 shapes of 512 to 8192 queries over 6000 to 20,000
 // tokens took 0.90 to 1.09 of their time with one, half of them more, and twice the workspace.)
 static int64_t max_prefill_splits(int64_t T, int64_t H, int64_t max_kv) {
-  const int64_t s = device_cus() / (cdiv(T, 256) * H);
+  const int64_t s = prefill_cus(H) / (cdiv(T, 256) * H);
   return std::min({(int64_t)kMaxPrefillSplits, s, cdiv(max_kv, 128)});
 }
 static size_t prefill_part_bytes(int64_t T, int64_t H, int64_t D, int64_t splits) {
@@ -458,7 +460,7 @@ static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_
 // us on 64-query tiles; 256 over 6256, 40 heads, 152 -> 58 us on 256-query tiles in 6 parts).
 static PrefillPlan plan_prefill(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int64_t ctx_slots_count,
                                 size_t workspace_bytes) {
-  const int64_t avg = T / C, cus = device_cus();
+  const int64_t avg = T / C, cus = prefill_cus(H);
   PrefillPlan p{avg >= 192 ? 256 : avg >= 96 ? 128 : 64, 1};
   if (cdiv(T, p.tile_q) * H > 4 * cus || C * H > 4 * cus || C > kScanChunks) return p;
   const int64_t kv_rows = std::min(ctx_slots_count, C * max_kv);  // the slot list may be longer than the contexts

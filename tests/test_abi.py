@@ -108,6 +108,13 @@ def test_parts_have_to_promise_more_than_another_tile():
     assert _prefill_plan([1024], [7024], 32) == (256, 2)
 
 
+def test_a_prefill_of_few_heads_counts_the_chiplets_it_reaches():
+    """Head h runs on chiplet h mod 8: with two heads a quarter of the device works, with twenty five sixths of it."""
+    assert _prefill_plan([8192], [10192], 2) == (128, 1)   # 64 units: no room for parts of 32 tiles of two heads
+    assert _prefill_plan([512], [6512], 4) == (128, 8)     # 128 units: one round of the wider tile
+    assert _prefill_plan([1000], [10000], 20) == (256, 2)  # 213 units: a third part would begin a second round
+
+
 @pytest.mark.parametrize("heads,dim", [(32, 128), (40, 128), (4, 128), (32, 64), (12, 96)])
 def test_a_prefill_workspace_for_the_largest_call_serves_the_smaller_ones(heads, dim):
     """The workspace protocol is one allocation for the largest call: sizes do not fall as the call grows, and every
