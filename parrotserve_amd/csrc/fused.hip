@@ -193,13 +193,17 @@ __device__ __forceinline__ float silu_mul_one(float g, float u) {
   return s * u;
 }
 
-// UN 16-byte chunks per thread, a workgroup's chunks consecutive over the rows, all loads before the first exponential
-// and past the caches (gate and up are read once).  Bound by HBM, with the exponential and the division close behind:
-// index arithmetic in 64 bits and a second trip around the loop cost as much as the loads' policy.  13,824 wide bf16,
-// 9404 rows: 146.9 us with 64-bit indexes, plain loads and a capped grid, 136.5 with 32-bit indexes and no cap, 127.8
-// with non-temporal loads too, 125.7 with two chunks per thread; 11,008 wide fp16, 9404 rows 113.3 -> 95.1, 3000 rows
-// 33.9 -> 33.4 us.
-template <typename E, typename IDX, int UN>
+// UN 16-byte chunks per thread, a workgroup's chunks consecutive over the rows, all loads before the first exponential.
+// NT: gate and up are read past the caches.  Bound by HBM, with the exponential and the division close behind: index
+// arithmetic in 64 bits and a second trip around a capped grid cost as much as the loads' policy.  Two forms, by whether
+// gate, up and out fit the 256 MB of the last cache: there the GEMM before may have left them, and reading past it costs
+// (3000 rows of 13,824 bf16 on the same buffers: 38.4 us plain, one chunk; 44.6 past the caches, two chunks; 39.9 with
+// 64-bit indexes and a capped grid), as two chunks per thread do on launches of few workgroups (200 rows of 11,008,
+// inputs out of the caches: 4.7, 5.4).  Beyond it nothing is found there (9404 rows of 13,824 on the same buffers: 135.0
+// plain, one chunk, 124.9 past the caches, two chunks; 6200 rows 90.9, 84.8; out of the caches 133.6, 122.4 and 89.9,
+// 82.9).  At the line, 4000 rows of 13,824 (332 MB) take 58.7 and 59.9 us on the same buffers, 59.3 and 55.6 out of the
+// caches, 4000 of 11,008 (264 MB) 40.7 and 48.9, 46.1 and 45.0.
+template <typename E, typename IDX, int UN, bool NT>
 __global__ __launch_bounds__(256) void silu_mul_vec(uint16_t* __restrict__ out, const uint16_t* __restrict__ gate,
                                                     const uint16_t* __restrict__ up, IDX total, IDX chunks,
                                                     int64_t g_stride, int64_t u_stride, int64_t o_stride) {
@@ -213,8 +217,8 @@ __global__ __launch_bounds__(256) void silu_mul_vec(uint16_t* __restrict__ out, 
         const IDX r = i / chunks;
         const int64_t c = (int64_t)(i - r * chunks) * 8;
         const uint16_t *gp = gate + (int64_t)r * g_stride + c, *upp = up + (int64_t)r * u_stride + c;
-        g[k] = ld16_nt(gp);
-        u[k] = ld16_nt(upp);
+        g[k] = NT ? ld16_nt(gp) : ld16(gp);
+        u[k] = NT ? ld16_nt(upp) : ld16(upp);
         dst[k] = out + (int64_t)r * o_stride + c;
       }
     }
@@ -255,12 +259,12 @@ static int launch_silu_mul(void* out, const void* gate, const void* up, int64_t 
   const dim3 block(256);
   if (vec) {
     const int64_t chunks = d / 8, total = rows * chunks;
-#define PH_SILU(IDX, UN, BLOCKS)                                                                                 \
-  hipLaunchKernelGGL((silu_mul_vec<E, IDX, UN>), dim3((unsigned)(BLOCKS)), block, 0, st, (uint16_t*)out,           \
+#define PH_SILU(IDX, UN, NT, BLOCKS)                                                                               \
+  hipLaunchKernelGGL((silu_mul_vec<E, IDX, UN, NT>), dim3((unsigned)(BLOCKS)), block, 0, st, (uint16_t*)out,         \
                      (const uint16_t*)gate, (const uint16_t*)up, (IDX)total, (IDX)chunks, gs, us, os)
-    if (total < 256 * 512) PH_SILU(uint32_t, 1, (total + 255) / 256);  // two workgroups a unit: as many as there can be
-    else if (total < (int64_t)1 << 30) PH_SILU(uint32_t, 2, (total + 511) / 512);  // no index passes 2^32
-    else PH_SILU(int64_t, 2, 256 * 64);
+    if (total * 48 <= (int64_t)256 << 20) PH_SILU(uint32_t, 1, false, (total + 255) / 256);  // three operands of 16 bytes
+    else if (total < (int64_t)1 << 30) PH_SILU(uint32_t, 2, true, (total + 511) / 512);      // no index passes 2^32
+    else PH_SILU(int64_t, 2, true, 256 * 64);
 #undef PH_SILU
   } else {
     int64_t blocks = (rows * d + 255) / 256;
