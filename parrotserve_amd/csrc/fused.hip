@@ -193,48 +193,33 @@ __device__ __forceinline__ float silu_mul_one(float g, float u) {
   return s * u;
 }
 
-// UN 16-byte chunks per thread, a workgroup's chunks consecutive over the rows, all loads before the first exponential.
-// NT: gate and up are read past the caches.  Bound by HBM, with the exponential and the division close behind: index
-// arithmetic in 64 bits and a second trip around a capped grid cost as much as the loads' policy.  Two forms, by whether
-// gate, up and out fit the 256 MB of the last cache: there the GEMM before may have left them, and reading past it costs
-// (3000 rows of 13,824 bf16 on the same buffers: 38.4 us plain, one chunk; 44.6 past the caches, two chunks; 39.9 with
-// 64-bit indexes and a capped grid), as two chunks per thread do on launches of few workgroups (200 rows of 11,008,
-// inputs out of the caches: 4.7, 5.4).  Beyond it nothing is found there (9404 rows of 13,824 on the same buffers: 135.0
-// plain, one chunk, 124.9 past the caches, two chunks; 6200 rows 90.9, 84.8; out of the caches 133.6, 122.4 and 89.9,
-// 82.9).  At the line, 4000 rows of 13,824 (332 MB) take 58.7 and 59.9 us on the same buffers, 59.3 and 55.6 out of the
-// caches, 4000 of 11,008 (264 MB) 40.7 and 48.9, 46.1 and 45.0.
-template <typename E, typename IDX, int UN, bool NT>
+// One 16-byte chunk per thread, a workgroup's chunks consecutive over the rows.  Bound by HBM, with the exponential and
+// the division close behind: index arithmetic in 64 bits and a second trip around a capped grid cost as much as the
+// loads' policy (9404 rows of 13,824 bf16, same buffers: 143.5 us with both; 135.0 without; 125.2 past the caches too).
+// gate and up are read once; past the caches they leave the 256 MB of the last one to the passes around.  All
+// element-wise passes of a layer, 13,824 wide, on the same inputs, with plain loads and so: 4000 rows 168.6 and 159.2 us,
+// 2500 rows 109.4 and 99.9, 300 rows 22.2 and 21.4; on three sets in turn 1000 rows 48.7 and 44.8.  After a kernel that
+// writes gate and up: 3000 rows of 11,008 36.6 and 30.1, 4000 of 13,824 53.6 and 49.6, 1000 15.4 and 15.4.  (Slower where
+// everything stays in the cache: the layer's passes over 1000 rows of one set 41.8 and 45.4, the activation alone on the
+// same buffers 3000 rows 38.4 and 44.2.)  Two chunks per thread gain on the activation alone from 3000 rows on (6200
+// rows fp16 91.0, 86.1), not within the layer (5000 rows 208.0, 210.6), and cost where workgroups are few (300 rows of
+// 11,008 out of the caches 6.0, 6.6).
+template <typename E, typename IDX>
 __global__ __launch_bounds__(256) void silu_mul_vec(uint16_t* __restrict__ out, const uint16_t* __restrict__ gate,
                                                     const uint16_t* __restrict__ up, IDX total, IDX chunks,
                                                     int64_t g_stride, int64_t u_stride, int64_t o_stride) {
-  for (IDX i0 = (IDX)blockIdx.x * (256 * UN) + threadIdx.x; i0 < total; i0 += (IDX)gridDim.x * (256 * UN)) {
-    u32x4 g[UN], u[UN];
-    uint16_t* dst[UN];
+  for (IDX i = (IDX)blockIdx.x * 256 + threadIdx.x; i < total; i += (IDX)gridDim.x * 256) {
+    const IDX r = i / chunks;
+    const int64_t c = (int64_t)(i - r * chunks) * 8;
+    const u32x4 g = ld16_nt(gate + (int64_t)r * g_stride + c), u = ld16_nt(up + (int64_t)r * u_stride + c);
+    u32x4 o;
 #pragma unroll
-    for (int k = 0; k < UN; ++k) {
-      const IDX i = i0 + k * 256;
-      if (i < total) {
-        const IDX r = i / chunks;
-        const int64_t c = (int64_t)(i - r * chunks) * 8;
-        const uint16_t *gp = gate + (int64_t)r * g_stride + c, *upp = up + (int64_t)r * u_stride + c;
-        g[k] = NT ? ld16_nt(gp) : ld16(gp);
-        u[k] = NT ? ld16_nt(upp) : ld16(upp);
-        dst[k] = out + (int64_t)r * o_stride + c;
-      }
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t gw = g[j], uw = u[j];
+      o[j] = pack2<E>(silu_mul_one<E>(Elem<E>::lo(gw), Elem<E>::lo(uw)),
+                      silu_mul_one<E>(Elem<E>::hi(gw), Elem<E>::hi(uw)));
     }
-#pragma unroll
-    for (int k = 0; k < UN; ++k) {
-      if (i0 + k * 256 < total) {
-        u32x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t gw = g[k][j], uw = u[k][j];
-          o[j] = pack2<E>(silu_mul_one<E>(Elem<E>::lo(gw), Elem<E>::lo(uw)),
-                          silu_mul_one<E>(Elem<E>::hi(gw), Elem<E>::hi(uw)));
-        }
-        st16(dst[k], o);
-      }
-    }
+    st16(out + (int64_t)r * o_stride + c, o);
   }
 }
 
@@ -259,12 +244,11 @@ static int launch_silu_mul(void* out, const void* gate, const void* up, int64_t 
   const dim3 block(256);
   if (vec) {
     const int64_t chunks = d / 8, total = rows * chunks;
-#define PH_SILU(IDX, UN, NT, BLOCKS)                                                                               \
-  hipLaunchKernelGGL((silu_mul_vec<E, IDX, UN, NT>), dim3((unsigned)(BLOCKS)), block, 0, st, (uint16_t*)out,         \
+#define PH_SILU(IDX, BLOCKS)                                                                                       \
+  hipLaunchKernelGGL((silu_mul_vec<E, IDX>), dim3((unsigned)(BLOCKS)), block, 0, st, (uint16_t*)out,                 \
                      (const uint16_t*)gate, (const uint16_t*)up, (IDX)total, (IDX)chunks, gs, us, os)
-    if (total * 48 <= (int64_t)256 << 20) PH_SILU(uint32_t, 1, false, (total + 255) / 256);  // three operands of 16 bytes
-    else if (total < (int64_t)1 << 30) PH_SILU(uint32_t, 2, true, (total + 511) / 512);      // no index passes 2^32
-    else PH_SILU(int64_t, 2, true, 256 * 64);
+    if (total < (int64_t)1 << 30) PH_SILU(uint32_t, (total + 255) / 256);  // no index passes 2^32
+    else PH_SILU(int64_t, 256 * 64);
 #undef PH_SILU
   } else {
     int64_t blocks = (rows * d + 255) / 256;
