@@ -23,98 +23,62 @@ __device__ __forceinline__ float block_sum4(float v, float* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// One workgroup per ROWS consecutive rows; ITERS 16-byte chunks per thread and row stay in registers between the sum
-// and the write.  Bound by HBM (four passes over the rows).  Every load of the ROWS rows is requested before the first
-// store: x and residual may not alias, but the compiler cannot know that two chunks of the residual do not, and kept
-// each chunk's loads behind the store of the one before.  Launches of many rows read both inputs past the caches.
-// Measured with inputs out of the caches, one row per workgroup with plain interleaved loads against three with
-// non-temporal loads ahead: 9404 rows of 5120 bf16 72.7 -> 63.2 us (1 row: 61.1, 2 rows: 60.7), 9404 of 4096 fp16
-// 50.1 -> 49.5, 3000 of 4096 fp16 18.7 -> 17.4 (19.5, 18.9), but 2500 of 5120 bf16 20.3 -> 21.3 us.  Plain loads
-// ahead with one row take what the interleaved ones took (71.2 and 18.7 us).
-template <typename E, int ITERS, bool ROUND_FIRST, int ROWS>
+// One workgroup per row; ITERS 16-byte chunks per thread stay in registers between the sum and the write.  Bound by HBM
+// (four passes over the rows) and, for few rows, by the launch.  Plain loads, each chunk's behind the store of the one
+// before: with x written by the kernel before and the residual out of the caches, as a layer has them, three rows per
+// workgroup with all loads ahead and past the caches take no less (9404 rows of 5120 bf16 71.1 us here, 72.9 so; two rows
+// 71.4, one row 71.1; 3000 of 4096 18.7, 18.4), cost launches that fit the cache (the same buffers, 8192 rows of 5120
+// 49.3, 56.8; 6200 37.9, 45.3) and small ones (64 rows of 4096 3.04, 4.65; one row ahead 3.23).  They gain where both
+// inputs are out of the caches or the operands are just too large for them (9404 of 5120 70.9, 62.9; 16,000 of 4096,
+// written before, 107.6, 102.7).
+template <typename E, int ITERS, bool ROUND_FIRST>
 __global__ __launch_bounds__(kFusedThreads) void add_rms_norm_vec(uint16_t* __restrict__ out, uint16_t* residual,
                                                                  const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ w, float eps, int n,
-                                                                 int64_t rows, int64_t x_stride, int64_t r_stride,
+                                                                 int64_t x_stride, int64_t r_stride,
                                                                  int64_t out_stride) {
-  __shared__ float red[ROWS][4];
-  const int64_t row0 = (int64_t)blockIdx.x * ROWS;
+  __shared__ float red[4];
+  const int64_t row = blockIdx.x;
+  const uint16_t* xr = x + row * x_stride;
+  uint16_t* rr = residual + row * r_stride;
+  uint16_t* orow = out + row * out_stride;
   const int chunks = n >> 3;
-  u32x4 v[ROWS][ITERS], b[ROWS][ITERS], wv[ITERS];
+  u32x4 v[ITERS];
+  float ss = 0.f;
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) {
-    const int64_t row = row0 + r < rows ? row0 + r : row0;  // a row past the end: row0's loads again, nothing stored
-    const uint16_t* xr = x + row * x_stride;
-    const uint16_t* rr = residual + row * r_stride;
+  for (int i = 0; i < ITERS; ++i) {
+    const int c = threadIdx.x + i * kFusedThreads;
+    if (c < chunks) {
+      const u32x4 a = ld16(xr + c * 8), b = ld16(rr + c * 8);
 #pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int c = threadIdx.x + i * kFusedThreads;
-      if (c < chunks) {
-        v[r][i] = ROWS > 1 ? ld16_nt(xr + c * 8) : ld16(xr + c * 8);
-        b[r][i] = ROWS > 1 ? ld16_nt(rr + c * 8) : ld16(rr + c * 8);
+      for (int j = 0; j < 4; ++j) {
+        // the sum is stored (rounded) as the new residual, and the norm runs on the stored value
+        const uint32_t s = pack2<E>(Elem<E>::lo(a[j]) + Elem<E>::lo(b[j]), Elem<E>::hi(a[j]) + Elem<E>::hi(b[j]));
+        v[i][j] = s;
+        const float lo = Elem<E>::lo(s), hi = Elem<E>::hi(s);
+        ss += lo * lo + hi * hi;
       }
+      st16(rr + c * 8, v[i]);
     }
   }
-  if (ROWS > 1) {
+  ss = block_sum4(ss, red);
+  const float rstd = rsqrtf(ss / (float)n + eps);
 #pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int c = threadIdx.x + i * kFusedThreads;
-      if (c < chunks) wv[i] = ld16(w + c * 8);
-    }
-  }
+  for (int i = 0; i < ITERS; ++i) {
+    const int c = threadIdx.x + i * kFusedThreads;
+    if (c < chunks) {
+      const u32x4 wv = ld16(w + c * 8);
+      u32x4 o;
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) {
-    const bool live = row0 + r < rows;
-    uint16_t* rr = residual + (row0 + r) * r_stride;
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int c = threadIdx.x + i * kFusedThreads;
-      if (c < chunks) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          // the sum is stored (rounded) as the new residual, and the norm runs on the stored value
-          const uint32_t xw = v[r][i][j], bw = b[r][i][j];
-          const uint32_t s = pack2<E>(Elem<E>::lo(xw) + Elem<E>::lo(bw), Elem<E>::hi(xw) + Elem<E>::hi(bw));
-          v[r][i][j] = s;
-          const float lo = Elem<E>::lo(s), hi = Elem<E>::hi(s);
-          ss += lo * lo + hi * hi;
+      for (int j = 0; j < 4; ++j) {
+        float a = Elem<E>::lo(v[i][j]) * rstd, b = Elem<E>::hi(v[i][j]) * rstd;
+        if (ROUND_FIRST) {
+          a = rnd<E>(a);
+          b = rnd<E>(b);
         }
-        if (live) st16(rr + c * 8, v[r][i]);
+        o[j] = pack2<E>(a * Elem<E>::lo(wv[j]), b * Elem<E>::hi(wv[j]));
       }
-    }
-    ss = group_sum<64>(ss);
-    if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = ss;
-  }
-  __syncthreads();
-  if (ROWS == 1) {
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int c = threadIdx.x + i * kFusedThreads;
-      if (c < chunks) wv[i] = ld16(w + c * 8);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < ROWS; ++r) {
-    if (row0 + r >= rows) break;
-    const float rstd = rsqrtf((red[r][0] + red[r][1] + red[r][2] + red[r][3]) / (float)n + eps);
-    uint16_t* orow = out + (row0 + r) * out_stride;
-#pragma unroll
-    for (int i = 0; i < ITERS; ++i) {
-      const int c = threadIdx.x + i * kFusedThreads;
-      if (c < chunks) {
-        u32x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float lo = Elem<E>::lo(v[r][i][j]) * rstd, hi = Elem<E>::hi(v[r][i][j]) * rstd;
-          if (ROUND_FIRST) {
-            lo = rnd<E>(lo);
-            hi = rnd<E>(hi);
-          }
-          o[j] = pack2<E>(lo * Elem<E>::lo(wv[i][j]), hi * Elem<E>::hi(wv[i][j]));
-        }
-        st16(orow + c * 8, o);
-      }
+      st16(orow + c * 8, o);
     }
   }
 }
@@ -159,26 +123,13 @@ static int launch_add_rms(void* out, void* residual, const void* x, const void* 
   dim3 grid((unsigned)rows), block(kFusedThreads);
   if (vec) {
     const int iters = (int)((n / 8 + kFusedThreads - 1) / kFusedThreads);
-    // Three rows per workgroup from ten workgroups per compute unit on: with three or four each, the units that get one
-    // more than the others are what the launch waits for (2500 rows of 5120: 20.3 us with one row, 21.3 with three).
-    const bool multi = rows >= 8192 && iters <= 4;
-    const dim3 vgrid((unsigned)(multi ? (rows + 2) / 3 : rows));
-#define PH_ARMS(I)                                                                                            \
-  do {                                                                                                        \
-    if (multi)                                                                                                \
-      hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF, 3>), vgrid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, \
-                         xs, rs, os);                                                                         \
-    else                                                                                                      \
-      hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF, 1>), vgrid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, \
-                         xs, rs, os);                                                                         \
-  } while (0)
+#define PH_ARMS(I) \
+  hipLaunchKernelGGL((add_rms_norm_vec<E, I, RF>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, xs, rs, os)
     if (iters <= 1) PH_ARMS(1);
     else if (iters <= 2) PH_ARMS(2);
     else if (iters <= 3) PH_ARMS(3);
     else if (iters <= 4) PH_ARMS(4);
-    else
-      hipLaunchKernelGGL((add_rms_norm_vec<E, 8, RF, 1>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, rows, xs, rs,
-                         os);
+    else PH_ARMS(8);
 #undef PH_ARMS
   } else {
     hipLaunchKernelGGL((add_rms_norm_generic<E, RF>), grid, block, 0, st, o, r, xi, wi, eps, (int)n, xs, rs, os);
