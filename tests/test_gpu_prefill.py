@@ -1,5 +1,7 @@
 """GPU parity of prefill-with-parent-context (packed ragged chunks, bottom-right
 causal over scattered parent slots) against the CPU oracle."""
+import ctypes
+
 import pytest
 import torch
 
@@ -8,6 +10,19 @@ from oracle.ref_ops import ref_cos_sin_cache, ref_prefill_with_parent, ref_rope_
 pytestmark = pytest.mark.gpu
 
 TOL = {torch.float16: dict(atol=2e-3, rtol=1e-2), torch.bfloat16: dict(atol=1e-2, rtol=2e-2)}
+
+
+def prefill_plan(q_lens, ctx_lens, H, D, dtype, workspace_bytes=None):
+    """(queries per workgroup, parts per context) of a call of these sizes; the workspace it asks for by default"""
+    from parrotserve_amd import _lib
+
+    lib, tile, parts = _lib.load(), ctypes.c_int32(), ctypes.c_int32()
+    code = _lib.PH_F16 if dtype == torch.float16 else _lib.PH_BF16
+    if workspace_bytes is None:
+        workspace_bytes = lib.ph_prefill_workspace_bytes(sum(q_lens), H, D, code, max(ctx_lens))
+    assert lib.ph_prefill_plan(sum(q_lens), len(q_lens), H, D, code, max(ctx_lens), sum(ctx_lens), workspace_bytes,
+                               ctypes.byref(tile), ctypes.byref(parts)) == _lib.PH_OK
+    return tile.value, parts.value
 
 
 def run_prefill_case(case, dev, fused_path=True):
@@ -187,16 +202,18 @@ def test_prefill_short_heads_on_the_wide_tile(dev, D, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("q_lens,parent,H,D", [
-    ([61], 1987, 4, 128),      # many parts of one 64-query tile
-    ([1], 1100, 3, 128),       # nine steps: the last of several parts is empty
-    ([16, 5], 900, 5, 128),    # two chunks of different visible lengths
-    ([33], 1500, 2, 96),       # short heads
-    ([40, 7], 800, 4, 64),     # head pairs
-    ([700], 5000, 2, 64),      # head pairs on more than one tile, parts beyond the slot window's length
-    ([300], 6100, 9, 128),     # several tiles, the last one partly filled
+@pytest.mark.parametrize("q_lens,parent,H,D,plan", [
+    ([61], 1987, 4, 128, (64, 16)),      # many parts of one 64-query tile
+    ([1], 1100, 3, 128, (64, 9)),        # nine steps: the last of several parts is empty
+    ([16, 5], 900, 5, 128, (64, 8)),     # two chunks of different visible lengths
+    ([33], 1500, 2, 96, (64, 12)),       # short heads
+    ([40, 7], 800, 4, 64, (64, 7)),      # head pairs
+    ([700], 5000, 2, 64, (256, 9)),      # head pairs on more than one tile, parts beyond the slot window's length
+    ([300], 6100, 9, 128, (64, 3)),      # several tiles, the last one partly filled
+    ([200], 3000, 40, 128, (128, 3)),    # the 128-query tile
+    ([1000], 5000, 8, 128, (256, 8)),    # the 256-query tile on whole heads
 ])
-def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, dtype):
+def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, plan, dtype):
     """Few queries over long contexts: every tile's visible tokens are cut into parts folded afterwards.  A call with
     only the smallest workspace takes the same chunks in one part per tile."""
     from parrotserve_amd import _lib, kernels, synth
@@ -209,6 +226,9 @@ def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, dtype):
     shape = (T, H, D, _lib.PH_F16 if dtype == torch.float16 else _lib.PH_BF16, parent + max(q_lens))
     least = lib.ph_prefill_workspace_min_bytes(*shape)
     assert lib.ph_prefill_workspace_bytes(*shape) > least
+    ctx_lens = [parent + n for n in q_lens]
+    assert prefill_plan(q_lens, ctx_lens, H, D, dtype) == plan
+    assert prefill_plan(q_lens, ctx_lens, H, D, dtype, least)[1] == 1
     kc, vc = synth.pool_to_device(torch.cat([case.k_rows, case.k_new]), torch.cat([case.v_rows, case.v_new]),
                                   case.used_slots, case.pool_slots, dev)
     q = case.q.to(dev)
@@ -226,18 +246,21 @@ def test_prefill_long_contexts_in_parts(dev, q_lens, parent, H, D, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bad", ["key nan", "key inf", "query nan", "query inf", "value nan"])
-@pytest.mark.parametrize("T,parent,D", [
-    (61, 1987, 128),   # parts of one 64-query tile
-    (300, 3000, 128),  # parts of several tiles
-    (33, 1500, 96),    # short heads
-    (33, 500, 128),    # few parts
+@pytest.mark.parametrize("T,parent,H,D,tile", [
+    (61, 1987, 4, 128, 64),    # parts of one 64-query tile
+    (300, 3000, 4, 128, 64),   # parts of several tiles
+    (200, 3000, 40, 128, 128),
+    (1000, 5000, 8, 128, 256),
+    (33, 1500, 4, 96, 64),     # short heads
 ])
-def test_prefill_in_parts_keeps_non_finite_values(dev, T, parent, D, bad, dtype):
+def test_prefill_in_parts_keeps_non_finite_values(dev, T, parent, H, D, tile, bad, dtype):
     """A non-finite key, value or query in a prefill in parts: NaN wherever the same attention in plain fp32 has it,
     the other heads and queries as without it."""
     from parrotserve_amd import kernels
 
-    H, head, n = 4, 1, parent + T
+    head, n = 1, parent + T
+    used, parts = prefill_plan([T], [n], H, D, dtype)
+    assert used == tile and parts > 1
     g = torch.Generator().manual_seed(77 + T)
     q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (T, n, n))
     what, value = bad.split()
@@ -260,8 +283,8 @@ def test_prefill_in_parts_keeps_non_finite_values(dev, T, parent, D, bad, dtype)
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("q_lens,ctx_lens,D", [
-    ([16] * 4, [8192, 64, 64, 64], 128),                      # parts made for one long context: the others fill one
-    ([64, 3, 64, 1], [512, 4100, 64, 1], 128),                # the long one in the middle, a chunk of one token
+    ([16] * 4, [8192, 64, 64, 64], 128),               # eight parts made for one long context: the others fill one
+    ([64, 3, 64, 1], [512, 4100, 64, 1], 128),         # the long one in the middle, a chunk of one token
     ([61] * 6, [100, 200, 400, 800, 1600, 3200], 96),
     ([256, 40], [6256, 40], 64),
 ])
@@ -270,6 +293,7 @@ def test_prefill_contexts_of_different_lengths(dev, q_lens, ctx_lens, D, dtype):
     from parrotserve_amd import kernels
 
     H = 8
+    assert prefill_plan(q_lens, ctx_lens, H, D, dtype)[1] > 1
     g = torch.Generator().manual_seed(5 + sum(ctx_lens))
     n = sum(ctx_lens)
     q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (sum(q_lens), n, n))
