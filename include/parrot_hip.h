@@ -527,8 +527,12 @@ int ph_suffix_plan_build(const int32_t* suffix_lens, int64_t num_reqs, int64_t m
  *   (descending x, equal values by ascending id) is <= top_p[r];
  *   out_ids[r] = the first id whose cumulative surviving mass, in ascending id
  *   order, exceeds uniform[r] * (surviving mass).
- * The filter is found by bisection over the element type's ordered bit
- * patterns instead of a sort.  uniform[r] in [0, 1) comes from the caller's
+ * The filter is found from histograms of the mass over the bit patterns of the
+ * exponentials (long or unaligned rows, rows of few distinct values: by
+ * bisection over the element type's ordered bit patterns) instead of a sort.
+ * The two round the mass differently: where top_p falls within a few 1e-7 of
+ * the mass before a token they may differ by that token, and so may this call
+ * and ph_top_p_probs.  uniform[r] in [0, 1) comes from the caller's
  * random generator, so the draw is reproducible from the inputs; the
  * distribution of the drawn token is that of the reference, the mapping from
  * a seed to a token is not (that one is torch.multinomial's).

@@ -31,6 +31,8 @@ FLAGS = [
 ]
 # The matrix-core kernels never produce NaNs from finite inputs (masked scores are -inf and every
 # difference of two infinities is guarded), so their max trees may drop the NaN-quieting of each input.
+# (A NaN in the inputs still reaches the result, through the exponentials and their sum: tests/test_gpu_prefill.py
+# and tests/test_gpu_decode.py hold it to that.)
 EXTRA_FLAGS = {"prefix_mfma.hip": ["-fno-honor-nans"]}
 
 

@@ -151,7 +151,7 @@ struct PrefillArgs {
   int head_dim;              // 0 / 128, or 80 / 96 / 112: a short head on the 128-wide tile (set by launch_prefill_mfma)
   int n_splits;              // > 1: every tile's visible tokens are cut into this many parts,
   float* opart;              //      [n_splits][num_tokens][H] rows of head_dim (paired: 64) floats
-  float* ml;                 //      and (m, l) each, folded by the merge kernel
+  float* ml;                 //      and (m, l) each, folded by fold_parts_kernel
 };
 
 // The parts of a split prefill and where their fold goes (16-bit elements).

@@ -1154,7 +1154,7 @@ __global__ __launch_bounds__(64) void prefill_tiles_kernel(const int32_t* q_cu, 
 // Prefill with parent context, eight waves: workgroup = (head, tile of 32 * (8 / TQ) queries of one chunk)
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
 // SPLIT: the tile's visible tokens are cut into a.n_splits runs, this workgroup takes run `split` and writes an
-// (O, m, l) part for the merge kernel instead of the output row.
+// (O, m, l) part for fold_parts_kernel instead of the output row.
 template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
 __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const PrefillTile& pt, int split, char* smem) {
   constexpr int QB = 8 / TQ, NDB = 4 / TQ, QT = 32 * QB;

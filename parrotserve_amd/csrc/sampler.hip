@@ -11,14 +11,18 @@
 // The draw is the inverse-CDF draw over ascending token ids from a uniform number the caller passes, so the
 // result is a function of the inputs (the reference draws through torch.multinomial's own random stream).
 //
-// One workgroup of 1024 lanes per row.  Two kernels, same arithmetic:
+// One workgroup of 1024 lanes per row.  Two kernels, the same e values:
 //   sample_rows_kernel   rows on the 16-byte grid of up to 57,344 tokens: the row lives in registers, the cut
-//                        comes from histograms of the mass over the bit patterns of e;
+//                        comes from histograms of the mass over the bit patterns of e (16-bit rows of few
+//                        distinct values, rows with NaN or infinite logits: from the bisection);
 //   sample_top_p_kernel  any other row: e values in LDS up to 36 K tokens, longer rows are re-read and
 //                        re-exponentiated in every pass (they sit in L2; slower); the cut comes from a bisection
 //                        over the patterns of the element type, a compare-and-add over the row per bit.
-// Histogram sums are whole numbers (atomic order does not matter), float sums are taken in a fixed order (per-lane partial sums, a wave tree, then the sixteen wave sums in
-// sequence): the same tokens on every run.
+// Histogram sums are whole numbers (atomic order does not matter), float sums are taken in a fixed order (per-lane
+// partial sums, a wave tree, then the sixteen wave sums in sequence): the same tokens on every run.  The histograms'
+// masses are exact, the bisection's carry the rounding of fp32 sums (a few 1e-7 of the row's mass): where top_p falls
+// that close to the mass before a token, the two can differ by that token, and so can the two kernels (and with them
+// ph_sample_top_p and ph_top_p_probs, which takes the second).
 #include "common.hpp"
 
 namespace ph {

@@ -294,9 +294,9 @@ def sample_top_p(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_
                  uniform: torch.Tensor) -> torch.Tensor:
     """Temperature, top-p filter and one draw per row of ``logits [B, V]`` (fp16, bf16 or fp32) in one launch: the
     body of the reference's ``Sampler.forward`` after the logits GEMM (models/sampler.py:33-64), with the filter
-    found from histograms (long or unaligned rows: by bisection) instead of two sorts and the draw taken from
-    ``uniform [B]`` (float32 in [0, 1), from the caller's generator) by inverse CDF over ascending token ids.  ``temperature`` / ``top_p``: float32 ``[B]`` on the
-    device, or ``None`` for 1.  Returns int64 ``[B]``."""
+    found from histograms (long or unaligned rows, rows of few distinct values: by bisection) instead of two sorts and
+    the draw taken from ``uniform [B]`` (float32 in [0, 1), from the caller's generator) by inverse CDF over ascending
+    token ids.  ``temperature`` / ``top_p``: float32 ``[B]`` on the device, or ``None`` for 1.  Returns int64 ``[B]``."""
     _require_gpu(logits, temperature, top_p, uniform)
     assert logits.dim() == 2 and logits.stride(1) == 1
     B, V = logits.shape

@@ -349,8 +349,8 @@ def test_fused_add_rms_norm(dev, dtype, rows, n):
 @pytest.mark.parametrize("rows", [8191, 8192, 8193, 8194])
 @pytest.mark.parametrize("n", [8, 2056, 8192, 8200])
 def test_fused_add_rms_norm_rows_per_workgroup(dev, dtype, rows, n):
-    """Many rows, row widths of one chunk to more than four per thread, strided inputs: the sum is a rounded add (exact), the norm equals the norm
-    kernel on the stored sum, and the rows behind the last stay as they were."""
+    """Many rows, row widths of one chunk to more than four per thread, strided inputs: the sum is a rounded add (exact),
+    the norm equals the norm kernel on the stored sum, and the rows behind the last stay as they were."""
     from parrotserve_amd import kernels
 
     g = torch.Generator().manual_seed(18)
