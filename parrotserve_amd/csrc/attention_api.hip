@@ -429,8 +429,10 @@ static size_t prefill_parts_room(int64_t T, int64_t H, int64_t D, int64_t max_kv
 // its steps, no faster than the K/V rows come from memory; a split launch adds the parts' write and fold.  The host
 // knows the query total, the chunk count, the longest context and the sum of all contexts (kv_rows): tiles per chunk
 // and visible lengths are averages, and the longest context bounds the launch from below.
-// Constants fitted to 27 shapes in bf16 (1 to 16 chunks of 16 to 4096 tokens over parents of 0 to 6000, 32 and 40
-// heads), every tile with 1 to 16 splits: the choice is within 8 % of the best form on 24 of them, 20 % on one.
+// Constants fitted in bf16 at head size 128 (1 to 16 chunks of 16 to 4096 tokens over parents of 0 to 6000, 32 and 40
+// heads).  Checked against one part per context on the tile of the average chunk length: 384 launches of 64-, 96- and
+// 128-wide heads, 2 to 80 of them, 1 to 300 chunks, equal and very different contexts, take 0.15 to 1.013 of its time,
+// 0.69 in the geometric mean, three of them more than 1.002 (profiles/prefill_plan_sweep.txt).
 static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int64_t kv_rows, int tile_q,
                               int64_t splits, int64_t cus) {
   const double start = tile_q == 256 ? 9.0 : 8.5;
