@@ -336,3 +336,44 @@ def test_more_tile_rows_than_the_grid_holds(dev):
     out = kernels.prefill_attention(q, k, v, tabs)
     torch.cuda.synchronize()
     assert torch.equal(out, v[perm.to(dev)])
+
+
+@pytest.mark.parametrize("warm", ["the call", "a larger call", "a call of one part"])
+def test_prefill_in_parts_replays_from_a_captured_graph(dev, warm):
+    """A prefill that is cut into parts, recorded after an eager run of itself, of a longer call that takes no parts, or
+    of a call whose scratch holds none (the recorded call then stays in one part): every replay, with eager work between
+    them, gives what the eager call with the same workspace gives."""
+    from parrotserve_amd import kernels
+
+    H, D, T, n = 32, 128, 61, 2048
+    g = torch.Generator(device=dev).manual_seed(41)
+    rand = lambda rows: torch.randn(rows, H, D, generator=g, device=dev, dtype=torch.bfloat16)
+    k, v, q = rand(4096), rand(4096), rand(T)
+    build = lambda new, length: kernels.PrefillTables.build([new], [list(range(length))], dev)
+    tables, out = build(T, n), torch.empty_like(q)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        if warm == "the call":
+            kernels.prefill_attention(q, k, v, tables)
+        elif warm == "a larger call":
+            kernels.prefill_attention(rand(4096), k, v, build(4096, 4096))
+        else:
+            kernels.prefill_attention(rand(1), k, v, build(1, 1))
+        room = kernels._workspaces[(dev.index or 0, side.cuda_stream)].numel()
+    torch.cuda.synchronize()
+    parts = prefill_plan([T], [n], H, D, torch.bfloat16, room)[1]
+    assert parts > 1 or warm == "a call of one part"  # (a stream used before may hold more)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        kernels.prefill_attention(q, k, v, tables, out=out)
+    for rep in range(3):
+        q.copy_(rand(T))
+        out.zero_()
+        eager = kernels.prefill_attention(q, k, v, tables)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        if parts > 1:
+            assert torch.equal(out, eager), f"replay {rep} differs from the eager result"
+        torch.testing.assert_close(out.float(), eager.float(), **TOL[torch.bfloat16])
