@@ -551,8 +551,12 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   constexpr int NDBV = HALF ? 2 : 4;
   float16_t oacc[4];
   float m = -INFINITY, lsum = 0.f, mtrue = -INFINITY;
-  const int lane = threadIdx.x & 63;
-  const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = w8 / QB, qb = w8 % QB;
+  // (the thread's number anew for every tile: what follows from it would be kept, and spilled, across the units of a
+  // workgroup that walks several)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63;
+  const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6), g = w8 / QB, qb = w8 % QB;
   const int h = lane >> 5, ql = lane & 31;
   char* gl = smem + g * NST * SBYTES;
   int32_t* win = reinterpret_cast<int32_t*>(smem + kWinOff);
@@ -562,12 +566,37 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
 
-  // slot window [win0, win0 + kWin) of the list, clamped to the list's end
+  // slot window [win0, win0 + kWin) of the list, clamped to the list's end; filled as far as the steps left reach
   int win0 = s0;
-  auto fill_window = [&]() {
-    for (int i = threadIdx.x; i < kWin; i += 512) win[i] = wk.slots[min(win0 + i, wk.slots_len - 1)];
-  };
-  fill_window();
+  const int steps_end = s0 + (s1 - s0 + STEP * TQ - 1) / (STEP * TQ) * (STEP * TQ);
+#pragma unroll
+  for (int k = 0; k < kWin / 512; ++k)
+    if (512 * k < steps_end - s0)
+      lds_dma4(wk.slots + min(s0 + 512 * k + tid, wk.slots_len - 1),
+               lds_addr_of(smem) + kWinOff + (512 * k + 64 * w8) * 4);
+
+  // The query rows are requested right behind the slot ids, as whole rows (four per load, 16 lanes a row) that land in
+  // the upper half of the group's ring: every wave brings the 32 rows it multiplies, in the K tiles' layout, and takes
+  // its operands from there.  (Loaded as operands, 16 bytes of a row per lane, they are 64 cache lines a load, and
+  // behind the ring they arrive after all of it.)
+  const uint32_t q_lds = lds_addr_of(gl) + (NST / 2) * SBYTES + qb * 8192;
+  static_assert((NST - NST / 2) * SBYTES >= QB * 8192, "the query rows fit the upper half of the ring");
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4), q = 32 * qb + r, qc = q < wk.nq ? q : 0;
+    int cg = (lane & 15) ^ (r & 15);  // the 16-byte chunk of the row at this place
+    const uint16_t* qp = wk.qrow0;
+    if (wk.pair_half >= 0) {
+      // a 64-wide head as one half of a head pair: the row pointer points at this half's 64 values; 2: rows alternate
+      // between the two heads of the pair, row q = request q >> 1, half q & 1
+      cg &= 7;
+      qp += wk.pair_half == 2 ? (int64_t)(qc >> 1) * wk.q_stride + 64 * (qc & 1) : (int64_t)qc * wk.q_stride;
+    } else {
+      cg = cg * 8 < wk.head_dim ? cg : 0;  // past a short row its first chunk
+      qp += (int64_t)(qc >> wk.gshift) * wk.q_stride + (qc & ((1 << wk.gshift) - 1)) * kPD;
+    }
+    lds_dma16<false>(qp + cg * 8, q_lds + i * 1024);
+  }
 
   // staging: row group L (0..7 K, 8..15 V) covers tokens 4 (L & 7) .. +3, 16 lanes per token row; this wave
   // brings row groups qb LPT .. + LPT - 1 (same swizzles as the four-wave form)
@@ -600,11 +629,13 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   const int ntile = (s1 - s0 + STEP - 1) / STEP;
   const int iters = (ntile + TQ - 1) / TQ;                 // same for all eight waves
   const int my_iters = ntile > g ? (ntile - g + TQ - 1) / TQ : 0;  // tiles of this token group
+  wait_vmcnt<8>();                                         // this wave's part of the window; its query rows are behind
   __syncthreads();                                         // window visible
   PH_TL(1);
-  // the whole ring is filled up front: tiles 0 .. A (the main loop issues tile it + A at step it >= 1)
+  // the whole ring is filled up front: tiles 0 .. A (the main loop issues tile it + A at step it >= 1), its upper half
+  // once every wave has taken its queries
 #pragma unroll
-  for (int j = 0; j < NST; ++j)
+  for (int j = 0; j < NST / 2; ++j)
     if (j < my_iters) fetch_rows(s0 + STEP * (g + TQ * j), j);
 
   // Q as the B operand: column = query 32 qb + ql, contraction chunk (h, s) = dims 64h + 8s .. +8
@@ -612,24 +643,22 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   {
     const int q = 32 * qb + ql;
     const bool ok = q < wk.nq;
-    const uint16_t* qp = wk.qrow0 + (int64_t)(ok ? q : 0) * wk.q_stride + 64 * h;
     // a 64-wide head as one half of a head pair: the other half of the query is zero, which cancels the
-    // neighbouring head's keys in the score (the row pointer already points at this half's 64 values)
-    int half = wk.pair_half;
-    if (wk.pair_half == 2) {  // rows alternate between the two heads of the pair: row q = request q >> 1, half q & 1
-      half = q & 1;
-      qp = wk.qrow0 + (int64_t)(ok ? q >> 1 : 0) * wk.q_stride + 64 * half;
-    } else if (wk.pair_half >= 0) {
-      qp = wk.qrow0 + (int64_t)(ok ? q : 0) * wk.q_stride;
-    }
-    if (wk.gshift > 0)
-      qp = wk.qrow0 + (int64_t)(ok ? q >> wk.gshift : 0) * wk.q_stride + (q & ((1 << wk.gshift) - 1)) * kPD + 64 * h;
+    // neighbouring head's keys in the score
+    const int half = wk.pair_half == 2 ? q & 1 : wk.pair_half;
     const bool mine = wk.pair_half < 0 || h == half;
-    const bool padded = wk.head_dim < kPD;  // (never together with head pairs or grouped rows)
+    u32x4 raw[8];
+    if (my_iters >= NST / 2) wait_vmcnt<NST / 2 * LPT>(); else wait_vmcnt<0>();  // the query rows, not the ring behind
+#pragma unroll
+    for (int s = 0; s < 8; ++s) raw[s] = lds_ld16_a(q_lds + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16));
+    __syncthreads();
+#pragma unroll
+    for (int j = NST / 2; j < NST; ++j)
+      if (j < my_iters) fetch_rows(s0 + STEP * (g + TQ * j), j);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      const bool in = !padded || 64 * h + 8 * s < wk.head_dim;  // dims beyond a short head: read its first dims, use zero
-      u32x4 v = ld16(in ? qp + 8 * s : qp - 64 * h);
+      const bool in = 64 * h + 8 * s < wk.head_dim;  // dims beyond a short head are zero
+      u32x4 v = raw[s];
       if (!ok || !mine || !in) v = u32x4{0, 0, 0, 0};
       if (PRESC) {
         // PRESC: q takes the factor scale * log2(e) here and is rounded to the element type again (what the
@@ -651,10 +680,13 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   mid();
   PH_TL(3);
 
-  // Operand read addresses of ring stage 0 (and of stage 4, beyond the reach of the 16-bit immediate).
+  // Operand read addresses in the ring's current half (stages beyond the 16-bit immediate's 64 KB: the addresses move
+  // there and back, which leaves the registers of a second set to the row loads' addresses; those were spilled, and
+  // every reload from scratch waited for the rows in flight).
   // K: row ql, chunk (8h + s) swizzled by the row; V: the transposing read's row/column of this lane.
-  constexpr int NHI = NST * SBYTES > 65536 ? 2 : 1;
-  uint32_t kaddr[NHI][8], vaddr[NHI][4];
+  constexpr bool TWO_HALVES = NST * SBYTES > 65536;
+  static_assert(NST * SBYTES <= 2 * 65536, "two halves of the immediate's reach");
+  uint32_t kaddr[8], vaddr[4];
   {
     const uint32_t gl_a = lds_addr_of(gl);
     const int sl = lane & 15, rh = (lane >> 4) & 1;
@@ -662,20 +694,23 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     const int tcol = 2 * rh + ((sl & 3) >> 1);                // + 4db, in 16-byte chunks
     const int tswz = 4 * (sl >> 2);                           // = 4 * (row & 3)
 #pragma unroll
-    for (int hi = 0; hi < NHI; ++hi) {
+    for (int s = 0; s < 8; ++s) {
+      kaddr[s] = gl_a + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16);
+      asm("" : "+v"(kaddr[s]));  // keep the sum in one register (otherwise it is re-added at every read)
+    }
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        kaddr[hi][s] = gl_a + hi * 65536 + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16);
-        asm("" : "+v"(kaddr[hi][s]));  // keep the sum in one register (otherwise it is re-added at every read)
-      }
-#pragma unroll
-      for (int db = 0; db < NDBV; ++db) {
-        const int dbr = HALF ? 2 * wk.pair_half + db : db;  // 32-dim block of the 128-wide row
-        vaddr[hi][db] = gl_a + hi * 65536 + kVtOff + trow * 256 + (sl & 1) * 8 + (((4 * dbr + tcol) ^ tswz) * 16);
-        asm("" : "+v"(vaddr[hi][db]));
-      }
+    for (int db = 0; db < NDBV; ++db) {
+      const int dbr = HALF ? 2 * wk.pair_half + db : db;  // 32-dim block of the 128-wide row
+      vaddr[db] = gl_a + kVtOff + trow * 256 + (sl & 1) * 8 + (((4 * dbr + tcol) ^ tswz) * 16);
+      asm("" : "+v"(vaddr[db]));
     }
   }
+  auto move_half = [&](uint32_t by) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) asm volatile("v_add_u32 %0, %1, %0" : "+v"(kaddr[s]) : "s"(by));
+#pragma unroll
+    for (int db = 0; db < NDBV; ++db) asm volatile("v_add_u32 %0, %1, %0" : "+v"(vaddr[db]) : "s"(by));
+  };
   // the ring position is a compile-time constant in the unrolled inner loop, so every LDS address of a
   // step is a fixed register plus an immediate offset
   for (int it0 = 0; it0 < iters; it0 += NST) {
@@ -683,11 +718,15 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
    for (int stage = 0; stage < NST; ++stage) {
     const int it = it0 + stage;
     if (it >= iters) break;
+    if (TWO_HALVES && stage == NST / 2) move_half(65536u);
+    if (TWO_HALVES && stage == 0 && it > 0) move_half(-65536u);
     const int tb = s0 + STEP * (g + TQ * it);
     // Tile `it` of this group has landed once at most the (A - 1) LPT loads issued after it are outstanding
     // (near the end fewer were issued, so everything is awaited); the barrier publishes all parts of the
     // tile and tells everyone that the stage read in the previous step is free again.
-    if (it + A - 1 >= my_iters) {
+    if (it == 0 && my_iters > A) {
+      wait_vmcnt<A * LPT>();  // the whole ring is in flight
+    } else if (it + A - 1 >= my_iters) {
       wait_vmcnt<0>();
     } else if (PREFETCH && pf_steps > 0 && it >= 1 && it <= pf_steps) {
       wait_vmcnt<(A - 1) * LPT + 1>();  // the line touches issued behind the last row loads may still be out
@@ -700,16 +739,18 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
       const int front = s0 + STEP * TQ * (it + A);           // first token of the step being staged
       if (front < s1 && front >= win0 + kWin) {              // workgroup-uniform: slide the slot window
         win0 += kWin;
-        fill_window();
+        const int n = min(kWin, steps_end - win0);
+#pragma unroll 2
+        for (int i = tid; i < n; i += 512) win[i] = wk.slots[min(win0 + i, wk.slots_len - 1)];
         __syncthreads();
       }
       if (it > 0 && it + A < my_iters) fetch_rows(front + STEP * g, (stage + A) % NST);
       if (PREFETCH && it < pf_steps) {
         // token (of all four groups) and line of the step after `front`, clamped into the list and the window
-        const int pt = min(min(front + STEP * TQ + (int)(threadIdx.x >> 2), s1 - 1), win0 + kWin - 1);
+        const int pt = min(min(front + STEP * TQ + (int)(tid >> 2), s1 - 1), win0 + kWin - 1);
         const uint32_t slot = (uint32_t)win[pt - win0];
-        const char* base = reinterpret_cast<const char*>((threadIdx.x & 2) ? vc : kc) +
-                           (int64_t)head * (wk.head_dim * 2) + (threadIdx.x & 1) * 128;
+        const char* base = reinterpret_cast<const char*>((tid & 2) ? vc : kc) +
+                           (int64_t)head * (wk.head_dim * 2) + (tid & 1) * 128;
         lds_dma4(base + (uint64_t)slot * row_bytes, pf_lds);
       }
     }
@@ -717,11 +758,10 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     float16_t sacc[SUB];
 #pragma unroll
     for (int sb = 0; sb < SUB; ++sb) {
-      const int off = stage * SBYTES + sb * kStage;
-      const int shi = off >> 16, slo = off & 65535;
+      const int slo = (stage * SBYTES + sb * kStage) & 65535;
       u32x4 ka[8];
 #pragma unroll
-      for (int s = 0; s < 8; ++s) ka[s] = lds_ld16_a(kaddr[shi][s] + slo);
+      for (int s = 0; s < 8; ++s) ka[s] = lds_ld16_a(kaddr[s] + slo);
       if (SUB == 1) __builtin_amdgcn_sched_barrier(0);
       const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       sacc[sb] = Mfma32<E>::run(ka[0], qop[0], PRESC ? cinit : zero);
@@ -733,14 +773,13 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     u32x4 va[SUB][4][2];
 #pragma unroll
     for (int sb = 0; sb < SUB; ++sb) {
-      const int off = stage * SBYTES + sb * kStage;
-      const int shi = off >> 16, slo = off & 65535;
+      const int slo = (stage * SBYTES + sb * kStage) & 65535;
 #pragma unroll
       for (int db = 0; db < NDBV; ++db)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const u32x2 lo = lds_tr16_a(vaddr[shi][db] + slo + (16 * u) * 256);
-          const u32x2 hi = lds_tr16_a(vaddr[shi][db] + slo + (16 * u + 8) * 256);
+          const u32x2 lo = lds_tr16_a(vaddr[db] + slo + (16 * u) * 256);
+          const u32x2 hi = lds_tr16_a(vaddr[db] + slo + (16 * u + 8) * 256);
           va[sb][db][u] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
     }
@@ -918,10 +957,11 @@ __device__ __forceinline__ void prefix_unit8(const PrefixArgs& a, int split, int
   const int g = z / mtiles, mt = z - g * mtiles;
   int r0 = 0, r1 = a.B, poff = 0, plen = a.fixed_prefix_len;
   if (a.prefix_cu) {
-    r0 = a.group_req_cu[g] << a.req_shift;
-    r1 = a.group_req_cu[g + 1] << a.req_shift;
-    poff = a.prefix_cu[g];
-    plen = a.prefix_cu[g + 1] - poff;
+    // (a workgroup that walks several units reads these behind its own stores: as vector loads, unless told)
+    r0 = __builtin_amdgcn_readfirstlane(a.group_req_cu[g]) << a.req_shift;
+    r1 = __builtin_amdgcn_readfirstlane(a.group_req_cu[g + 1]) << a.req_shift;
+    poff = __builtin_amdgcn_readfirstlane(a.prefix_cu[g]);
+    plen = __builtin_amdgcn_readfirstlane(a.prefix_cu[g + 1]) - poff;
   }
   const int qbase = r0 + mt * QT;
   const int nq = min(QT, r1 - qbase);
@@ -1016,7 +1056,8 @@ struct WideTile {
 // DS = head size of the suffix phase: 128, or 64 when the prefix phase runs on head pairs (pa.req_shift == 1).
 // NQ > 1 (grouped KV heads, ia.nq): the suffix waves divide runs of NQ query heads that share a KV head and stream a
 // row for the run at once.
-template <typename E, int TQ, int DS = kPD, int NQ = 1>
+// ROLES: the form (np > 0), a kernel each: with both in one, the tile loops shared its registers and spilled.
+template <typename E, int TQ, int DS, int NQ, bool ROLES>
 __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mtiles, int n_units, int np,
                                                            ItemArgs ia) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1026,7 +1067,7 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
   constexpr int HPW = HeadLanes<DS>::HPW;
   const int hgroups = (ia.H / NQ + HPW - 1) / HPW;
   const int slots = ia.num_lanes * hgroups;
-  if (np > 0) {
+  if constexpr (ROLES) {
     if ((int)blockIdx.x < np) {
       for (int u = blockIdx.x; u < n_units; u += np) {
         if (u != (int)blockIdx.x) __syncthreads();  // the fold scratch of the last unit is the staging ring of the next
@@ -1042,9 +1083,7 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
         run_piece<E, DS, 4, 2, NQ>(ia, piece, s - piece * hgroups);
       }
     }
-    PH_TL(11);
-    return;
-  }
+  } else {
   const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 8 + (threadIdx.x >> 6));
   // this wave's first suffix piece: its record is requested before anything else
   const int piece0 = wave < slots ? wave / hgroups : -1;
@@ -1074,6 +1113,7 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
     }
   } else {
     suffix();
+  }
   }
   PH_TL(11);
 }
@@ -1339,10 +1379,12 @@ static int launch_fused_tq(const PrefixArgs& a, const ItemArgs& ia, int num_grou
     if (grid < unit_grid) grid = unit_grid;
   }
   if (grid <= 0) return PH_OK;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_fused_kernel<E, TQ, DS, NQ>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kTile8Lds);
-  PH_LAUNCH_TIMED((decode_fused_kernel<E, TQ, DS, NQ>), dim3(grid), dim3(512), kTile8Lds, st, ev, a, mtiles,
-                        n_units, np, ia);
+  auto launch = [&](auto kernel) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kTile8Lds);
+    PH_LAUNCH_TIMED(kernel, dim3(grid), dim3(512), kTile8Lds, st, ev, a, mtiles, n_units, np, ia);
+  };
+  if (np > 0) launch(&decode_fused_kernel<E, TQ, DS, NQ, true>);
+  else launch(&decode_fused_kernel<E, TQ, DS, NQ, false>);
   return launch_status();
 }
 

@@ -42,6 +42,21 @@ def test_shared_prefix_decode(dev, dtype, B, P, H):
     _check(case, dev)
 
 
+@pytest.mark.parametrize("sizes,P,s_hi,dtype", [((256, 131), 2100, 40, torch.float16), ((256,), 700, 3, torch.bfloat16),
+                                                ((97, 128, 65), 2050, 100, torch.bfloat16),
+                                                ((64, 33, 1), 4224, 90, torch.float16)])
+def test_units_back_to_back_on_each_tile(dev, sizes, P, s_hi, dtype):
+    """A workgroup that walks several prefix units stages every unit's slots and query rows over the last one's ring: the
+    64-, 128- and 256-query tiles with groups that fill their last 32-row block and groups that do not, short suffixes
+    (every workgroup runs both phases) and long ones."""
+    from parrotserve_amd import synth
+
+    g = torch.Generator().manual_seed(P)
+    s = torch.randint(1, s_hi + 1, (sum(sizes),), generator=g).tolist()
+    case = synth.make_decode_case("units", P, dtype, len(sizes), 0, P, s, 40, 128, 1 << 16, group_sizes=sizes)
+    _check(case, dev)
+
+
 def test_config1_shape_in_fp16(dev):
     """Config 1's shape (B 8, P 512, S U[32,128], 32x128, seed 0) cast to fp16 for the GPU."""
     from parrotserve_amd import synth

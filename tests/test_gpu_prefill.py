@@ -145,6 +145,35 @@ def test_prefill_long_parents_all_tile_sizes(dev, q_lens, parent):
     torch.testing.assert_close(out.float(), ref.float(), **TOL[torch.float16])
 
 
+@pytest.mark.parametrize("n,tile", [(61, 64), (125, 128), (255, 256)])
+@pytest.mark.parametrize("ctx", [512, 513, 4032, 4095, 4097])
+def test_prefill_window_filled_in_part(dev, n, tile, ctx):
+    """The slot window is filled 512 entries at a time as far as the tile's steps reach (64 or 128 tokens a step): contexts
+    that end on, before and behind an edge of either, and at the window's own end, with query rows missing from the last
+    block (its rows are staged as whole 32-row blocks).  More than four rounds of workgroups, so that none is
+    cut into parts."""
+    from parrotserve_amd import synth
+
+    q_lens, H = [n] * 32, 40
+    assert prefill_plan(q_lens, [ctx] * 32, H, 128, torch.float16) == (tile, 1)
+    case = synth.make_prefill_case("win", ctx + n, torch.float16, q_lens[:2], ctx - n, 2, 128, 1 << 14)
+    k_all, v_all = torch.cat([case.k_rows, case.k_new]), torch.cat([case.v_rows, case.v_new])
+    lists = [torch.cat([p, m]) for p, m in zip(case.parent_lists, case.new_lists)]
+    from parrotserve_amd import kernels
+
+    kc, vc = synth.pool_to_device(k_all, v_all, case.used_slots, case.pool_slots, dev)
+    # the two chunks sixteen times each, their two heads twenty times
+    tables = kernels.PrefillTables.build(q_lens, [case.used_slots[lists[i % 2]].tolist() for i in range(32)], dev)
+    q = case.q.view(2, n, 2, 128).repeat(16, 1, 20, 1).view(32 * n, H, 128)
+    wide = lambda t: t.repeat(1, 20, 1).contiguous()  # noqa: E731
+    out = kernels.prefill_attention(q.to(dev), wide(kc), wide(vc), tables)
+    torch.cuda.synchronize()
+    ref = ref_prefill_with_parent(case.q, k_all, v_all, q_lens[:2], lists)
+    got = out.cpu().view(16, 2 * n, 20, 2, 128)
+    assert (got == got[:1, :, :1]).all()
+    torch.testing.assert_close(got[0, :, 0].float(), ref.float(), **TOL[torch.float16])
+
+
 def test_prefill_heads_not_multiple_of_eight_and_tail_tiles(dev):
     """Head counts that leave part of the padded head axis empty, chunks that end inside every tile size."""
     from parrotserve_amd import synth
