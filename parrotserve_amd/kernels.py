@@ -15,6 +15,7 @@ from __future__ import annotations
 import collections
 import ctypes
 import dataclasses
+import functools
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -81,14 +82,24 @@ def _require_gpu(*ts: torch.Tensor) -> torch.device:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream() -> int:
-    """Handle of torch's current stream on the current device (the raw getter costs a fraction of a
-    microsecond; building a torch.cuda.Stream object per launch costs several)."""
+    """Handle of torch's current stream on the current device (the raw getters cost a fraction of a
+    microsecond; building a torch.cuda.Stream object per launch costs several).  Callers hold GPU tensors: the
+    device is initialised."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_raw_device())
     return torch.cuda.current_stream().cuda_stream
+
+
+def _empty_rows(t: torch.Tensor) -> torch.Tensor:
+    """A new contiguous tensor of the shape, type and device of ``t`` (two thirds of ``torch.empty``'s host time where
+    ``t`` is contiguous, and with it the layout that ``empty_like`` keeps)."""
+    if t.is_contiguous():
+        return torch.empty_like(t)
+    return torch.empty(t.shape, dtype=t.dtype, device=t.device)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -237,14 +248,18 @@ def _rms(x, weight, eps, round_first, name):
     _require_gpu(x, weight)
     assert x.shape[-1] == weight.shape[0], "weight size mismatch"
     assert x.dtype == weight.dtype, "weight dtype mismatch"
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if x2.stride(1) != 1:
         x2 = x2.contiguous()
-    out = torch.empty((x2.shape[0], x2.shape[1]), dtype=x.dtype, device=x.device)
-    rc = _lib.load().ph_rms_norm(_ptr(out), _ptr(x2), _ptr(weight.contiguous()), float(eps), x2.shape[0], x2.shape[1],
-                                 x2.stride(0), out.stride(0), _dtype_code(x), int(round_first), _stream())
-    check(rc, name)
-    return out.view(x.shape)
+    if not weight.is_contiguous():
+        weight = weight.contiguous()
+    out = _empty_rows(x2)
+    rows, n = x2.shape
+    rc = _lib.load().ph_rms_norm(out.data_ptr(), x2.data_ptr(), weight.data_ptr(), float(eps), rows, n, x2.stride(0),
+                                 out.stride(0), _dtype_code(x), round_first, _stream())
+    if rc:
+        check(rc, name)
+    return out if x.dim() == 2 else out.view(x.shape)
 
 
 def vllm_rms_norm(input, weight, eps):
@@ -265,13 +280,16 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Te
     _require_gpu(x, residual, weight)
     n = x.shape[-1]
     assert x.shape == residual.shape and weight.shape == (n,) and x.dtype == residual.dtype == weight.dtype
-    x2, r2 = x.reshape(-1, n), residual.view(-1, n)
+    flat = x.dim() == 2
+    x2, r2 = (x, residual) if flat else (x.reshape(-1, n), residual.view(-1, n))
     assert x2.stride(1) == 1 and r2.stride(1) == 1
-    out = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
-    check(_lib.load().ph_add_rms_norm(_ptr(out), _ptr(r2), _ptr(x2), _ptr(weight), float(eps), x2.shape[0], n,
-                                      x2.stride(0), r2.stride(0), out.stride(0), _dtype_code(x),
-                                      1 if round_before_weight else 0, _stream()), "fused_add_rms_norm")
-    return out.view(x.shape)
+    out = _empty_rows(x2)
+    rc = _lib.load().ph_add_rms_norm(out.data_ptr(), r2.data_ptr(), x2.data_ptr(), weight.data_ptr(), float(eps), x2.shape[0],
+                                     n, x2.stride(0), r2.stride(0), out.stride(0), _dtype_code(x),
+                                     1 if round_before_weight else 0, _stream())
+    if rc:
+        check(rc, "fused_add_rms_norm")
+    return out if flat else out.view(x.shape)
 
 
 def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -279,15 +297,19 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] =
     _require_gpu(gate, up)
     d = gate.shape[-1]
     assert gate.shape == up.shape and gate.dtype == up.dtype
-    g2 = gate if gate.dim() == 2 else gate.reshape(-1, d)
-    u2 = up if up.dim() == 2 else up.reshape(-1, d)
+    flat = gate.dim() == 2
+    g2, u2 = (gate, up) if flat else (gate.reshape(-1, d), up.reshape(-1, d))
     assert g2.stride(1) == 1 and u2.stride(1) == 1
     if out is None:
-        out = torch.empty(g2.shape, dtype=gate.dtype, device=gate.device)
-    o2 = out.view(-1, d)
-    check(_lib.load().ph_silu_mul(_ptr(o2), _ptr(g2), _ptr(u2), g2.shape[0], d, g2.stride(0), u2.stride(0),
-                                  o2.stride(0), _dtype_code(gate), _stream()), "silu_mul")
-    return out.view(gate.shape)
+        out = o2 = _empty_rows(g2)
+    else:
+        flat = False
+        o2 = out.view(-1, d)
+    rc = _lib.load().ph_silu_mul(o2.data_ptr(), g2.data_ptr(), u2.data_ptr(), g2.shape[0], d, g2.stride(0), u2.stride(0),
+                                 o2.stride(0), _dtype_code(gate), _stream())
+    if rc:
+        check(rc, "silu_mul")
+    return out if flat else out.view(gate.shape)
 
 
 def sample_top_p(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_p: Optional[torch.Tensor],
@@ -356,12 +378,13 @@ def rope_and_cache(positions, query, key, value, cos_sin_cache, head_size, key_c
     assert key_cache.stride() == value_cache.stride() and key_cache.stride(2) == 1 and key_cache.stride(1) == head_size
     assert query.dtype == key.dtype == value.dtype == key_cache.dtype == cos_sin_cache.dtype
     assert slot_mapping.numel() == T and cos_sin_cache.is_contiguous()
-    check(_lib.load().ph_rope_append(_ptr(positions), _ptr(q2), _ptr(k2), _ptr(v2), _ptr(cos_sin_cache),
-                                     _ptr(key_cache), _ptr(value_cache), _ptr(slot_mapping), _index_code(slot_mapping),
-                                     T, hq, hk, head_size, cos_sin_cache.shape[-1], q2.stride(0), k2.stride(0),
-                                     v2.stride(0), key_cache.stride(0), _dtype_code(query), 1 if key_in_place else 0,
-                                     _stream()),
-          "rope_and_cache")
+    rc = _lib.load().ph_rope_append(positions.data_ptr(), q2.data_ptr(), k2.data_ptr(), v2.data_ptr(),
+                                    cos_sin_cache.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
+                                    slot_mapping.data_ptr(), _index_code(slot_mapping), T, hq, hk, head_size,
+                                    cos_sin_cache.shape[-1], q2.stride(0), k2.stride(0), v2.stride(0),
+                                    key_cache.stride(0), _dtype_code(query), 1 if key_in_place else 0, _stream())
+    if rc:
+        check(rc, "rope_and_cache")
 
 
 def vllm_rotary_emb(positions, query, key, cos_sin_cache, head_size):
@@ -656,6 +679,12 @@ def plan_suffix_items(lens: Sequence[int], num_lanes: int):
     return items, lane_cu, req_cu
 
 
+@functools.lru_cache(maxsize=1024)
+def _decode_workspace_bytes(device: int, *shape: int) -> int:
+    """``ph_decode_workspace_bytes``: a function of its numbers and the current device (3 us a call, a lookup 0.4)."""
+    return _lib.load().ph_decode_workspace_bytes(*shape)
+
+
 def decode_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, tables: DecodeTables,
                      scale: Optional[float] = None, out: Optional[torch.Tensor] = None,
                      events6=None, head_mapping: Optional[torch.Tensor] = None, kv_group: int = 0) -> torch.Tensor:
@@ -676,34 +705,37 @@ def decode_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: 
         assert key_cache.shape[2] == D and head_mapping.dtype == torch.int32 and head_mapping.numel() == H
         assert head_mapping.is_contiguous() and head_mapping.device == query.device
     assert query.dtype == key_cache.dtype == value_cache.dtype
-    assert query.stride(2) == 1 and query.stride(1) == D
-    assert key_cache.stride(2) == 1 and key_cache.stride(1) == D and key_cache.stride() == value_cache.stride()
+    qs, ks = query.stride(), key_cache.stride()
+    assert qs[2] == 1 and qs[1] == D
+    assert ks[2] == 1 and ks[1] == D and ks == value_cache.stride()
     if out is None:
-        out = torch.empty((B, H, D), dtype=query.dtype, device=query.device)
+        out = _empty_rows(query)
     if B == 0:
         return out
     scale = D ** -0.5 if scale is None else scale
     lib = _lib.load()
     plan = tables.plan
-    nbytes = lib.ph_decode_workspace_bytes(B, H, D, tables.num_groups, tables.max_prefix_len, tables.max_suffix_len,
-                                           tables.chunk_tokens, 0 if plan is None else plan.num_items)
+    max_prefix, max_suffix, chunk = tables.max_prefix_len, tables.max_suffix_len, tables.chunk_tokens
+    nbytes = _decode_workspace_bytes(_raw_device(), B, H, D, tables.num_groups, max_prefix, max_suffix, chunk,
+                                     0 if plan is None else plan.num_items)
     ws = _workspace(nbytes, query.device)
     args = (
-        _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), B, H, D, _dtype_code(query),
-        query.stride(0), out.stride(0), key_cache.stride(0), float(scale),
+        out.data_ptr(), query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), B, H, D, _dtype_code(query),
+        qs[0], out.stride(0), ks[0], float(scale),
         tables.num_groups, _ptr(tables.prefix_slots), _ptr(tables.prefix_cu), _ptr(tables.group_req_cu),
-        _ptr(tables.group_req_cu_host), tables.max_prefix_len,
+        _ptr(tables.group_req_cu_host), max_prefix,
         _ptr(tables.suffix_slots), _ptr(tables.suffix_offsets), tables.suffix_table_stride,
         tables.suffix_slots_count(), _ptr(tables.suffix_lens),
-        tables.max_suffix_len, tables.chunk_tokens, None if plan is None else ctypes.byref(plan),
-        _ptr(ws), ws.numel(), _stream())
+        max_suffix, chunk, None if plan is None else ctypes.byref(plan),
+        ws.data_ptr(), ws.numel(), _stream())
     if head_mapping is not None:
         rc = lib.ph_decode_attention_gqa(*args[:6], key_cache.shape[1], _ptr(head_mapping), int(kv_group), *args[6:])
     elif events6 is None:
         rc = lib.ph_decode_attention(*args)
     else:
         rc = lib.ph_decode_attention_timed(*args, events6)
-    check(rc, "decode_attention")
+    if rc:
+        check(rc, "decode_attention")
     return out
 
 
