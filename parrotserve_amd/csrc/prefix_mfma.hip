@@ -680,13 +680,16 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   mid();
   PH_TL(3);
 
-  // Operand read addresses in the ring's current half (stages beyond the 16-bit immediate's 64 KB: the addresses move
-  // there and back, which leaves the registers of a second set to the row loads' addresses; those were spilled, and
-  // every reload from scratch waited for the rows in flight).
+  // Operand read addresses (a ring of 128 KB is two times the 16-bit immediate's reach).  Prefill holds a set for each
+  // half.  Decode, whose kernels have no registers left for a second set (the row loads' addresses were spilled, and
+  // every reload from scratch waited for the rows in flight), moves one set there and back; in prefill that costs
+  // more than it gives (an 8192-token Fill: 1 % slower than the start of the comparison, with two sets 0.7 % faster).
   // K: row ql, chunk (8h + s) swizzled by the row; V: the transposing read's row/column of this lane.
   constexpr bool TWO_HALVES = NST * SBYTES > 65536;
   static_assert(NST * SBYTES <= 2 * 65536, "two halves of the immediate's reach");
-  uint32_t kaddr[8], vaddr[4];
+  constexpr bool MOVES = TWO_HALVES && !CAUSAL;
+  constexpr int NHI = TWO_HALVES && CAUSAL ? 2 : 1;
+  uint32_t kaddr[NHI][8], vaddr[NHI][4];
   {
     const uint32_t gl_a = lds_addr_of(gl);
     const int sl = lane & 15, rh = (lane >> 4) & 1;
@@ -694,22 +697,25 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     const int tcol = 2 * rh + ((sl & 3) >> 1);                // + 4db, in 16-byte chunks
     const int tswz = 4 * (sl >> 2);                           // = 4 * (row & 3)
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      kaddr[s] = gl_a + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16);
-      asm("" : "+v"(kaddr[s]));  // keep the sum in one register (otherwise it is re-added at every read)
-    }
+    for (int hi = 0; hi < NHI; ++hi) {
 #pragma unroll
-    for (int db = 0; db < NDBV; ++db) {
-      const int dbr = HALF ? 2 * wk.pair_half + db : db;  // 32-dim block of the 128-wide row
-      vaddr[db] = gl_a + kVtOff + trow * 256 + (sl & 1) * 8 + (((4 * dbr + tcol) ^ tswz) * 16);
-      asm("" : "+v"(vaddr[db]));
+      for (int s = 0; s < 8; ++s) {
+        kaddr[hi][s] = gl_a + hi * 65536 + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16);
+        asm("" : "+v"(kaddr[hi][s]));  // keep the sum in one register (otherwise it is re-added at every read)
+      }
+#pragma unroll
+      for (int db = 0; db < NDBV; ++db) {
+        const int dbr = HALF ? 2 * wk.pair_half + db : db;  // 32-dim block of the 128-wide row
+        vaddr[hi][db] = gl_a + hi * 65536 + kVtOff + trow * 256 + (sl & 1) * 8 + (((4 * dbr + tcol) ^ tswz) * 16);
+        asm("" : "+v"(vaddr[hi][db]));
+      }
     }
   }
   auto move_half = [&](uint32_t by) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) asm volatile("v_add_u32 %0, %1, %0" : "+v"(kaddr[s]) : "s"(by));
+    for (int s = 0; s < 8; ++s) asm volatile("v_add_u32 %0, %1, %0" : "+v"(kaddr[0][s]) : "s"(by));
 #pragma unroll
-    for (int db = 0; db < NDBV; ++db) asm volatile("v_add_u32 %0, %1, %0" : "+v"(vaddr[db]) : "s"(by));
+    for (int db = 0; db < NDBV; ++db) asm volatile("v_add_u32 %0, %1, %0" : "+v"(vaddr[0][db]) : "s"(by));
   };
   // the ring position is a compile-time constant in the unrolled inner loop, so every LDS address of a
   // step is a fixed register plus an immediate offset
@@ -718,8 +724,8 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
    for (int stage = 0; stage < NST; ++stage) {
     const int it = it0 + stage;
     if (it >= iters) break;
-    if (TWO_HALVES && stage == NST / 2) move_half(65536u);
-    if (TWO_HALVES && stage == 0 && it > 0) move_half(-65536u);
+    if (MOVES && stage == NST / 2) move_half(65536u);
+    if (MOVES && stage == 0 && it > 0) move_half(-65536u);
     const int tb = s0 + STEP * (g + TQ * it);
     // Tile `it` of this group has landed once at most the (A - 1) LPT loads issued after it are outstanding
     // (near the end fewer were issued, so everything is awaited); the barrier publishes all parts of the
@@ -758,10 +764,11 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     float16_t sacc[SUB];
 #pragma unroll
     for (int sb = 0; sb < SUB; ++sb) {
-      const int slo = (stage * SBYTES + sb * kStage) & 65535;
+      const int off = stage * SBYTES + sb * kStage;
+      const int shi = NHI == 2 ? off >> 16 : 0, slo = off & 65535;
       u32x4 ka[8];
 #pragma unroll
-      for (int s = 0; s < 8; ++s) ka[s] = lds_ld16_a(kaddr[s] + slo);
+      for (int s = 0; s < 8; ++s) ka[s] = lds_ld16_a(kaddr[shi][s] + slo);
       if (SUB == 1) __builtin_amdgcn_sched_barrier(0);
       const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       sacc[sb] = Mfma32<E>::run(ka[0], qop[0], PRESC ? cinit : zero);
@@ -773,13 +780,14 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     u32x4 va[SUB][4][2];
 #pragma unroll
     for (int sb = 0; sb < SUB; ++sb) {
-      const int slo = (stage * SBYTES + sb * kStage) & 65535;
+      const int off = stage * SBYTES + sb * kStage;
+      const int shi = NHI == 2 ? off >> 16 : 0, slo = off & 65535;
 #pragma unroll
       for (int db = 0; db < NDBV; ++db)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const u32x2 lo = lds_tr16_a(vaddr[db] + slo + (16 * u) * 256);
-          const u32x2 hi = lds_tr16_a(vaddr[db] + slo + (16 * u + 8) * 256);
+          const u32x2 lo = lds_tr16_a(vaddr[shi][db] + slo + (16 * u) * 256);
+          const u32x2 hi = lds_tr16_a(vaddr[shi][db] + slo + (16 * u + 8) * 256);
           va[sb][db][u] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
     }
