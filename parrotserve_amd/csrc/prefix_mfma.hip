@@ -651,6 +651,9 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     const bool mine = wk.pair_half < 0 || h == half;
     u32x4 raw[8];
     if (my_iters >= NST / 2) wait_vmcnt<NST / 2 * LPT>(); else wait_vmcnt<0>();  // the query rows, not the ring behind
+    // (the rows come by loads the compiler does not know of: nothing else ties the reads below to the wait)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int s = 0; s < 8; ++s) raw[s] = lds_ld16_a(q_lds + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16));
     __syncthreads();
