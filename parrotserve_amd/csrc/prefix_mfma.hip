@@ -577,16 +577,21 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
                lds_addr_of(smem) + kWinOff + (512 * k + 64 * w8) * 4);
 
   // The query rows are requested right behind the slot ids, as whole rows (four per load, 16 lanes a row) that land in
-  // the upper half of the group's ring: every wave brings the 32 rows it multiplies, in the K tiles' layout, and takes
-  // its operands from there.  (Loaded as operands, 16 bytes of a row per lane, they are 64 cache lines a load, and
-  // behind the ring they arrive after all of it: 64 requests, 32 heads over 8 KV heads, 4096 tokens 39.8 us against 36.7,
-  // a Fill of 61 queries over 1987 tokens 17.9 against 16.8.)
-  const uint32_t q_lds = lds_addr_of(gl) + (NST / 2) * SBYTES + qb * 8192;
+  // the upper half of the first group's ring, in the K tiles' layout, and are read back as operands.  (Loaded as operands,
+  // 16 bytes of a row per lane, they are 64 cache lines a load, and behind the ring they arrive after all of it.)
+  // The token groups multiply the same rows, so the workgroup brings them once, QB loads a wave, and leaves out the
+  // loads without a live row.  (Every group for itself, all rows live or not, is 64 KB whatever the tile holds: a Fill of
+  // one query over 101 tokens took 8.2 us instead of 7.5, of 16 over 516 11.9 instead of 11.3, and a decode step of 8
+  // requests over 512 + 128 tokens 16.4 instead of 15.4; with the operands loaded directly 7.5, 11.3 and 18.1.)
+  // One token group (256 queries): a wave's loads are the rows it multiplies, all eight of them always.
+  const uint32_t q_lds = lds_addr_of(smem) + (NST / 2) * SBYTES;
   static_assert((NST - NST / 2) * SBYTES >= QB * 8192, "the query rows fit the upper half of the ring");
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane >> 4), q = 32 * qb + r, qc = q < wk.nq ? q : 0;
-    int cg = (lane & 15) ^ (r & 15);  // the 16-byte chunk of the row at this place
+  for (int i = 0; i < QB; ++i) {
+    const int first = 4 * (QB * w8 + i);
+    if (TQ > 1 && first >= wk.nq) break;  // wave-uniform
+    const int q = first + (lane >> 4), qc = q < wk.nq ? q : 0;
+    int cg = (lane & 15) ^ (q & 15);  // the 16-byte chunk of the row at this place
     const uint16_t* qp = wk.qrow0;
     if (wk.pair_half >= 0) {
       // a 64-wide head as one half of a head pair: the row pointer points at this half's 64 values; 2: rows alternate
@@ -597,7 +602,7 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
       cg = cg * 8 < wk.head_dim ? cg : 0;  // past a short row its first chunk
       qp += (int64_t)(qc >> wk.gshift) * wk.q_stride + (qc & ((1 << wk.gshift) - 1)) * kPD;
     }
-    lds_dma16<false>(qp + cg * 8, q_lds + i * 1024);
+    lds_dma16<false>(qp + cg * 8, q_lds + first * 256);
   }
 
   // staging: row group L (0..7 K, 8..15 V) covers tokens 4 (L & 7) .. +3, 16 lanes per token row; this wave
@@ -631,8 +636,9 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   const int ntile = (s1 - s0 + STEP - 1) / STEP;
   const int iters = (ntile + TQ - 1) / TQ;                 // same for all eight waves
   const int my_iters = ntile > g ? (ntile - g + TQ - 1) / TQ : 0;  // tiles of this token group
-  wait_vmcnt<8>();                                         // this wave's part of the window; its query rows are behind
-  __syncthreads();                                         // window visible
+  // this wave's part of the window and of the shared query rows; its own eight query loads may still be out
+  if constexpr (TQ > 1) wait_vmcnt<0>(); else wait_vmcnt<8>();
+  __syncthreads();                                         // window and shared query rows visible
   PH_TL(1);
   // the whole ring is filled up front: tiles 0 .. A (the main loop issues tile it + A at step it >= 1), its upper half
   // once every wave has taken its queries
@@ -650,12 +656,14 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
     const int half = wk.pair_half == 2 ? q & 1 : wk.pair_half;
     const bool mine = wk.pair_half < 0 || h == half;
     u32x4 raw[8];
-    if (my_iters >= NST / 2) wait_vmcnt<NST / 2 * LPT>(); else wait_vmcnt<0>();  // the query rows, not the ring behind
-    // (the rows come by loads the compiler does not know of: nothing else ties the reads below to the wait)
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
+    if constexpr (TQ == 1) {  // this wave's own query rows, not the ring behind them
+      if (my_iters >= NST / 2) wait_vmcnt<NST / 2 * LPT>(); else wait_vmcnt<0>();
+      // (the rows come by loads the compiler does not know of: nothing else ties the reads below to the wait)
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+    }
 #pragma unroll
-    for (int s = 0; s < 8; ++s) raw[s] = lds_ld16_a(q_lds + ql * 256 + (((8 * h + s) ^ (ql & 15)) * 16));
+    for (int s = 0; s < 8; ++s) raw[s] = lds_ld16_a(q_lds + q * 256 + (((8 * h + s) ^ (ql & 15)) * 16));
     __syncthreads();
 #pragma unroll
     for (int j = NST / 2; j < NST; ++j)

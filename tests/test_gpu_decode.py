@@ -57,6 +57,23 @@ def test_units_back_to_back_on_each_tile(dev, sizes, P, s_hi, dtype):
     _check(case, dev)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,H,sizes,P,s_hi", [(128, 40, (1, 3, 4, 5, 31, 32, 33, 36, 63, 64), 300, 60),
+                                              (128, 16, (65, 96, 97, 100, 101, 128), 300, 60),
+                                              (64, 40, (1, 2, 3, 15, 16, 17, 18, 32), 300, 60),
+                                              (96, 24, (1, 4, 5, 33, 64), 300, 60)])
+def test_query_rows_up_to_the_last_live_one(dev, dtype, D, H, sizes, P, s_hi):
+    """A tile's query rows are staged four per load, and loads without a live row are left out: groups that end on,
+    before and behind a load's rows and a 32-row block, of mixed sizes, so that the rows left out hold what an earlier
+    unit of the workgroup left in LDS."""
+    from parrotserve_amd import synth
+
+    g = torch.Generator().manual_seed(D + H)
+    s = torch.randint(1, s_hi + 1, (sum(sizes),), generator=g).tolist()
+    case = synth.make_decode_case("rows", D + H, dtype, len(sizes), 0, P, s, H, D, 1 << 15, group_sizes=sizes)
+    _check(case, dev)
+
+
 def test_config1_shape_in_fp16(dev):
     """Config 1's shape (B 8, P 512, S U[32,128], 32x128, seed 0) cast to fp16 for the GPU."""
     from parrotserve_amd import synth

@@ -174,6 +174,16 @@ def test_prefill_window_filled_in_part(dev, n, tile, ctx):
     torch.testing.assert_close(got[0, :, 0].float(), ref.float(), **TOL[torch.float16])
 
 
+@pytest.mark.parametrize("q_lens", [[1], [3], [4], [5], [33], [36, 1, 4], [65, 96, 97], [100, 128]])
+def test_prefill_query_rows_up_to_the_last_live_one(dev, q_lens):
+    """Short Fills on the 64- and 128-query tiles: only the loads of query rows that hold a live one are issued."""
+    from parrotserve_amd import synth
+
+    case = synth.make_prefill_case("rows", 40 + sum(q_lens), torch.bfloat16, q_lens, 100, 4, 128, 1 << 12)
+    out, ref = run_prefill_case(case, dev)
+    torch.testing.assert_close(out.float(), ref.float(), **TOL[torch.bfloat16])
+
+
 def test_prefill_heads_not_multiple_of_eight_and_tail_tiles(dev):
     """Head counts that leave part of the padded head axis empty, chunks that end inside every tile size."""
     from parrotserve_amd import synth
