@@ -85,6 +85,21 @@ __device__ __forceinline__ void stream_item(const uint16_t* __restrict__ kc, con
       }
     };
 
+    // NQ > 1: the accumulators are final before the rows that fed them are loaded over.  (Left alone, the compiler
+    // moves the P.V sums behind the next batch's loads and keeps every V row in up to three places: 236 registers in
+    // fp16, and in the launches whose workgroups also hold a prefix tile 33 of them spilled.  32 query heads over 8 KV
+    // heads, fp16, every workgroup running both phases: 4 groups of 16 over 8192 + up to 4096 tokens 165.8 us against
+    // 146.3, 8 groups of 32 over 1024 + up to 512 102.0 against 86.5; bf16, four spilled, 151.5 against 147.9 and 87.3
+    // against 86.8.)
+    auto settle = [&]() {
+      if constexpr (NQ > 1) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(o[n][i]));
+      }
+    };
+
     if (STAGES == 2) {
       // two-stage software pipeline: the next batch's rows are in flight while this one is reduced
       load(kb[0], vb[0], 0);
@@ -92,8 +107,10 @@ __device__ __forceinline__ void stream_item(const uint16_t* __restrict__ kc, con
         const bool more1 = j0 + TB < nb;
         if (more1) load(kb[STAGES - 1], vb[STAGES - 1], j0 + TB);
         compute(kb[0], vb[0], j0);
+        settle();
         if (j0 + 2 * TB < nb) load(kb[0], vb[0], j0 + 2 * TB);
         if (more1) compute(kb[STAGES - 1], vb[STAGES - 1], j0 + TB);
+        settle();
       }
     } else {
       for (int j0 = 0; j0 < nb; j0 += TB) {

@@ -501,6 +501,33 @@ def test_query_heads_of_a_kv_head_streamed_together(dev, dtype, Hq, Hkv):
     torch.testing.assert_close(out3.cpu().float(), ref.float(), **TOL[dtype])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("groups,per,P,S", [(16, 12, 512, 300), (16, 20, 512, 200), (16, 40, 128, 512)])
+def test_query_heads_streamed_together_where_every_workgroup_runs_both_phases(dev, dtype, groups, per, P, S):
+    """Many groups over short prefixes, 32 query heads over 8 KV heads: the suffix is streamed for four query heads at
+    once by workgroups that also run prefix units, on the 64-, 128- and 256-query tile (the form and the stream are read
+    off the lane count: the whole device's, over the waves that a quarter of the heads take)."""
+    from parrotserve_amd import kernels, synth
+
+    Hq, Hkv, D, B = 32, 8, 128, groups * per
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    shape = dict(num_reqs=B, num_groups=groups, max_prefix_len=P, max_suffix_len=S, dtype=dtype, kv_group=4)
+    assert kernels.suffix_lane_capacity(dev, Hq, D, **shape) == cus * 8 // 2, "not the form this test is about"
+    g = torch.Generator().manual_seed(per)
+    s = torch.randint(1, S + 1, (B,), generator=g).tolist()
+    s[3] = S
+    case = synth.make_decode_case("gqas", per, dtype, groups, per, P, s, Hkv, D, 1 << 18)
+    q = torch.randn(B, Hq, D, generator=g).to(dtype)
+    hm = torch.arange(Hkv, dtype=torch.int32).repeat_interleave(4)
+    kc, vc = synth.pool_to_device(case.k_rows, case.v_rows, case.used_slots, case.pool_slots, dev)
+    tables = kernels.DecodeTables.build(case.pool_lists(case.prefix_lists), case.group_req_cu,
+                                        case.pool_lists(case.suffix_lists), dev, num_heads=Hq, head_dim=D, dtype=dtype,
+                                        kv_group=4)
+    out = kernels.decode_attention(q.to(dev), kc, vc, tables, head_mapping=hm.to(dev), kv_group=4)
+    ref = ref_decode_attention(q, case.k_rows[:, hm.long()], case.v_rows[:, hm.long()], case.full_lists())
+    torch.testing.assert_close(out.cpu().float(), ref.float(), **TOL[dtype])
+
+
 def test_any_head_mapping_and_the_identity(dev):
     """A mapping that is not h // G (here a permutation with repeats) runs per request; multi-query attention (one
     KV head); and the identity mapping over equal head counts is the plain call, bit for bit.  The split entry
