@@ -95,11 +95,9 @@ def _stream() -> int:
 
 
 def _empty_rows(t: torch.Tensor) -> torch.Tensor:
-    """A new contiguous tensor of the shape, type and device of ``t`` (two thirds of ``torch.empty``'s host time where
-    ``t`` is contiguous, and with it the layout that ``empty_like`` keeps)."""
-    if t.is_contiguous():
-        return torch.empty_like(t)
-    return torch.empty(t.shape, dtype=t.dtype, device=t.device)
+    """A new dense tensor of the shape, type and device of ``t`` (1.3 us of host time, ``torch.empty`` 2.3).  The format is
+    named because ``empty_like`` alone keeps the outer stride of a one-row slice."""
+    return torch.empty_like(t, memory_format=torch.contiguous_format)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

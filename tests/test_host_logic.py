@@ -375,3 +375,17 @@ def test_model_cache_storage_takes_the_reference_call_form():
     same = mem.init_model_cache_storage(2, 10, 4, 16, torch.float32, "cpu", max_seq_len=32)
     assert torch.equal(same.cos_sin_cache, store.cos_sin_cache)
     mem.Model_Cache = None
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (5, 8), (0, 8), (1, 2, 8), (5, 2, 8), (1, 1, 8)])
+@pytest.mark.parametrize("slot", [0, 1])
+def test_results_are_dense_whatever_their_input_was_cut_from(shape, slot):
+    """A result's strides are those of a new tensor of its shape, also for one row cut from a fused projection (which
+    counts as contiguous at any outer stride)."""
+    import torch
+
+    from parrotserve_amd import kernels
+
+    part = torch.chunk(torch.zeros(shape[0], 3 * shape[1], *shape[2:], dtype=torch.float16), 3, dim=1)[slot]
+    out = kernels._empty_rows(part)
+    assert out.shape == part.shape and out.dtype == part.dtype and out.stride() == torch.empty(shape).stride()
