@@ -45,15 +45,38 @@ def test_shared_prefix_decode(dev, dtype, B, P, H):
 @pytest.mark.parametrize("sizes,P,s_hi,dtype", [((256, 131), 2100, 40, torch.float16), ((256,), 700, 3, torch.bfloat16),
                                                 ((97, 128, 65), 2050, 100, torch.bfloat16),
                                                 ((64, 33, 1), 4224, 90, torch.float16)])
-def test_units_back_to_back_on_each_tile(dev, sizes, P, s_hi, dtype):
-    """A workgroup that walks several prefix units stages every unit's slots and query rows over the last one's ring: the
-    64-, 128- and 256-query tiles with groups that fill their last 32-row block and groups that do not, short suffixes
-    (every workgroup runs both phases) and long ones."""
+def test_groups_that_fill_their_tile_and_groups_that_do_not(dev, sizes, P, s_hi, dtype):
+    """The 64-, 128- and 256-query tiles with groups that fill their last 32-row block and groups that do not, prefixes
+    that end inside a step, the two phases in workgroups of their own."""
     from parrotserve_amd import synth
 
     g = torch.Generator().manual_seed(P)
     s = torch.randint(1, s_hi + 1, (sum(sizes),), generator=g).tolist()
     case = synth.make_decode_case("units", P, dtype, len(sizes), 0, P, s, 40, 128, 1 << 16, group_sizes=sizes)
+    assert not _shared_form(dev, case)
+    _check(case, dev)
+
+
+@pytest.mark.parametrize("H,sizes,P,S,shared", [(40, (40, 33, 47), 130, 100, False),
+                                                (16, (100, 72, 128, 100), 130, 100, False),
+                                                (16, (150, 131, 169), 130, 200, False),
+                                                (64, (33, 1, 64, 40, 28, 32), 130, 16, True),
+                                                (32, (70, 66, 97, 128, 65, 33, 70, 71, 40, 60), 130, 3, True),
+                                                (32, (256, 131, 97, 129, 33, 130, 129, 128, 128), 130, 3, True)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_units_back_to_back_on_each_tile(dev, dtype, H, sizes, P, S, shared):
+    """A workgroup that walks several prefix units stages every unit's slots and query rows over the last one's ring: the
+    64-, 128- and 256-query tile in the form with prefix-only workgroups and in the one whose workgroups run both phases,
+    with more units (one split alone has groups x heads of them) than workgroups that take them."""
+    from parrotserve_amd import synth
+
+    g = torch.Generator().manual_seed(sum(sizes))
+    s = torch.randint(1, S + 1, (sum(sizes),), generator=g).tolist()
+    s[0] = S
+    case = synth.make_decode_case("units", H, dtype, len(sizes), 0, P, s, H, 128, 1 << 17, group_sizes=sizes)
+    np_, cus = _role_split(dev, case)
+    assert _shared_form(dev, case) == shared
+    assert len(sizes) * H > (cus if shared else np_), "every unit has a workgroup of its own"
     _check(case, dev)
 
 
@@ -132,6 +155,16 @@ def _role_split(dev, case):
     heads_per_wave = 4 if D > 64 else 8  # a head takes D / 8 lanes of a wave, rounded up to a power of two
     hgroups = (H + heads_per_wave - 1) // heads_per_wave
     return cus - (lanes * hgroups + 7) // 8, cus
+
+
+def _shared_form(dev, case):
+    """Does every workgroup of this batch's launch run both phases?  Then a plan is to be cut for the whole device."""
+    from parrotserve_amd import kernels
+
+    B, H, D = case.q.shape
+    shape = dict(num_reqs=B, num_groups=len(case.prefix_lists), max_prefix_len=max(len(p) for p in case.prefix_lists),
+                 max_suffix_len=max(len(x) for x in case.suffix_lists), dtype=case.dtype)
+    return kernels.suffix_lane_capacity(dev, H, D, **shape) == kernels.suffix_lane_capacity(dev, H, D)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
