@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <mutex>
 
 namespace ph {
@@ -133,15 +134,15 @@ static RoleChoice choose_roles(const FusedShape& f, int64_t max_prefix, int64_t 
   const double floor_us = 4.0 + (f.prefix_mb + f.suffix_mb) / kHbm;
   // a step of the 128- and 256-query tiles is twice and four times the matrix work of the 64-query tile's
   const double tile_mul = f.query_tile == 256 ? 1.5 : f.query_tile == 128 ? 1.1 : 1.0;
-  RoleChoice best{1, 1, 0.0};
-  double best_cost = -1.0;
+  RoleChoice best{1, 1, std::numeric_limits<double>::infinity()};
   const int64_t max_splits = std::max<int64_t>(1, cdiv(max_prefix, 4 * kPrefixTile));
   for (int64_t s = 1; s <= 64 && s <= max_splits; ++s) {
     const int64_t tok = round_up(cdiv(max_prefix, s), 2 * kPrefixTile);
     if (cdiv(max_prefix, tok) != s) continue;  // rounding left a split empty: the same plan as a smaller s
     const double steps = (double)cdiv(tok, 2 * kPrefixTile);
     const int64_t units = f.units_per_split * s;
-    for (int64_t r = 1; r <= 8; ++r) {
+    // up to eight units a workgroup, or as many as it takes to fit the device (64 groups x 32 heads: 2048 units)
+    for (int64_t r = 1, most = std::max<int64_t>(8, cdiv(units, std::max<int64_t>(1, cus - 1))); r <= most; ++r) {
       const int64_t np = cdiv(units, r);
       if (np > cus - 1) continue;
       const double t_prefix = kFirst + r * (steps * kStep * tile_mul + kFold) + (r - 1) * kNext + kMargin;
@@ -149,10 +150,7 @@ static RoleChoice choose_roles(const FusedShape& f, int64_t max_prefix, int64_t 
       const double t_suffix =
           6.0 + (double)cdiv(f.reqs, lanes) * kPiece + f.suffix_mb / std::min(kHbm, (double)(cus - np) * kCu);
       const double cost = std::max(std::max(t_prefix, t_suffix), floor_us) + 0.25 * s;
-      if (best_cost < 0 || cost < best_cost) {
-        best_cost = cost;
-        best = RoleChoice{(int)s, (int)np, cost};
-      }
+      if (cost < best.cost_us) best = RoleChoice{(int)s, (int)np, cost};
     }
   }
   return best;
@@ -214,7 +212,8 @@ static DecodePlan plan_decode(int64_t B, int64_t H, int64_t groups, int64_t max_
     int64_t splits = sc.splits;
     if (roles && max_suffix > 0) {
       const RoleChoice rc = choose_roles(f, max_prefix, cus);
-      if (rc.cost_us < sc.cost_us) {
+      // (a prefix launch of its own holds the groups in the grid's z extent)
+      if (rc.cost_us < sc.cost_us || groups > 65535) {
         splits = rc.splits;
         p.prefix_wgs = rc.prefix_wgs;
       }

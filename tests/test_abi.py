@@ -74,6 +74,10 @@ def test_how_the_planner_divides_a_256_unit_device():
     assert lanes(64, 32, 128, f16, 1, 4096, 512, 4) > 2 * lanes(64, 32, 128, f16, 1, 4096, 512, 1)
     assert lanes(64, 32, 128, f16, 1, 4096, 60, 4) <= 256
     assert lanes(64, 32, 128, f16, 0, 0, 512, 2) == 256
+    # more prefix units than eight times the device: still most compute units on the prefix, or the undivided form
+    for groups in (63, 64, 128, 1000):
+        for own in (20, 100, 3000):
+            assert lanes(2 * groups, 32, 128, f16, groups, 1000, own, 1) in [256, *range(1, 128)]
 
 
 def _prefill_plan(q_lens, ctx_lens, heads, dim=128, workspace=1 << 40, spare_slots=0):

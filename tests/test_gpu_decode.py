@@ -221,6 +221,17 @@ def test_prefix_workgroups_walk_several_units_each(dev):
     _check(case, dev)
 
 
+@pytest.mark.parametrize("groups,H,S", [(130, 16, 20), (130, 16, 400), (64, 32, 30)])
+def test_more_prefix_units_than_eight_times_the_device(dev, groups, H, S):
+    """Many small groups: 2048 prefix units and more in a single split."""
+    from parrotserve_amd import synth
+
+    g = torch.Generator().manual_seed(groups)
+    s = torch.randint(1, S + 1, (groups,), generator=g).tolist()
+    case = synth.make_decode_case("many", groups, torch.float16, groups, 1, 140, s, H, 128, 1 << 17)
+    _check(case, dev)
+
+
 def test_two_role_launch_with_empty_suffixes(dev):
     """Requests whose own list is empty inside a batch that takes the two-role launch (their output is the prefix
     part alone), and, with every list empty, the prefix phase on its own."""
