@@ -65,8 +65,8 @@ __device__ __forceinline__ void lds_dma16(const void* gptr, uint32_t lds_addr) {
   else
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
 }
-// 4 bytes per lane the same way: used only to pull cache lines towards L2 ahead of the row loads (the data
-// lands in an LDS area nobody reads, so no register waits for it)
+// 4 bytes per lane the same way: fills the slot window, and pulls cache lines towards L2 ahead of the row loads (that
+// data lands in an LDS area nobody reads, so no register waits for it)
 __device__ __forceinline__ void lds_dma4(const void* gptr, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
 }
@@ -695,9 +695,9 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
 
   // Operand read addresses (a ring of 128 KB is two times the 16-bit immediate's reach).  Prefill holds a set for each
   // half.  Decode, whose kernels have no registers left for a second set (the row loads' addresses were spilled, and
-  // every reload from scratch waited for the rows in flight), moves one set there and back; in prefill the
-  // moves are 1 % of the loop (against operands loaded from global memory, an 8192-token Fill took 701 us instead of 693
-  // with one set, 671 instead of 676 with two).
+  // every reload from scratch waited for the rows in flight), moves one set there and back; in prefill the moves are 1 %
+  // of the loop (device time of eight alternating runs within 0.5 %: a Fill of 8192 tokens, 40 heads, 682 us with one set
+  // and 676.5 with two, 16 chunks of 544 over 2048 tokens 546 and 541).
   // K: row ql, chunk (8h + s) swizzled by the row; V: the transposing read's row/column of this lane.
   constexpr bool TWO_HALVES = NST * SBYTES > 65536;
   static_assert(NST * SBYTES <= 2 * 65536, "two halves of the immediate's reach");
@@ -1070,8 +1070,8 @@ struct WideTile {
 // both kinds spread evenly over the chip.
 //
 // Shared (np == 0): workgroup b owns the prefix units b, b + grid, ... (normally at most one) and its eight waves one
-// suffix piece each.  Order inside a workgroup: suffix records requested, prefix prologue (slot window, first K/V
-// tiles sent on their way into LDS, Q), then the suffix stream (it needs no LDS), then the prefix main loop on tiles
+// suffix piece each.  Order inside a workgroup: suffix records requested, prefix prologue (slot window and query
+// rows, the ring's K/V tiles sent on their way), then the suffix stream (it needs no LDS), then the prefix main loop on tiles
 // that landed long ago, then the fold.  Taken when the suffix is too short to keep separate workgroups busy.
 //
 // The merge stays a separate launch: it needs every part.
@@ -1106,36 +1106,36 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
       }
     }
   } else {
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 8 + (threadIdx.x >> 6));
-  // this wave's first suffix piece: its record is requested before anything else
-  const int piece0 = wave < slots ? wave / hgroups : -1;
-  int4 rec0 = {0, 0, 0, 0}, rec1 = {0, 0, 0, 0};
-  if (piece0 >= 0) {
-    rec0 = ia.lane_rec[2 * piece0];
-    rec1 = ia.lane_rec[2 * piece0 + 1];
-  }
-  auto suffix = [&]() {
-    if (piece0 >= 0) run_piece_rec<E, DS, 4, 2, NQ>(ia, wave - piece0 * hgroups, rec0, rec1);
-    for (int s = wave + gridDim.x * 8; s < slots; s += gridDim.x * 8) {
-      const int piece = s / hgroups;
-      run_piece<E, DS, 4, 2, NQ>(ia, piece, s - piece * hgroups);
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 8 + (threadIdx.x >> 6));
+    // this wave's first suffix piece: its record is requested before anything else
+    const int piece0 = wave < slots ? wave / hgroups : -1;
+    int4 rec0 = {0, 0, 0, 0}, rec1 = {0, 0, 0, 0};
+    if (piece0 >= 0) {
+      rec0 = ia.lane_rec[2 * piece0];
+      rec1 = ia.lane_rec[2 * piece0 + 1];
     }
-  };
-  if ((int)blockIdx.x < n_units) {
-    // the suffix stream runs between the first unit's prologue and its main loop
-    const int u = blockIdx.x;
-    const int split = u % pa.n_splits;
-    const int rest = u / pa.n_splits;
-    prefix_unit8<E, TQ, decltype(suffix), SUB, PRESC>(pa, split, rest % pa.H, rest / pa.H, mtiles, smem, suffix);
-    for (int v = u + gridDim.x; v < n_units; v += gridDim.x) {
-      __syncthreads();  // the fold scratch of the last unit is the staging ring of the next
-      const int sp = v % pa.n_splits;
-      const int rs = v / pa.n_splits;
-      prefix_unit8<E, TQ, NoMid, SUB, PRESC>(pa, sp, rs % pa.H, rs / pa.H, mtiles, smem);
+    auto suffix = [&]() {
+      if (piece0 >= 0) run_piece_rec<E, DS, 4, 2, NQ>(ia, wave - piece0 * hgroups, rec0, rec1);
+      for (int s = wave + gridDim.x * 8; s < slots; s += gridDim.x * 8) {
+        const int piece = s / hgroups;
+        run_piece<E, DS, 4, 2, NQ>(ia, piece, s - piece * hgroups);
+      }
+    };
+    if ((int)blockIdx.x < n_units) {
+      // the suffix stream runs between the first unit's prologue and its main loop
+      const int u = blockIdx.x;
+      const int split = u % pa.n_splits;
+      const int rest = u / pa.n_splits;
+      prefix_unit8<E, TQ, decltype(suffix), SUB, PRESC>(pa, split, rest % pa.H, rest / pa.H, mtiles, smem, suffix);
+      for (int v = u + gridDim.x; v < n_units; v += gridDim.x) {
+        __syncthreads();  // the fold scratch of the last unit is the staging ring of the next
+        const int sp = v % pa.n_splits;
+        const int rs = v / pa.n_splits;
+        prefix_unit8<E, TQ, NoMid, SUB, PRESC>(pa, sp, rs % pa.H, rs / pa.H, mtiles, smem);
+      }
+    } else {
+      suffix();
     }
-  } else {
-    suffix();
-  }
   }
   PH_TL(11);
 }

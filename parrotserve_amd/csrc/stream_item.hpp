@@ -88,9 +88,8 @@ __device__ __forceinline__ void stream_item(const uint16_t* __restrict__ kc, con
     // NQ > 1: the accumulators are final before the rows that fed them are loaded over.  (Left alone, the compiler
     // moves the P.V sums behind the next batch's loads and keeps every V row in up to three places: 236 registers in
     // fp16, and in the launches whose workgroups also hold a prefix tile 33 of them spilled.  32 query heads over 8 KV
-    // heads, fp16, every workgroup running both phases: 4 groups of 16 over 8192 + up to 4096 tokens 165.8 us against
-    // 146.3, 8 groups of 32 over 1024 + up to 512 102.0 against 86.5; bf16, four spilled, 151.5 against 147.9 and 87.3
-    // against 86.8.)
+    // heads, every workgroup running both phases: 4 groups of 16 over 8192 + up to 4096 tokens in fp16 165.8 us against
+    // 146.3, 8 groups of 32 over 1024 + up to 512 102.0 against 86.5; in bf16 147.9 both, and 87.9 against 86.8.)
     auto settle = [&]() {
       if constexpr (NQ > 1) {
 #pragma unroll
