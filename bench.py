@@ -379,19 +379,19 @@ PREFILL_TIMELINE_MARKS = ["kernel entry", "slot window in LDS", "ring requested,
 
 
 def prefill_timeline(torch, lib, dev, launches=6):
-    """The same marks in the prefill kernel: one 256-query chunk over a 2048-token parent, 40 heads = 40 workgroups
-    that all start at once, so a workgroup's prologue (entry to step 0) and epilogue (loop done to exit) can be
-    read off beside its tile loop."""
+    """The same marks in the prefill kernel: six 256-query chunks over 2048-token parents, 40 heads = 240 workgroups of
+    256 queries that all start at once (fewer chunks get smaller tiles), so a workgroup's prologue (entry to step 0) and
+    epilogue (loop done to exit) can be read off beside its tile loop."""
     import numpy as np
     from parrotserve_amd import kernels
 
-    H, D, pool, n, par = 40, 128, 1 << 15, 256, 2048
+    H, D, pool, n, par, chunks = 40, 128, 1 << 15, 256, 2048, 6
     kc = torch.randn((pool, H, D), device=dev, dtype=torch.bfloat16)
     vc = torch.randn_like(kc)
-    slots = torch.randperm(pool, generator=torch.Generator().manual_seed(7))[: par + n].tolist()
-    q = torch.randn((n, H, D), device=dev, dtype=torch.bfloat16)
+    slots = torch.randperm(pool, generator=torch.Generator().manual_seed(7))[: chunks * (par + n)].view(chunks, -1)
+    q = torch.randn((chunks * n, H, D), device=dev, dtype=torch.bfloat16)
     o = torch.empty_like(q)
-    tab = kernels.PrefillTables.build([n], [slots], dev)
+    tab = kernels.PrefillTables.build([n] * chunks, slots.tolist(), dev)
     for _ in range(5):
         kernels.prefill_attention(q, kc, vc, tab, out=o)
     torch.cuda.synchronize()
@@ -405,8 +405,8 @@ def prefill_timeline(torch, lib, dev, launches=6):
         clk = np.zeros(4096 * 12, dtype=np.uint64)
         assert lib.ph_timeline_read(buf.ctypes.data_as(ctypes.c_void_p), buf.nbytes) == 0
         assert lib.ph_timeline_read_clocks(clk.ctypes.data_as(ctypes.c_void_p), clk.nbytes) == 0
-        t = buf.reshape(4096, 12).astype(np.float64)[: H * 8]
-        c = clk.reshape(4096, 12).astype(np.float64)[: H * 8]
+        t = buf.reshape(4096, 12).astype(np.float64)[: chunks * H * 8]
+        c = clk.reshape(4096, 12).astype(np.float64)[: chunks * H * 8]
         ok = (t[:, 7] > 0) & (t[:, 8] > t[:, 7])
         if ok.any():
             mhz.append(float(np.median((c[ok, 8] - c[ok, 7]) / ((t[ok, 8] - t[ok, 7]) / 100.0))))
@@ -429,7 +429,7 @@ def prefix_timeline(torch, lib, dev, launches=6):
     """The prefix kernel where the matrix pipe is the bound (one group of 1024 requests over 8192 tokens, 32 x 128
     fp16: 256 workgroups of 256 queries x 4096 tokens each, the same tile loop as the prefill's): time per 64-token
     step of a workgroup and the shader clock the compute units hold while every one of them runs the loop, from the
-    marks at the fourth step and at the end of the loop.  (The prefill timeline gives the same for 40 workgroups on
+    marks at the fourth step and at the end of the loop.  (The prefill timeline gives the same for 240 workgroups on
     256 compute units.)"""
     import numpy as np
 
