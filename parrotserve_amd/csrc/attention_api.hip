@@ -141,10 +141,10 @@ static RoleChoice choose_roles(const FusedShape& f, int64_t max_prefix, int64_t 
     if (cdiv(max_prefix, tok) != s) continue;  // rounding left a split empty: the same plan as a smaller s
     const double steps = (double)cdiv(tok, 2 * kPrefixTile);
     const int64_t units = f.units_per_split * s;
-    // up to eight units a workgroup, or as many as it takes to fit the device (64 groups x 32 heads: 2048 units)
-    for (int64_t r = 1, most = std::max<int64_t>(8, cdiv(units, std::max<int64_t>(1, cus - 1))); r <= most; ++r) {
+    // from the fewest units a workgroup that fit the device, up to eight or (64 groups x 32 heads: 2048 units) those
+    const int64_t least = std::max<int64_t>(1, cdiv(units, std::max<int64_t>(1, cus - 1)));
+    for (int64_t r = least; r <= std::max<int64_t>(8, least); ++r) {
       const int64_t np = cdiv(units, r);
-      if (np > cus - 1) continue;
       const double t_prefix = kFirst + r * (steps * kStep * tile_mul + kFold) + (r - 1) * kNext + kMargin;
       const int64_t lanes = std::max<int64_t>(1, (cus - np) * 8 / f.head_groups);
       const double t_suffix =
