@@ -134,16 +134,19 @@ static RoleChoice choose_roles(const FusedShape& f, int64_t max_prefix, int64_t 
   const double floor_us = 4.0 + (f.prefix_mb + f.suffix_mb) / kHbm;
   // a step of the 128- and 256-query tiles is twice and four times the matrix work of the 64-query tile's
   const double tile_mul = f.query_tile == 256 ? 1.5 : f.query_tile == 128 ? 1.1 : 1.0;
-  RoleChoice best{1, 1, std::numeric_limits<double>::infinity()};
+  // most units a prefix workgroup walks; where more are needed to fit the device (64 groups x 32 heads: 2048 units) this
+  // form is not a choice: one split on as many workgroups as fit, at no finite cost
+  constexpr int64_t kWalk = 8;
+  const int64_t room = std::max<int64_t>(1, cus - 1);
+  RoleChoice best{1, (int)cdiv(f.units_per_split, std::max<int64_t>(1, cdiv(f.units_per_split, room))),
+                  std::numeric_limits<double>::infinity()};
   const int64_t max_splits = std::max<int64_t>(1, cdiv(max_prefix, 4 * kPrefixTile));
   for (int64_t s = 1; s <= 64 && s <= max_splits; ++s) {
     const int64_t tok = round_up(cdiv(max_prefix, s), 2 * kPrefixTile);
     if (cdiv(max_prefix, tok) != s) continue;  // rounding left a split empty: the same plan as a smaller s
     const double steps = (double)cdiv(tok, 2 * kPrefixTile);
     const int64_t units = f.units_per_split * s;
-    // from the fewest units a workgroup that fit the device, up to eight or (64 groups x 32 heads: 2048 units) those
-    const int64_t least = std::max<int64_t>(1, cdiv(units, std::max<int64_t>(1, cus - 1)));
-    for (int64_t r = least; r <= std::max<int64_t>(8, least); ++r) {
+    for (int64_t r = std::max<int64_t>(1, cdiv(units, room)); r <= kWalk; ++r) {
       const int64_t np = cdiv(units, r);
       const double t_prefix = kFirst + r * (steps * kStep * tile_mul + kFold) + (r - 1) * kNext + kMargin;
       const int64_t lanes = std::max<int64_t>(1, (cus - np) * 8 / f.head_groups);
