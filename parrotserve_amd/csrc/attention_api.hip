@@ -117,7 +117,8 @@ constexpr double kHbmMbPerUs = 6.9;  // what the device sustains on this access 
 
 // Roles: the split count and the number of prefix-only workgroups.  A prefix workgroup is latency-bound next to
 // the suffix stream -- one 128-token step (64 KB) in flight ahead of the one it multiplies, about 2.7 us per step
-// with the memory system saturated, 12 us from launch to its first step -- so the prefix wants enough workgroups
+// with the memory system saturated, 12 us from launch to its first step (8.5 us since the query rows are no longer
+// loaded behind the ring; not refitted) -- so the prefix wants enough workgroups
 // to be done a little before the stream, and the stream wants the rest (it holds about 40 GB/s per compute unit).
 // A suffix wave spends about 4 us per piece before it streams (slot ids, then rows, then the partial's write), and
 // a lane walks at least requests / lanes pieces: with many short lists on few lanes that, not the bytes, is what
@@ -167,14 +168,17 @@ static RoleChoice choose_roles(const FusedShape& f, int64_t max_prefix, int64_t 
 // choose_roles' cost, which overstates a lightly loaded launch (its 12 us to the first step and 2.7 us per step are
 // what a prefix workgroup sees next to a saturating stream): the estimate of this form's time plus 11.5 us, that
 // offset fitted, with the step time of this form (3.1 us; x 1.44 on the 256-query tile, x 0.87 on the four-wave
-// tile) and its 9.3 us of start and end, to 106 shapes measured in both forms --
-// 1 .. 16 groups of 1 .. 256 requests, prefixes of 128 .. 16384 tokens, suffixes of up to 8 .. 4096 tokens, 32 and
-// 40 heads of 128.  Choosing by the two costs is within 0.3 % of the better form on average over those shapes and
-// 9 % at worst; the two phases in workgroups of their own win by 3 .. 25 % on most (small launches are chains of
-// memory latencies, which then run side by side: 16 requests x 256 over 1024 tokens 19.3 against 25.6 us; the
-// reference benchmark's 64 x 20 over 8192 at 40 heads 49.3 against 52.6 us) and lose by 3 .. 19 % where the prefix
-// wants every compute unit: long prefixes under tiny suffixes, 256-query tiles under short suffixes, and many
-// small groups whose units fill the device evenly (8 groups of 8 over 2000 tokens: 77 against 66 us).
+// tile) and its 9.3 us of start and end, to 106 shapes measured in both forms, as choose_roles' constants were.
+// The kernels have become faster since (the first step of a prefix workgroup at 8.5 us, no spills on the 256-query
+// tile), the roles form more so: over 166 shapes drawn at random -- 1 .. 16 groups of 1 .. 256 requests, prefixes of
+// 128 .. 16384 tokens, suffixes of up to 4 .. 4096 tokens, heads of 128 and 64, plain and grouped -- the choice by the
+// two costs is 1.4 % slower than the better form on average (4 query heads per KV head 2.8 %, 8 4.8 %), by more than
+// 5 % on 18 of them, where it keeps this form for small groups (profiles/decode_form_sweep.txt).  The two phases in
+// workgroups of their own win by 3 .. 40 % on most (small launches are chains of memory latencies, which then run side
+// by side: 16 requests x 256 over 1024 tokens 19.3 against 25.6 us; the reference benchmark's 64 x 20 over 8192 at 40
+// heads 49.3 against 52.6 us) and lose by 3 .. 19 % where the prefix wants every compute unit: long prefixes under tiny
+// suffixes, 256-query tiles under short suffixes, and many small groups whose units fill the device evenly (8 groups of
+// 8 over 2000 tokens: 77 against 66 us).
 struct SharedChoice {
   int splits;
   double cost_us;
@@ -432,9 +436,10 @@ static size_t prefill_parts_room(int64_t T, int64_t H, int64_t D, int64_t max_kv
 // knows the query total, the chunk count, the longest context and the sum of all contexts (kv_rows): tiles per chunk
 // and visible lengths are averages, and the longest context bounds the launch from below.
 // Constants fitted in bf16 at head size 128 (1 to 16 chunks of 16 to 4096 tokens over parents of 0 to 6000, 32 and 40
-// heads).  Checked against one part per context on the tile of the average chunk length: 384 launches of 64-, 96- and
-// 128-wide heads, 2 to 80 of them, 1 to 300 chunks, equal and very different contexts, take 0.15 to 1.013 of its time,
-// 0.69 in the geometric mean, three of them more than 1.002 (profiles/prefill_plan_sweep.txt).
+// heads) on kernels whose start took 1 to 2 us longer.  Checked on the present ones against one part per context on
+// the tile of the average chunk length: 384 launches of 64-, 96- and 128-wide heads, 2 to 80 of them, 1 to 300 chunks,
+// equal and very different contexts, take 0.14 to 1.20 of its time, 0.75 in the geometric mean, 43 of them more than
+// 1.002 and eleven more than 1.02 (profiles/prefill_plan_sweep.txt).
 static double prefill_cost_us(int64_t T, int64_t C, int64_t H, int64_t D, int64_t max_kv, int64_t kv_rows, int tile_q,
                               int64_t splits, int64_t cus) {
   const double start = tile_q == 256 ? 9.0 : 8.5;

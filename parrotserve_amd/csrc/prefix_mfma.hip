@@ -696,8 +696,9 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   // Operand read addresses (a ring of 128 KB is two times the 16-bit immediate's reach).  Prefill holds a set for each
   // half.  Decode, whose kernels have no registers left for a second set (the row loads' addresses were spilled, and
   // every reload from scratch waited for the rows in flight), moves one set there and back; in prefill the moves are 1 %
-  // of the loop (device time of eight alternating runs within 0.5 %: a Fill of 8192 tokens, 40 heads, 682 us with one set
-  // and 676.5 with two, 16 chunks of 544 over 2048 tokens 546 and 541).
+  // of the loop (captured launches, eight alternating runs within 0.5 %: a Fill of 8192 tokens, 40 heads, 682 us with one
+  // set and 676.5 with two, 16 chunks of 544 over 2048 tokens 546 and 541; in a queue of launches without a pause the chip
+  // lowers its clock further and neither is faster).
   // K: row ql, chunk (8h + s) swizzled by the row; V: the transposing read's row/column of this lane.
   constexpr bool TWO_HALVES = NST * SBYTES > 65536;
   static_assert(NST * SBYTES <= 2 * 65536, "two halves of the immediate's reach");
