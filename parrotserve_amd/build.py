@@ -33,7 +33,12 @@ FLAGS = [
 # difference of two infinities is guarded), so their max trees may drop the NaN-quieting of each input.
 # (A NaN in the inputs still reaches the result, through the exponentials and their sum: tests/test_gpu_prefill.py
 # and tests/test_gpu_decode.py hold it to that.)
-EXTRA_FLAGS = {"prefix_mfma.hip": ["-fno-honor-nans"]}
+# The sampler's passes over a row in registers are loops of up to fourteen rounds that stop early: the compiler unrolls
+# such a loop up to eight times by itself, and keeps the row in scratch memory where it does not.
+EXTRA_FLAGS = {
+    "prefix_mfma.hip": ["-fno-honor-nans"],
+    "sampler.hip": ["-mllvm", "-unroll-max-upperbound=16"],
+}
 
 
 def _compile(src: str, obj_dir: str, timeline: bool = False) -> str:

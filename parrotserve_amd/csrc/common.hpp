@@ -156,6 +156,24 @@ __device__ __forceinline__ float dpp_add(float v) {
   return v + __builtin_bit_cast(float, moved);
 }
 
+// max(v, v of the lane selected by a DPP control); a NaN in either is the result (v_maximum3_f32)
+template <int CTRL>
+__device__ __forceinline__ float dpp_maximum(float v) {
+  const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true);
+  return __builtin_elementwise_maximum(v, __builtin_bit_cast(float, moved));
+}
+
+// Every second row of 16 lanes of `a` trades places with the row before it of `b`; the upper half of `a` with the lower
+// half of `b`.  With both holding the same value, a lane of one then has its own and the same lane of the other its
+// neighbour's (lane ^ 16, lane ^ 32), in registers instead of a trip through LDS.  (Written as assembly because the
+// builtins' second result is mis-compiled by this toolchain.)
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+
 // Sum over aligned groups of W lanes (W a power of two <= 64); every lane of
 // the group ends with the group's sum.  Up to 16 lanes the exchange stays inside
 // a DPP row: quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror,
@@ -166,14 +184,47 @@ __device__ __forceinline__ float group_sum(float v) {
   if (W >= 4) v = dpp_add<0x4E>(v);
   if (W >= 8) v = dpp_add<0x141>(v);
   if (W >= 16) v = dpp_add<0x140>(v);
-  if (W >= 32) v += __shfl_xor(v, 16, kWave);
-  if (W >= 64) v += __shfl_xor(v, 32, kWave);
+  if (W >= 32) {
+    float o = v;
+    swap_rows(v, o);
+    v += o;
+  }
+  if (W >= 64) {
+    float o = v;
+    swap_halves(v, o);
+    v += o;
+  }
   return v;
 }
 template <int W>
 __device__ __forceinline__ float group_max(float v) {
 #pragma unroll
   for (int s = W / 2; s >= 1; s >>= 1) v = fmaxf(v, __shfl_xor(v, s, kWave));
+  return v;
+}
+// The wave's largest value, in every lane; NaN if there is one.
+__device__ __forceinline__ float wave_maximum(float v) {
+  v = dpp_maximum<0xB1>(v);
+  v = dpp_maximum<0x4E>(v);
+  v = dpp_maximum<0x141>(v);
+  v = dpp_maximum<0x140>(v);
+  float o = v;
+  swap_rows(v, o);
+  v = __builtin_elementwise_maximum(v, o);
+  o = v;
+  swap_halves(v, o);
+  return __builtin_elementwise_maximum(v, o);
+}
+
+// Inclusive sum over the wave's lanes, in registers (four shifts inside a row of 16 lanes, then the row totals
+// broadcast to the rows behind).
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2 and 3
   return v;
 }
 

@@ -482,12 +482,10 @@ constexpr int kMlOff = kWinOff + kWin * 4;        // (m, l, true max) of eight w
 constexpr int kPfOff = kMlOff + 8 * 3 * 256;    // landing area of the cache-line touches (256 bytes per wave)
 constexpr int kTile8Lds = kPfOff + 8 * 256;
 
-// max over the two 32-lane halves of the wave: lane l gets max(x[l], x[l ^ 32]).  One lane-swap instruction
-// (lanes 32..63 of the first register trade places with lanes 0..31 of the second) instead of a trip
-// through LDS; written as assembly because the builtin's second result is mis-compiled by this toolchain.
+// max over the two 32-lane halves of the wave: lane l gets max(x[l], x[l ^ 32])
 __device__ __forceinline__ float half_swap_max(float x) {
   float a = x, b = x;
-  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  swap_halves(a, b);
   return fmaxf(a, b);
 }
 
@@ -1139,18 +1137,6 @@ __global__ __launch_bounds__(512) void decode_fused_kernel(PrefixArgs pa, int mt
     }
   }
   PH_TL(11);
-}
-
-// Inclusive sum over the wave's lanes, in registers (four shifts inside a row of 16 lanes, then the row totals
-// broadcast to the rows behind).
-__device__ __forceinline__ int wave_prefix_sum(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2 and 3
-  return v;
 }
 
 // The query tile a workgroup takes: tile rows count from the last tile of the last chunk backwards (later tiles of a

@@ -23,6 +23,8 @@
 // masses are exact, the bisection's carry the rounding of fp32 sums (a few 1e-7 of the row's mass): where top_p falls
 // that close to the mass before a token, the two can differ by that token, and so can the two kernels (and with them
 // ph_sample_top_p and ph_top_p_probs, which takes the second).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace ph {
@@ -263,20 +265,55 @@ __global__ __launch_bounds__(kSampThreads) void sample_top_p_kernel(const SampAr
 // x / T rounded to nearest for many x and one T: r = 1 / T rounded to nearest, one Newton correction of x * r, exact
 // while nothing leaves the normal range; 3 instructions in place of a division's 10.
 __device__ __forceinline__ bool quotient_by_reciprocal(float T) { return T >= 0x1p-40f && T <= 0x1p40f; }
+template <typename E>
 __device__ __forceinline__ float div_by(float x, float T, float r) {
-  const float q = x * r;
-  return __builtin_fabsf(q) < INFINITY ? __builtin_fmaf(__builtin_fmaf(-q, T, x), r, q) : q;
+  const float q = x * r, c = __builtin_fmaf(__builtin_fmaf(-q, T, x), r, q);
+  // infinite logits; an fp16 quotient cannot become infinite otherwise, and one instruction tells
+  if (std::is_same<E, F16>::value) return __builtin_amdgcn_div_fixupf(c, T, x);
+  return __builtin_fabsf(q) < INFINITY ? c : q;
+}
+// N quotients x / T, rounded to the element type
+template <typename E, int N>
+__device__ __forceinline__ void divide(float (&x)[N], float T, float r, bool by_r) {
+  if (!by_r) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = Logit<E>::round(__fdiv_rn(x[j], T));
+    return;
+  }
+  if constexpr (Logit<E>::kBytes == 2) {
+#pragma unroll
+    for (int j = 0; j < N; j += 2) {
+      const uint32_t two = pack2<E>(div_by<E>(x[j], T, r), div_by<E>(x[j + 1], T, r));
+      x[j] = Elem<E>::lo(two);
+      x[j + 1] = Elem<E>::hi(two);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = div_by<E>(x[j], T, r);
+  }
+}
+// e^x: 2^n 2^f with n + f = x log2(e), the product carried in two floats; to the bit what expf returns (every float from
+// -110 to 1000 compared), two instructions shorter: nothing but +infinity needs the overflow case.
+__device__ __forceinline__ float exp_of(float x) {
+  constexpr float kHi = 0x1.715476p+0f, kLo = 0x1.4ae0bep-26f;  // log2(e)
+  const float hi = x * kHi, lo = __builtin_fmaf(x, kLo, __builtin_fmaf(x, kHi, -hi)), n = __builtin_rintf(hi);
+  const float y = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
+  return x < -0x1.9d1da0p+6f ? 0.f : y;  // (an x of -infinity, too)
 }
 
-// Histograms of the mass over the bit pattern of e: 32 bins per power of two, then 9 bits inside the bin the mass
-// crosses its target in, then the last 9 bits.  Values of one coarse bin differ in the low 18 bits of their mantissas
-// only, so a bin takes the tokens' count (from bit 40 up) and the sum of those bits: whole numbers, one add per token.
-// Masses of different bins are compared in units of 2^-46 (a row's mass stays below 2^62), inside a bin in mantissas.
+// Histograms of the mass over the bit pattern of e: 32 bins per power of two, then 8 bits inside the bin the mass
+// crosses its target in, then, where that finer bin holds more than one value, the last 10 bits.  Values of one coarse
+// bin differ in the low 18 bits of their mantissas only, so a bin takes the tokens' count (from bit 40 up) and the sum
+// of those bits: whole numbers, one add per token.  Masses of different bins are compared in units of 2^-46 (a row's
+// mass stays below 2^62), inside a bin in mantissas.
 typedef unsigned long long mass_t;
-constexpr int kHistShift = 18, kHistFine = 9, kHistCount = 40;
-constexpr int kHistBins = 4096;  // up to the bin of e == 1 and beyond (any pattern is masked into them)
-static_assert((0x3f800000 >> kHistShift) < kHistBins && kHistBins == 4 * kSampThreads, "four bins per lane");
+constexpr int kHistShift = 18, kHistFine = 8, kHistLast = kHistShift - kHistFine, kHistCount = 40;
+constexpr int kHistBins = 2048;  // the bins 2048 .. 4095 of the pattern: from below kHistLeast to beyond e == 1
 constexpr uint32_t kHistLeast = 0x21800000u;  // 2^-60: less is no mass
+constexpr int kHistFirst = kHistLeast >> kHistShift;  // the bins below hold what is no mass
+static_assert(kHistFirst >= kHistBins + kWave && (kHistLeast & ((1u << kHistShift) - 1)) == 0 &&
+                  (0x3f800000 >> kHistShift) < 2 * kHistBins && kHistBins == 2 * kSampThreads,
+              "two bins per lane");
 __device__ __forceinline__ uint32_t mantissa(uint32_t bits) { return (bits & 0x7fffffu) | 0x800000u; }
 __device__ __forceinline__ mass_t hist_entry(uint32_t bits) {
   return ((mass_t)1 << kHistCount) | (bits & ((1u << kHistShift) - 1));
@@ -291,64 +328,156 @@ __device__ __forceinline__ mass_t hist_mantissas(mass_t entry, uint32_t bin) {
 __device__ __forceinline__ int mass_shift(uint32_t bin) {  // mantissas of a coarse bin << this = units of 2^-46
   return (int)(bin >> (23 - kHistShift)) - (127 - 23);
 }
-__device__ __forceinline__ mass_t* hist_slot(mass_t* coarse, uint32_t bits) {
+__device__ __forceinline__ mass_t* hist_slot(mass_t* coarse, uint32_t bits) {  // (a pattern of no bin is masked into one)
   return reinterpret_cast<mass_t*>(reinterpret_cast<char*>(coarse) +
                                    ((bits >> (kHistShift - 3)) & ((kHistBins - 1) * sizeof(mass_t))));
 }
-__device__ __forceinline__ mass_t wave_prefix_mass(mass_t v, int lane) {
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const mass_t up = __shfl_up(v, d, kWave);
-    if (lane >= d) v += up;
-  }
+// Inclusive sum over the lanes, in registers (whole numbers: any order gives the same).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ mass_t mass_from(mass_t v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+  return ((mass_t)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+__device__ __forceinline__ mass_t row_prefix_mass(mass_t v) {  // over each row of 16 lanes
+  v += mass_from<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v += mass_from<0x112, 0xf>(v);
+  v += mass_from<0x114, 0xf>(v);
+  v += mass_from<0x118, 0xf>(v);
   return v;
 }
+__device__ __forceinline__ mass_t wave_prefix_mass(mass_t v) {
+  v = row_prefix_mass(v);
+  v += mass_from<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v += mass_from<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ mass_t lane_mass(mass_t v, int lane) {  // the value of one lane
+  return ((mass_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
+// a / b for a < 2^40 and 2^23 <= b < 2^24: a quotient that is no whole number is further than 2^-24 from one, the
+// division's error below 2^-35
+__device__ __forceinline__ int count_of(mass_t a, uint32_t b) { return (int)((double)a / (double)b); }
 
 struct SampHist {
-  mass_t coarse[kHistBins];
-  mass_t fine[2][1 << kHistFine];
+  alignas(16) mass_t coarse[kHistBins];
+  mass_t fine[1 << kHistFine];
+  uint32_t least[1 << kHistFine], most[1 << kHistFine];  // of the patterns in a fine bin
+  mass_t last[1 << kHistLast];
   mass_t wave_mass[kSampWaves];
   mass_t goal;     // what the bins still in question may hold above the cut, in mantissas
   uint32_t bin;    // the bin the mass crosses the target in
-  uint32_t thr;    // bit pattern of the smallest surviving e ...
+  uint32_t thr;    // bit pattern of the smallest surviving e (0: not known yet) ...
   int n_equal;     // ... how many tokens of that value survive
   int equal;       // ... and how many there are
 };
 
+// One wave looks through the bins of a level, from the top down, for the one the mass crosses the goal in: bins[],
+// BITS of them, whose leading bits are `top`.
+template <int BITS>
+__device__ __forceinline__ void find_in_level(SampHist& hist, const mass_t* level, uint32_t top, int lane, bool last) {
+  constexpr int kPer = (1 << BITS) / kWave;
+  mass_t bins[kPer], sum = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    bins[i] = level[(1 << BITS) - 1 - (kPer * lane + i)];
+    sum += bins[i];
+  }
+  const mass_t goal = hist.goal;
+  mass_t at = wave_prefix_mass(sum) - sum;
+  if (at <= goal && goal < at + sum) {  // one lane
+    mass_t in_bin = 0;
+    int bin = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      if (in_bin == 0 && goal < at + bins[i]) {
+        in_bin = bins[i];
+        bin = (1 << BITS) - 1 - (kPer * lane + i);
+      }
+      if (in_bin == 0) at += bins[i];
+    }
+    uint32_t b = (top << BITS) | bin;
+    bool one = true;  // one value in the bin
+    if (!last) {
+      one = hist.least[bin] == hist.most[bin];
+      b = one ? hist.least[bin] : b;
+    }
+    if (one) {
+      hist.n_equal = count_of(goal - at, mantissa(b)) + 1;
+      hist.equal = count_of(in_bin, mantissa(b));
+      hist.thr = b;
+    } else {
+      hist.goal = goal - at;
+      hist.bin = b;
+    }
+  }
+}
+
 // Rows that fit the register file: 16-byte aligned rows of up to 1024 * kSampRegFloats tokens.  Lane t owns the
 // 16-byte chunks t, t + 1024, t + 2048, ... of the row (K "rounds" of 1024 chunks); the row is read once, the
-// exponentials are taken once, and every later pass is compares and adds on registers.  Bound by vector issue on one
-// compute unit per row: the cut by three histogram levels instead of a bisection of 16 to 32 compare-and-add passes
-// with a reduction each took 64 rows of 32,000 fp16 logits from 37.7 to 24.4 us.  Token-id order is
+// exponentials are taken once, and every later pass is compares and adds on registers.  Token-id order is
 // (round, lane, position in the chunk), so the two places that need it -- ranking equal values at the cut and
 // the cumulative sum of the draw -- take one batched reduction over the rounds to find the round in which the
 // count / the sum crosses, and one scan over the lanes inside that round.
+// Bound by vector issue on one compute unit per row and by a chain of ten reductions over the workgroup.  64 rows of
+// 32,000 logits, top-p 0.9, fp16 / fp32: 15.7 / 14.2 us.  It was 24.6 / 58 us with one round's load awaited before the
+// next was requested, reductions through LDS shuffles, the top-p cut always from three levels, equal values counted lane
+// by lane, the uniform number fetched at the draw, and fp32 rows in scratch memory; by bisection alone 37.7 us.  About
+// 31 thousand cycles now: load 5.3, quotients and maximum 3.2, exponentials and coarse bins 9.5, cut 8.2, draw 5.4.
+// FLOATS: tokens a lane holds, 32 or kSampRegFloats: the passes are unrolled over them (rows of up to 32,768 tokens
+// fetch three fifths of the instructions).
 constexpr int kSampRegFloats = 56;
+constexpr int kSampShortFloats = 32;
 
-template <typename E>
+template <typename E, int FLOATS>
 __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArgs a) {
   constexpr int N = 16 / Logit<E>::kBytes;  // tokens per chunk
-  constexpr int K = kSampRegFloats / N;     // chunks per lane
+  constexpr int K = FLOATS / N;             // chunks per lane
   constexpr int SH = key_shift<E>();
   __shared__ SampShared sh;
   __shared__ SampHist hist;
-  __shared__ float fred[K][kSampWaves];
-  __shared__ int ired[K][kSampWaves];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  __shared__ __attribute__((aligned(16))) float fred[K][kSampWaves];
+  __shared__ int ired[K * kSampWaves];
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int64_t row = blockIdx.x;
   const int V = a.V;
   const char* lrow = static_cast<const char*>(a.logits) + row * a.row_stride * Logit<E>::kBytes;
-  float T = a.temperature ? a.temperature[row] : 1.f;
-  float p = a.top_p ? a.top_p[row] : 1.f;
-  if (!(T > 0.f)) {
-    T = 1.f;
-    p = 0.f;
+
+  // the whole row is requested before anything waits for it; chunks that are not whole read the first one instead
+  const int chunks = (V + N - 1) / N, whole = V / N;
+  const int rounds = (chunks + kSampThreads - 1) / kSampThreads;  // rounds that hold tokens; the rest stay zero
+  u32x4 raw[K];
+  if (whole > 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = t + k * kSampThreads;
+      if (k < rounds) raw[k] = ld16(lrow + (int64_t)(c < whole ? c : 0) * 16);
+    }
   }
   if (t == 0) {
     sh.found = INT_MAX;
     sh.found_after = INT_MAX;
     sh.last = -1;
+    hist.thr = 0;
   }
+  reinterpret_cast<u32x4*>(hist.coarse)[t] = u32x4{0, 0, 0, 0};
+  if (t < 1 << kHistFine) {
+    hist.fine[t] = 0;
+    hist.least[t] = 0xffffffffu;
+    hist.most[t] = 0;
+  }
+  hist.last[t] = 0;
+  static_assert(1 << kHistLast == kSampThreads, "one bin of the last level per lane");
+  float T = a.temperature ? a.temperature[row] : 1.f;
+  float p = a.top_p ? a.top_p[row] : 1.f;
+  const float uniform = a.uniform[row];
+  if (!(T > 0.f)) {
+    T = 1.f;
+    p = 0.f;
+  }
+  const bool filter = p < 1.f;
+
   int par = 0;
   auto block_sum = [&](float v) {
     v = group_sum<64>(v);
@@ -361,29 +490,36 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
     return s;
   };
 
-  const bool filter = p < 1.f;
-  if (filter) {
+  auto block_maximum = [&](float v) {
+    v = wave_maximum(v);
+    if (lane == 0) sh.red[par][w] = v;
+    __syncthreads();
+    float s = sh.red[par][0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) hist.coarse[t + i * kSampThreads] = 0;
-    if (t < 2 << kHistFine) hist.fine[t >> kHistFine][t & ((1 << kHistFine) - 1)] = 0;
-  }
+    for (int i = 1; i < kSampWaves; ++i) s = __builtin_elementwise_maximum(s, sh.red[par][i]);
+    par ^= 1;
+    return s;
+  };
 
   float e[K][N];
-  const int chunks = (V + N - 1) / N;
-  const int rounds = (chunks + kSampThreads - 1) / kSampThreads;  // rounds that hold tokens; the rest stay zero
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int c = t + k * kSampThreads;
     if (k >= rounds) {
 #pragma unroll
       for (int j = 0; j < N; ++j) e[k][j] = 0.f;
-    } else if (c < chunks && (c + 1) * N <= V) {
-      Logit<E>::unpack(ld16(lrow + (int64_t)c * 16), e[k]);
-    } else {  // the row's last, partial chunk, and chunks past the row
+      continue;
+    }
+    const int c = t + k * kSampThreads;
+    if (whole > 0) Logit<E>::unpack(raw[k], e[k]);
+    if (k == rounds - 1) {  // the row's last, partial chunk, and places past the row
+      if (c >= whole) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const int i = c * N + j;
-        e[k][j] = i < V ? Logit<E>::load(lrow, i) : -INFINITY;
+        for (int j = 0; j < N; ++j) e[k][j] = -INFINITY;
+        if (c * N < V) {
+#pragma unroll
+          for (int j = 0; j < N - 1; ++j)
+            if (c * N + j < V) e[k][j] = Logit<E>::load(lrow, c * N + j);
+        }
       }
     }
   }
@@ -393,13 +529,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       if (k >= rounds) break;
-      if (by_r) {
-#pragma unroll
-        for (int j = 0; j < N; ++j) e[k][j] = Logit<E>::round(div_by(e[k][j], T, r));
-      } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) e[k][j] = Logit<E>::round(__fdiv_rn(e[k][j], T));
-      }
+      divide<E>(e[k], T, r, by_r);
     }
   }
   float m = -INFINITY;
@@ -407,17 +537,17 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   for (int k = 0; k < K; ++k) {
     if (k >= rounds) break;
 #pragma unroll
-    for (int j = 0; j < N; ++j) m = fmaxf(m, e[k][j]);
+    for (int j = 0; j < N; ++j) m = __builtin_elementwise_maximum(m, e[k][j]);
   }
-  m = group_max<64>(m);
+  m = wave_maximum(m);
   // Adds of a wave to one address are taken one lane after the other, so a row of few distinct values (equal logits, a
-  // high temperature) makes the histograms slow: with all tokens in one coarse bin by about 25 us at 32,000 tokens, with
-  // all of one value by as much again at each finer level.  Every wave compares one token per chunk with lane 0's: the
-  // share in its bin (by distance, half a bin's width) and twice the share of its value.  From one half on the row goes
-  // to the bisection, whose time does not depend on the values.  64 rows of 32,000 fp16 logits, histograms and
-  // bisection: all equal 79.3 and 37.4 us, two values at random 64.1 and 37.4, four 44.9 and 37.4, five 41.2 and 38.6,
-  // normal logits of deviation 0.005 48.5 and 38.5; eight values (share 0.38) take 35.7 us by histograms, normal logits
-  // of deviation 4 25.0 (24.6 without the look).  32-bit logits stay (all equal 108 us against 174: twice the bits).
+  // high temperature) makes the histograms slow.  Every wave compares one token per chunk with lane 0's: the share in its
+  // bin (by distance, half a bin's width) and twice the share of its value.  From one half on the row goes to the
+  // bisection, whose time hardly depends on the values.  64 rows of 32,000 fp16 logits, histograms and bisection: all
+  // equal 120 and 15.4 us, two values at random 69 and 17.7, four 43.2 and 37.3, five 39.3 and 38.9, normal logits of
+  // deviation 0.005 43.4 and 38.3; eight values (share 0.38) 30.9 and 36.9, deviation 0.02 29.3 and 38.7, deviation 4 15.4
+  // and 34 (15.6 with the look).  32-bit logits take the histograms whatever they hold: all equal 99 us against 16, but
+  // from four values on 44 against 50, deviation 4 14.1 against 48.
   constexpr bool kLooks = Logit<E>::kBytes == 2;
   constexpr float kNoMass = 41.5f;  // this far below the maximum a token is no mass (kHistLeast)
   if (kLooks && filter) {
@@ -437,7 +567,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   __syncthreads();
   m = sh.red[par][0];
 #pragma unroll
-  for (int i = 1; i < kSampWaves; ++i) m = fmaxf(m, sh.red[par][i]);
+  for (int i = 1; i < kSampWaves; ++i) m = __builtin_elementwise_maximum(m, sh.red[par][i]);
   bool flat = false;
   if (kLooks && filter) {
     int share = 0;
@@ -446,158 +576,199 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
     flat = 2 * share > kSampThreads * rounds;
   }
   par ^= 1;
-  if (!(m > -INFINITY && m < INFINITY)) m = 0.f;
-  float z = 0.f;
+  const bool finite = m > -INFINITY && m < INFINITY;  // and no NaN in the row
+  const bool by_bins = filter && finite && !flat;
+  if (!finite) {  // the largest number among NaN and infinite logits, 0 where that is infinite
+    m = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) break;
+#pragma unroll
+      for (int j = 0; j < N; ++j) m = fmaxf(m, e[k][j]);
+    }
+    m = group_max<64>(m);
+    if (lane == 0) sh.red[par][w] = m;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSampWaves; ++i) m = fmaxf(m, sh.red[par][i]);
+    par ^= 1;
+    if (!(m > -INFINITY && m < INFINITY)) m = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k >= rounds) break;
+#pragma unroll
+      for (int j = 0; j < N; ++j) e[k][j] = e[k][j] == INFINITY ? 1000.f : e[k][j];  // the same exponential
+    }
+  }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     if (k >= rounds) break;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      e[k][j] = expf(e[k][j] - m);
-      z += e[k][j];
-    }
-  }
-  if (filter && !flat) {
+    for (int j = 0; j < N; ++j) e[k][j] = exp_of(e[k][j] - m);
+    if (!by_bins) continue;
+    // the most likely token has e == 1, every e is in [0, 1]
+    // where all lanes hold the same value, one of them adds for all (rows of 16-bit logits like that are bisected)
+    const float e0 = e[k][0];
+    const bool same =
+        !kLooks && __builtin_amdgcn_ballot_w64(e0 != __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                                                                __builtin_bit_cast(int, e0)))) == 0;
+    if (same) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if (k >= rounds) break;
-      // where all lanes hold the same value, one of them adds for all (rows of 16-bit logits like that are bisected)
-      const float e0 = e[k][0];
-      const bool same =
-          !kLooks && __builtin_amdgcn_ballot_w64(e0 != __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                                                  __builtin_bit_cast(int, e0)))) == 0;
-      if (same) {
+      for (int j = 0; j < N; ++j) {
+        const uint32_t v = __builtin_bit_cast(uint32_t, e[k][j]);
+        const bool all = __builtin_amdgcn_ballot_w64(v != (uint32_t)__builtin_amdgcn_readfirstlane((int)v)) == 0;
+        if (v >= kHistLeast && (!all || lane == 0))
+          atomicAdd(hist_slot(hist.coarse, v), hist_entry(v) << (all ? 6 : 0));
+      }
+    } else {
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-          const uint32_t v = __builtin_bit_cast(uint32_t, e[k][j]);
-          const bool all = __builtin_amdgcn_ballot_w64(v != (uint32_t)__builtin_amdgcn_readfirstlane((int)v)) == 0;
-          if (v >= kHistLeast && (!all || lane == 0))
-            atomicAdd(hist_slot(hist.coarse, v), hist_entry(v) << (all ? 6 : 0));
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-          const uint32_t v = __builtin_bit_cast(uint32_t, e[k][j]);
-          if (v >= kHistLeast) atomicAdd(hist_slot(hist.coarse, v), hist_entry(v));
-        }
+      for (int j = 0; j < N; ++j) {
+        // a token of no mass adds to one of the bins nobody reads, each lane to its own: no branch
+        const float x = e[k][j];
+        const uint32_t v = max(__builtin_bit_cast(uint32_t, x), (uint32_t)(kHistBins + lane) << kHistShift);
+        atomicAdd(hist_slot(hist.coarse, v), hist_entry(v));
       }
     }
   }
-  z = block_sum(z);
 
   if (filter) {  // zero the e of every token that does not survive
     float thr;
     int n_equal = INT_MAX, equal = INT_MAX;  // equal: tokens of value thr, or more
-    // the most likely token has e == 1 and no e is NaN: every e is in [0, 1]
-    if (z >= 1.f && z < INFINITY && !flat) {
+    if (by_bins) {
+      __syncthreads();
       // the value at which the mass of the values from the top down passes the target
-      mass_t four[4], mine = 0;
+      const u32x4 pair = reinterpret_cast<const u32x4*>(hist.coarse)[kSampThreads - 1 - t];
+      mass_t two[2], mine = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int bin = kHistBins - 1 - (4 * t + i);  // from the top down
-        const mass_t sum = hist_mantissas(hist.coarse[bin], bin);
+      for (int i = 0; i < 2; ++i) {
+        const int bin = 2 * kHistBins - 1 - (2 * t + i);  // from the top down
+        const mass_t entry = ((mass_t)pair[3 - 2 * i] << 32) | pair[2 - 2 * i];
+        const mass_t sum = hist_mantissas(entry, bin);
         const int up = mass_shift(bin);
-        four[i] = up >= 0 ? sum << up : up > -64 ? sum >> -up : 0;
-        mine += four[i];
+        two[i] = bin < kHistFirst ? 0 : up >= 0 ? sum << up : sum >> -up;
+        mine += two[i];
       }
-      const mass_t inc = wave_prefix_mass(mine, lane);
+      const mass_t inc = wave_prefix_mass(mine);
       if (lane == kWave - 1) hist.wave_mass[w] = inc;
       __syncthreads();
-      mass_t before = inc - mine, total = 0;
-#pragma unroll
-      for (int i = 0; i < kSampWaves; ++i) {
-        if (i == w) before += total;
-        total += hist.wave_mass[i];
-      }
+      static_assert(kSampWaves == 16, "one row of lanes holds the waves' sums");
+      const mass_t waves = row_prefix_mass(hist.wave_mass[lane & (kSampWaves - 1)]);  // every row of lanes the same
+      const mass_t total = lane_mass(waves, kSampWaves - 1);
+      mass_t before = inc - mine + (w > 0 ? lane_mass(waves, w - 1) : 0);
       const mass_t target = (mass_t)((double)fmaxf(p, 0.f) * (double)total);
       if (before <= target && target < before + mine) {  // one lane of the workgroup
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (before <= target && target < before + four[i]) {
-            const int bin = kHistBins - 1 - (4 * t + i), up = mass_shift(bin);
+        for (int i = 0; i < 2; ++i) {
+          if (before <= target && target < before + two[i]) {
+            const int bin = 2 * kHistBins - 1 - (2 * t + i), up = mass_shift(bin);
             hist.bin = bin;
             hist.goal = up >= 0 ? (target - before) >> up : (target - before) << -up;
           }
-          before += four[i];
+          before += two[i];
         }
       }
       __syncthreads();
-      uint32_t top = hist.bin;  // the leading bits found so far
+      uint32_t top = __builtin_amdgcn_readfirstlane(hist.bin);  // the leading bits found so far
 #pragma unroll
-      for (int level = 0; level < 2; ++level) {
-        const int low = level == 0 ? kHistFine : 0;  // bits below this level's
+      for (int k = 0; k < K; ++k) {
+        if (k >= rounds) break;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const uint32_t b = __builtin_bit_cast(uint32_t, e[k][j]);
+          if (b >> kHistShift == top) {
+            const uint32_t bin = (b >> kHistLast) & ((1 << kHistFine) - 1);
+            atomicAdd(&hist.fine[bin], (mass_t)mantissa(b));
+            atomicMin(&hist.least[bin], b);
+            atomicMax(&hist.most[bin], b);
+          }
+        }
+      }
+      __syncthreads();
+      if (w == 0) find_in_level<kHistFine>(hist, hist.fine, top, lane, false);
+      __syncthreads();
+      if (hist.thr == 0) {  // several values in that bin: its last bits
+        top = __builtin_amdgcn_readfirstlane(hist.bin);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           if (k >= rounds) break;
 #pragma unroll
           for (int j = 0; j < N; ++j) {
             const uint32_t b = __builtin_bit_cast(uint32_t, e[k][j]);
-            if (b >> (low + kHistFine) == top)
-              atomicAdd(&hist.fine[level][(b >> low) & ((1 << kHistFine) - 1)], (mass_t)mantissa(b));
+            if (b >> kHistLast == top) atomicAdd(&hist.last[b & ((1 << kHistLast) - 1)], (mass_t)mantissa(b));
           }
         }
         __syncthreads();
-        if (w == 0) {  // eight bins per lane
-          constexpr int kPer = (1 << kHistFine) / kWave;
-          mass_t bins[kPer], sum = 0;
-#pragma unroll
-          for (int i = 0; i < kPer; ++i) {
-            bins[i] = hist.fine[level][(1 << kHistFine) - 1 - (kPer * lane + i)];
-            sum += bins[i];
-          }
-          const mass_t goal = hist.goal;
-          mass_t at = wave_prefix_mass(sum, lane) - sum;
-          if (at <= goal && goal < at + sum) {
-            mass_t in_bin = 0;
-            int bin = 0;
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-              if (in_bin == 0 && goal < at + bins[i]) {
-                in_bin = bins[i];
-                bin = (1 << kHistFine) - 1 - (kPer * lane + i);
-              }
-              if (in_bin == 0) at += bins[i];
-            }
-            hist.bin = bin;
-            hist.goal = goal - at;
-            if (level == 1) {
-              const uint32_t b = (top << kHistFine) | bin;
-              hist.thr = b;
-              hist.n_equal = (int)((goal - at) / mantissa(b)) + 1;
-              hist.equal = (int)(in_bin / mantissa(b));
-            }
-          }
-        }
+        if (w == 0) find_in_level<kHistLast>(hist, hist.last, top, lane, true);
         __syncthreads();
-        if (level == 0) top = (top << kHistFine) | hist.bin;
       }
       const uint32_t tb = hist.thr;  // a copy: the cast is applied to a plain scalar
       thr = __builtin_bit_cast(float, tb);
       n_equal = hist.n_equal;
       equal = hist.equal;
     } else {  // NaN or infinite logits, few distinct values: bisection over the element type's patterns
+      float z = 0.f, e_lo = INFINITY;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (k >= rounds) break;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          z += e[k][j];
+          e_lo = fminf(e_lo, e[k][j] > 0.f ? e[k][j] : INFINITY);
+        }
+      }
+      z = block_sum(z);
       const float target = fmaxf(p, 0.f) * z;
-      uint32_t lo = to_key<SH>(-INFINITY), hi = to_key<SH>(m);
-      float g_hi = 0.f;
-      while (lo < hi) {  // lo, hi and g are the same in every lane
-        const uint32_t mid = lo + ((hi - lo) >> 1);
-        const float cut = expf(from_key<SH>(mid) - m);
-        float g = 0.f;
+      float g_hi = 0.f, e_hi = 1.f;
+      // the value looked for is one of the row's, from e_lo to e_hi: two cuts halfway between them, each moving one of
+      // them to the nearest value, and a row of one to three values is through (in a row with an infinite maximum the
+      // bits alone decide)
+      e_lo = finite ? -block_maximum(-e_lo) : 0.f;
+      for (int looks = finite ? 2 : 0; looks > 0 && e_lo < e_hi; --looks) {  // the same in every lane
+        const float cut = 0.5f * (e_lo + e_hi);
+        float g = 0.f, above = INFINITY, up_to = 0.f;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           if (k >= rounds) break;
 #pragma unroll
-          for (int j = 0; j < N; ++j) g += e[k][j] > cut ? e[k][j] : 0.f;
+          for (int j = 0; j < N; ++j) {
+            const bool over = e[k][j] > cut;
+            g += over ? e[k][j] : 0.f;
+            above = fminf(above, over ? e[k][j] : INFINITY);
+            up_to = fmaxf(up_to, over ? 0.f : e[k][j]);
+          }
         }
         g = block_sum(g);
         if (g <= target) {
-          hi = mid;
           g_hi = g;
+          e_hi = block_maximum(up_to);
         } else {
-          lo = mid + 1;
+          e_lo = -block_maximum(-above);
         }
       }
-      thr = expf(from_key<SH>(hi) - m);
+      thr = e_hi;
+      if (!(e_lo >= e_hi)) {
+        uint32_t lo = to_key<SH>(-INFINITY), hi = to_key<SH>(m);
+        g_hi = 0.f;
+        while (lo < hi) {  // lo, hi and g are the same in every lane
+          const uint32_t mid = lo + ((hi - lo) >> 1);
+          const float cut = expf(from_key<SH>(mid) - m);
+          float g = 0.f;
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            if (k >= rounds) break;
+#pragma unroll
+            for (int j = 0; j < N; ++j) g += e[k][j] > cut ? e[k][j] : 0.f;
+          }
+          g = block_sum(g);
+          if (g <= target) {
+            hi = mid;
+            g_hi = g;
+          } else {
+            lo = mid + 1;
+          }
+        }
+        thr = expf(from_key<SH>(hi) - m);
+      }
       if (thr > 0.f) {
         const float r = floorf((target - g_hi) / thr);
         n_equal = r >= 2.0e9f ? INT_MAX : max((int)r + 1, 1);
@@ -611,67 +782,54 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
         for (int j = 0; j < N; ++j) e[k][j] = e[k][j] >= thr ? e[k][j] : 0.f;
       }
     } else {
-    // tokens equal to thr, per round; they survive in id order until n_equal of them have
-    int cnt[K], tot[K];
+      // tokens equal to thr survive in id order until n_equal of them have: counted per round and wave, which is the
+      // order of the ids, then ranked inside the (round, wave) in which the count passes n_equal
+      int cnt[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      cnt[k] = 0;
-      if (k >= rounds) continue;
+      for (int k = 0; k < K; ++k) {
+        cnt[k] = 0;
+        if (k < rounds) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) cnt[k] += e[k][j] == thr ? 1 : 0;
-      int v = cnt[k];
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
-      if (lane == 0) ired[k][w] = v;
-    }
-    __syncthreads();
-    int kc = K, before_kc = 0, run = 0;  // the round in which the count passes n_equal (K: it never does)
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      tot[k] = 0;
-      if (k < rounds) {
-#pragma unroll
-        for (int i = 0; i < kSampWaves; ++i) tot[k] += ired[k][i];
+          for (int j = 0; j < N; ++j) cnt[k] += __builtin_popcountll(__builtin_amdgcn_ballot_w64(e[k][j] == thr));
+        }
+        if (lane == 0) ired[k * kSampWaves + w] = cnt[k];
       }
-      if (kc == K && run + tot[k] > n_equal) {
-        kc = k;
-        before_kc = run;
-      }
-      run += tot[k];
-    }
-    int rank_kc = 0;  // rank of this lane's first equal token of round kc
-    if (kc < K) {     // same in every lane
-      int mine = 0;
-#pragma unroll
-      for (int k = 0; k < K; ++k) mine = k == kc ? cnt[k] : mine;
-      int inc = mine;
-#pragma unroll
-      for (int d = 1; d < kWave; d <<= 1) {
-        const int up = __shfl_up(inc, d, kWave);
-        if (lane >= d) inc += up;
-      }
-      if (lane == kWave - 1) sh.ipart[w] = inc;
       __syncthreads();
-      rank_kc = before_kc + inc - mine;
-      for (int i = 0; i < w; ++i) rank_kc += sh.ipart[i];
-    }
+      constexpr int kPerWave = kWave / kSampWaves;  // rounds whose counts the lanes of a wave hold at once
+      int carry = 0, upto = 0;                      // tokens equal to thr in the rounds before; up to a lane's entry
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if (k >= rounds) break;
-      int rank = rank_kc;
+      for (int k = 0; k < K; ++k) {
+        if (k % kPerWave == 0) {
+          const int at = k * kSampWaves + lane;
+          upto = carry + wave_prefix_sum(at < K * kSampWaves ? ired[at] : 0);
+          carry = __builtin_amdgcn_readlane(upto, kWave - 1);
+        }
+        if (k >= rounds) continue;
+        const int before = __builtin_amdgcn_readlane(upto, (k % kPerWave) * kSampWaves + w) - cnt[k];
+        if (before + cnt[k] <= n_equal) {  // same in every lane of the wave
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const float v = e[k][j];
-        bool keep = v > thr;
-        if (v == thr) keep = k < kc || (k == kc && rank++ < n_equal);
-        e[k][j] = keep ? v : 0.f;
+          for (int j = 0; j < N; ++j) e[k][j] = e[k][j] >= thr ? e[k][j] : 0.f;
+        } else {
+          int rank = before;  // of this lane's first equal token: the equal tokens of the lanes before
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const uint64_t eq = __builtin_amdgcn_ballot_w64(e[k][j] == thr);
+            rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(eq >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)eq, rank));
+          }
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const float v = e[k][j];
+            bool keep = v > thr;
+            if (v == thr) keep = rank++ < n_equal;
+            e[k][j] = keep ? v : 0.f;
+          }
+        }
       }
-    }
     }
   }
 
   // the draw: first token, in id order, at which the running sum of e passes uniform * (sum of e)
-  float cs[K], tot[K];
+  float cs[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     cs[k] = 0.f;
@@ -682,17 +840,18 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
     if (lane == 0) fred[k][w] = v;
   }
   __syncthreads();
-  float kept = 0.f;
+  float round_sum = 0.f;  // lane k: of round k
+  if (lane < rounds) {
+#pragma unroll
+    for (int i = 0; i < kSampWaves; ++i) round_sum += fred[lane][i];
+  }
+  float tot[K], kept = 0.f;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    tot[k] = 0.f;
-    if (k < rounds) {
-#pragma unroll
-      for (int i = 0; i < kSampWaves; ++i) tot[k] += fred[k][i];
-    }
+    tot[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, round_sum), k));
     kept += tot[k];
   }
-  const float goal = a.uniform[row] * kept;
+  const float goal = uniform * kept;
   int kd = K;  // the round in which the running sum passes the goal
   float before_kd = 0.f, run = 0.f;
 #pragma unroll
@@ -715,7 +874,8 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   if (lane == kWave - 1) sh.fpart[w] = finc;
   __syncthreads();
   float running = before_kd;
-  for (int i = 0; i < w; ++i) running += sh.fpart[i];
+#pragma unroll
+  for (int i = 0; i < kSampWaves - 1; ++i) running += i < w ? sh.fpart[i] : 0.f;
   running += finc - mine;
   int found = INT_MAX;
 #pragma unroll
@@ -757,8 +917,10 @@ template <typename E>
 static int launch_sample(const SampArgs& a, int64_t rows, hipStream_t st) {
   dim3 grid((unsigned)rows), block(kSampThreads);
   const bool rows_aligned = aligned16(a.logits) && (a.row_stride * Logit<E>::kBytes) % 16 == 0;
-  if (rows_aligned && a.V <= kSampThreads * kSampRegFloats) {
-    hipLaunchKernelGGL((sample_rows_kernel<E>), grid, block, 0, st, a);
+  if (rows_aligned && a.V <= kSampThreads * kSampShortFloats) {
+    hipLaunchKernelGGL((sample_rows_kernel<E, kSampShortFloats>), grid, block, 0, st, a);
+  } else if (rows_aligned && a.V <= kSampThreads * kSampRegFloats) {
+    hipLaunchKernelGGL((sample_rows_kernel<E, kSampRegFloats>), grid, block, 0, st, a);
   } else if (a.V <= kSampLdsFloats) {
     const size_t lds = (size_t)a.V * sizeof(float);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&sample_top_p_kernel<E, true>),

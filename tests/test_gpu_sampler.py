@@ -303,3 +303,21 @@ def test_the_time_does_not_hang_on_equal_values(dtype):
     coins = torch.rand(B, V, generator=g, device="cuda")
     for rows in (torch.zeros(B, V, device="cuda"), (coins < 0.5).float() * 0.5, (coins < 0.1).float() * 3):
         assert best(rows) < 2.2 * normal
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("V", [5, 8191, 8192, 8193, 32761, 32768, 32769, 57337])
+def test_row_lengths_around_the_rounds_and_forms_of_the_register_kernel(dtype, V):
+    """No whole chunk, a last chunk of one token and of all but one, a round that is full and one that holds a single
+    chunk, the longest row of the 32-token form and the shortest of the other; rows start on the 16-byte grid whatever
+    their length.  Values in steps of 1/4 (several equal ones at every cut, ranked over rounds and waves), and values so
+    close that the finer bin in question holds several, so that its last bits decide."""
+    B = 6
+    pad = -V % 8 + 8
+    x, temps, tops, u = _case(V, B, V, dtype, quantum=0.25)
+    _check(x, temps, tops, u, dtype, min_compared=0.5, stride_pad=pad)
+    g = torch.Generator().manual_seed(V)
+    # in steps of 2^-22: fp32 exponentials just under 1 lie 2^-24 apart and are right to one such step, so values closer
+    # than 2^-23 may share one, and the kernel ranks equal exponentials by id
+    close = ((torch.rand(B, V, generator=g) * 1024).floor() * 2.0 ** -22).to(DT[dtype])
+    _check(close, torch.ones(B), torch.tensor([0.9003, 0.3007, 0.6002] * 2), u, dtype, min_compared=0.3, stride_pad=pad)
