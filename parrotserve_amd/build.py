@@ -3,7 +3,8 @@
 Run ``python -m parrotserve_amd.build`` or call ``build()``; the shared library
 lands next to the sources' package (parrotserve_amd/libparrot_hip.so) so it
 travels with the tree.  ``python -m parrotserve_amd.build --timeline`` also links the
-profiling variant (libparrot_hip_timeline.so, what ``bench.py --timeline`` loads).
+profiling variant (libparrot_hip_timeline.so, what ``bench.py --timeline`` loads).  The C++ form of the wrappers'
+plain calls (csrc/host_calls.cpp, no device code) is built against torch by g++ into ``_host.so`` beside it.
 """
 from __future__ import annotations
 
@@ -17,6 +18,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libparrot_hip.so")
 # profiling variant: the same sources with the fused decode kernel's timeline marks switched on (csrc/timeline.hpp)
 TIMELINE_LIB_PATH = os.path.join(PKG_DIR, "libparrot_hip_timeline.so")
+HOST_LIB_PATH = os.path.join(PKG_DIR, "_host.so")
 SOURCES = ["move_tokens.hip", "gather_blocked.hip", "norm_rope.hip", "fused.hip", "sampler.hip", "tables.hip", "decode.hip", "prefix_mfma.hip", "attention_api.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -51,12 +53,31 @@ def _compile(src: str, obj_dir: str, timeline: bool = False) -> str:
     return obj
 
 
+def _build_host() -> None:
+    """csrc/host_calls.cpp, a CPython module over torch's C++ interface."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"), "-isystem",
+           os.path.join(root, "include", "torch", "csrc", "api", "include"), os.path.join(CSRC, "host_calls.cpp"),
+           "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", HOST_LIB_PATH]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"the build of host_calls.cpp failed:\n{r.stdout}\n{r.stderr}")
+
+
 def build(verbose: bool = True, timeline: bool = False) -> str:
     """Compile and link the product library; ``timeline=True`` also links the profiling variant."""
     obj_dir = os.path.join(PKG_DIR, "build")
     os.makedirs(obj_dir, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(lambda s: _compile(s, obj_dir), SOURCES))
+        host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

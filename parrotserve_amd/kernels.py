@@ -138,6 +138,25 @@ def _workspace(nbytes: int, device: torch.device, least: Optional[int] = None) -
     return buf
 
 
+_host = None  # the C++ form of the plain calls (csrc/host_calls.cpp), bound at the first call
+
+
+def _load_host():
+    """Loads ``_host.so`` and gives it the library's addresses and what this module keeps.  Its functions return
+    ``None`` for a call that is not of the plain form; the body behind such a call here decides about it."""
+    global _host
+    from . import _host as host
+
+    lib = _lib.load()
+    host.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _lib.SIGNATURES},
+              dict(check=check, raw_stream=_raw_stream or (lambda device: torch.cuda.current_stream().cuda_stream),
+                   raw_device=_raw_device, capturing=torch.cuda.is_current_stream_capturing, workspaces=_workspaces,
+                   workspace=_workspace, decode_workspace_bytes=_decode_workspace_bytes, decode_tables=DecodeTables,
+                   prefill_tables=PrefillTables))
+    _host = host
+    return host
+
+
 # --------------------------------------------------------------------------- #
 # token move / KV append
 # --------------------------------------------------------------------------- #
@@ -243,6 +262,9 @@ def vllm_reshape_and_cache(key_to_cache, value_to_cache, key_cache, value_cache,
 # RMSNorm / RoPE
 # --------------------------------------------------------------------------- #
 def _rms(x, weight, eps, round_first, name):
+    out = (_host or _load_host()).rms_norm(x, weight, eps, round_first, name)
+    if out is not None:
+        return out
     _require_gpu(x, weight)
     assert x.shape[-1] == weight.shape[0], "weight size mismatch"
     assert x.dtype == weight.dtype, "weight dtype mismatch"
@@ -275,6 +297,9 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Te
                        round_before_weight: bool = True) -> torch.Tensor:
     """``residual += x`` in place, returns ``RMSNorm(residual) * weight`` (one launch for the residual add of
     the decoder layer and the norm that follows it)."""
+    out = (_host or _load_host()).add_rms_norm(x, residual, weight, eps, round_before_weight)
+    if out is not None:
+        return out
     _require_gpu(x, residual, weight)
     n = x.shape[-1]
     assert x.shape == residual.shape and weight.shape == (n,) and x.dtype == residual.dtype == weight.dtype
@@ -292,6 +317,10 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Te
 
 def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``silu(gate) * up`` in one launch; ``gate`` / ``up`` may be column slices of one fused projection."""
+    if out is None:
+        done = (_host or _load_host()).silu_mul(gate, up)
+        if done is not None:
+            return done
     _require_gpu(gate, up)
     d = gate.shape[-1]
     assert gate.shape == up.shape and gate.dtype == up.dtype
@@ -317,6 +346,9 @@ def sample_top_p(logits: torch.Tensor, temperature: Optional[torch.Tensor], top_
     found from histograms (long or unaligned rows, rows of few distinct values: by bisection) instead of two sorts and
     the draw taken from ``uniform [B]`` (float32 in [0, 1), from the caller's generator) by inverse CDF over ascending
     token ids.  ``temperature`` / ``top_p``: float32 ``[B]`` on the device, or ``None`` for 1.  Returns int64 ``[B]``."""
+    done = (_host or _load_host()).sample_top_p(logits, temperature, top_p, uniform)
+    if done is not None:
+        return done
     _require_gpu(logits, temperature, top_p, uniform)
     assert logits.dim() == 2 and logits.stride(1) == 1
     B, V = logits.shape
@@ -365,6 +397,9 @@ def rope_and_cache(positions, query, key, value, cos_sin_cache, head_size, key_c
     in one launch: q and k rotated in place, rotated k rows and v rows written to their slots.
     ``key_in_place=False``: the caller reads K from the cache from here on, so ``key`` is not written back
     (its contents afterwards are unspecified) and the pass is a quarter shorter."""
+    if (_host or _load_host()).rope_append(positions, query, key, value, cos_sin_cache, head_size, key_cache, value_cache,
+                                           slot_mapping, key_in_place):
+        return
     _require_gpu(query, key, value, key_cache, value_cache, cos_sin_cache, positions, slot_mapping)
     assert positions.dtype == torch.int64 and positions.dim() == 1
     T = positions.shape[0]
@@ -692,6 +727,10 @@ def decode_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: 
     kernels (``ph_decode_attention_timed``).  ``head_mapping`` (int32 device ``[H]``): query head h reads KV head
     ``head_mapping[h]`` of caches ``[slots, H_kv, D]``; ``kv_group = G > 0`` states that it is ``h // G``
     (``ph_decode_attention_gqa``)."""
+    if out is None and events6 is None:
+        done = (_host or _load_host()).decode_attention(query, key_cache, value_cache, tables, scale, head_mapping, kv_group)
+        if done is not None:
+            return done
     _require_gpu(query, key_cache, value_cache)
     assert query.dim() == 3 and key_cache.dim() == 3 and value_cache.shape == key_cache.shape
     B, H, D = query.shape
@@ -962,6 +1001,10 @@ def prefill_attention(query, key_cache, value_cache, tables: PrefillTables, scal
     ancestors' and its own KV read through the slot table -- the op the
     reference assembles from a gather plus xformers' block-diagonal FMHA
     (parrot/engine/builtin/attn_func.py:635-674)."""
+    if out is None:
+        done = (_host or _load_host()).prefill_attention(query, key_cache, value_cache, tables, scale)
+        if done is not None:
+            return done
     _require_gpu(query, key_cache, value_cache)
     T, H, D = query.shape
     assert T == tables.num_tokens
