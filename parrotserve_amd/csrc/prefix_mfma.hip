@@ -30,6 +30,9 @@
 
 namespace ph {
 
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+
 template <typename E>
 struct Mfma32;
 template <>
@@ -44,6 +47,28 @@ struct Mfma32<BF16> {
   static __device__ __forceinline__ float16_t run(u32x4 a, u32x4 b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
                                                    c, 0, 0, 0);
+  }
+};
+
+// c[0..3] + the sum of a lane's own four elements, in every element of c: the 4 x 4 x 4 form multiplies sixteen blocks
+// of four lanes each, and with a first operand of ones every row of a result column is that column's sum.  It runs on the
+// matrix pipe (9 cycles), where a v_dot2 behind a matrix instruction costs 18 issue cycles: the loop below with v_dot2
+// in its place takes 681 instead of 666 us for a Fill of 8192 tokens at 40 heads.
+template <typename E>
+struct LaneSum4;
+template <>
+struct LaneSum4<F16> {
+  static __device__ __forceinline__ float4_t run(uint32_t lo, uint32_t hi, float4_t c) {
+    const u32x2 ones = {Elem<F16>::kOnes, Elem<F16>::kOnes}, b = {lo, hi};
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, ones), __builtin_bit_cast(half4_t, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct LaneSum4<BF16> {
+  static __device__ __forceinline__ float4_t run(uint32_t lo, uint32_t hi, float4_t c) {
+    const u32x2 ones = {Elem<BF16>::kOnes, Elem<BF16>::kOnes}, b = {lo, hi};
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(short4_t, ones), __builtin_bit_cast(short4_t, b), c,
+                                                  0, 0, 0);
   }
 };
 
@@ -77,7 +102,6 @@ __device__ __forceinline__ uint32_t lds_addr_of(const char* p) {
 
 __device__ __forceinline__ u32x4 lds_ld16(const char* p) { return *reinterpret_cast<const u32x4*>(p); }
 
-typedef short short4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x2 lds_tr16(const char* p) {
   const short4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (short4_t __attribute__((address_space(3)))*)(const_cast<char*>(p)));
@@ -511,7 +535,8 @@ struct NoMid {
   __device__ __forceinline__ void operator()() const {}
 };
 
-template <typename E, bool CAUSAL, int TQ, typename Mid = NoMid, int SUB = 1, bool HALF = false, bool PRESC = false>
+template <typename E, bool CAUSAL, int TQ, typename Mid = NoMid, int SUB = 1, bool HALF = false, bool PRESC = false,
+          bool SUMS = false>
 __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* __restrict__ kc,
                                            const uint16_t* __restrict__ vc, int64_t row_stride, int head,
                                            float scale_log2e, char* smem, float16_t (&ofold)[4 / TQ], float& mfin,
@@ -543,12 +568,26 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   constexpr bool PREFETCH = !CAUSAL && A == 1 && STEP * TQ == 128;
   constexpr int kPfSteps = 2;
   constexpr float kSlack = 8.f;
+  // SUMS: no maximum is taken in an ordinary step.  The exponentials are taken against the reference as it stands, and
+  // their sums, which the denominator needs anyway, say whether it still serves: up to kSumLimit no single one can have
+  // left the range of its 16-bit type (a larger exponential has the same relative rounding, a smaller one is further
+  // from the subnormals than under its own maximum).  Only beyond it, and in steps that mask or have no reference yet,
+  // the scores are multiplied anew from LDS and the maximum is taken.  That leaves the matrix instructions of one
+  // sub-tile's scores to run under the exponentials of the other's, and P.V of the one under the exponentials of the
+  // other (the maximum of both stood between them before).
+  // 8192 tokens, 40 heads: 684 -> 666 us, 4 % fewer cycles at a clock 1 % lower; 16 chunks over 2048 tokens 545 -> 536.
+  // (256 requests over 8192 tokens 81.0 -> 80.9: the decode kernels, whose units are short, keep the maximum.)  Measured against this form and not kept: P.V behind both sub-tiles'
+  // exponentials (740), the two waves of a SIMD half a step apart with a barrier every half step (748 against 720 before
+  // and 702), one barrier for two steps (679 against 664).
+  static_assert(!SUMS || (PRESC && SUB == 2 && TQ == 1), "the sums stand for a maximum in the pre-scaled 256-query form");
+  constexpr uint32_t kSumLimitBits = 0x45800000u;  // 2^12, where a lane sums sixteen exponentials
   // HALF: a 64-wide head as half wk.pair_half (0 / 1) of a head pair -- only that half's two 32-dim blocks of the
   // output are wanted, so only they are multiplied (accumulators 0 and 1 stand for blocks 2 half, 2 half + 1)
   static_assert(!HALF || TQ == 1, "the half-output form has no fold across token groups");
   constexpr int NDBV = HALF ? 2 : 4;
   float16_t oacc[4];
   float m = -INFINITY, lsum = 0.f, mtrue = -INFINITY;
+  bool seeded = false;  // SUMS: every lane has an exponent reference
   // (the thread's number anew for every tile: what follows from it would be kept, and spilled, across the units of a
   // workgroup that walks several.  The 256-query tile then spilled 184 bytes a lane, reloads in the tile loop among
   // them: 256 requests over 8192 tokens 101 us against 79.9, both with the query rows through LDS.)
@@ -774,9 +813,7 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
       }
     }
     if (it >= my_iters || tb > wave_last) continue;           // wave-uniform
-    float16_t sacc[SUB];
-#pragma unroll
-    for (int sb = 0; sb < SUB; ++sb) {
+    auto scores = [&](int sb) {
       const int off = stage * SBYTES + sb * kStage;
       const int shi = NHI == 2 ? off >> 16 : 0, slo = off & 65535;
       u32x4 ka[8];
@@ -784,28 +821,150 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
       for (int s = 0; s < 8; ++s) ka[s] = lds_ld16_a(kaddr[shi][s] + slo);
       if (SUB == 1) __builtin_amdgcn_sched_barrier(0);
       const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      sacc[sb] = Mfma32<E>::run(ka[0], qop[0], PRESC ? cinit : zero);
+      float16_t r = Mfma32<E>::run(ka[0], qop[0], PRESC ? cinit : zero);
 #pragma unroll
-      for (int s = 1; s < 8; ++s) sacc[sb] = Mfma32<E>::run(ka[s], qop[s], sacc[sb]);
-    }
+      for (int s = 1; s < 8; ++s) r = Mfma32<E>::run(ka[s], qop[s], r);
+      return r;
+    };
+    float16_t sacc[SUB];
+#pragma unroll
+    for (int sb = 0; sb < SUB; ++sb) sacc[sb] = scores(sb);
     // A operand of O^T += V^T P^T (row = dim 32db + ql, contraction = the 8 tokens of (h, u)): two
     // transposing reads, tokens 16u + 4h + {0..3} and 16u + 8 + 4h + {0..3}
     u32x4 va[SUB][4][2];
+    auto read_v = [&]() {
 #pragma unroll
-    for (int sb = 0; sb < SUB; ++sb) {
-      const int off = stage * SBYTES + sb * kStage;
-      const int shi = NHI == 2 ? off >> 16 : 0, slo = off & 65535;
+      for (int sb = 0; sb < SUB; ++sb) {
+        const int off = stage * SBYTES + sb * kStage;
+        const int shi = NHI == 2 ? off >> 16 : 0, slo = off & 65535;
+#pragma unroll
+        for (int db = 0; db < NDBV; ++db)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const u32x2 lo = lds_tr16_a(vaddr[shi][db] + slo + (16 * u) * 256);
+            const u32x2 hi = lds_tr16_a(vaddr[shi][db] + slo + (16 * u + 8) * 256);
+            va[sb][db][u] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+          }
+      }
+    };
+    if (!SUMS) read_v();
+    if (SUB == 1) __builtin_amdgcn_sched_barrier(0);
+
+    if constexpr (SUMS) {
+      const bool full = tb + STEP <= s1 && (!CAUSAL || tb + STEP - 1 <= wk.causal_off + 32 * qb);
+      u32x4 pop[2][2];
+      auto exponentials = [&](int sb, const float16_t& s) {
+        float4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            pop[sb][u][e] = pack2<E>(__builtin_amdgcn_exp2f(s[8 * u + 2 * e]), __builtin_amdgcn_exp2f(s[8 * u + 2 * e + 1]));
+          sum[0] = LaneSum4<E>::run(pop[sb][u][0], pop[sb][u][1], sum[0]);
+          sum[1] = LaneSum4<E>::run(pop[sb][u][2], pop[sb][u][3], sum[1]);
+        }
+        return sum[0][0] + sum[1][0];
+      };
+      // sub-tiles first .. 1 by their maximum: tokens out of sight masked, the exponent reference moved where the scores
+      // have outgrown it (the scores in sacc and the sums so far follow)
+      auto settle = [&](int first) {
+        if (!full) {
+          const int tmax = CAUSAL ? min(s1 - 1, wk.causal_off + 32 * qb + ql) : s1 - 1;  // last visible token
+#pragma unroll
+          for (int sb = first; sb < 2; ++sb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const int t = kTile * sb + 8 * (r >> 2) + 4 * h + (r & 3);
+              sacc[sb][r] = (tb + t <= tmax) ? sacc[sb][r] : -INFINITY;
+            }
+        }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int sb = first; sb < 2; ++sb)
+#pragma unroll
+          for (int r = 0; r < 16; r += 4)
+            mloc = fmaxf(mloc, fmaxf(fmaxf(sacc[sb][r], sacc[sb][r + 1]), fmaxf(sacc[sb][r + 2], sacc[sb][r + 3])));
+        const bool had = m != -INFINITY;
+        mloc = half_swap_max(mloc) + (had ? m : 0.f);  // the scores are relative to the reference so far
+        const bool move = mloc > m + kSlack;
+        const float mnew = move ? mloc : m;
+        const float mref = (mnew == -INFINITY) ? 0.f : mnew;
+        const float alpha = (move && had) ? __builtin_amdgcn_exp2f(m - mref) : 1.f;
+        const float delta = mref - (had ? m : 0.f);  // 0 on the lanes whose reference stays
+#pragma unroll
+        for (int sb = first; sb < 2; ++sb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sacc[sb][r] -= delta;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) cinit[r] = -mref;
+        m = mnew;
+        lsum *= alpha;
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+          // wait states cover the matrix results being read by the vector ALU and the rewritten registers feeding the
+          // next C operand
+          asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+          for (int db = 0; db < NDBV; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) asm volatile("v_mul_f32 %0, %0, %1" : "+v"(oacc[db][r]) : "v"(alpha));
+          asm volatile("s_nop 7" ::: "memory");
+        }
+      };
+      auto beyond = [&](float s) {  // compared as bits: a NaN, whatever its sign, is beyond the limit too
+        return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, s) > kSumLimitBits) != 0;
+      };
+      // under the scores of sub-tile 1 (its matrix instructions one to two exponentials): the order is pinned, left alone
+      // the scheduler groups them by kind (1 % slower)
+      float ps = exponentials(0, sacc[0]);
+      __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+        __builtin_amdgcn_sched_group_barrier(0x400, 2, 1);
+        __builtin_amdgcn_sched_group_barrier(0x002, 1, 1);
+      }
+      bool settled = false;
+      if (!full || !seeded || beyond(ps)) {
+        asm volatile("" ::: "memory");  // K is read again, not kept
+        sacc[0] = scores(0);
+        settle(0);
+        seeded = __builtin_amdgcn_ballot_w64(m == -INFINITY) == 0;
+        settled = true;
+        ps = exponentials(0, sacc[0]);
+      }
+      lsum += ps;
+      read_v();
 #pragma unroll
       for (int db = 0; db < NDBV; ++db)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const u32x2 lo = lds_tr16_a(vaddr[shi][db] + slo + (16 * u) * 256);
-          const u32x2 hi = lds_tr16_a(vaddr[shi][db] + slo + (16 * u + 8) * 256);
-          va[sb][db][u] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-        }
+        for (int u = 0; u < 2; ++u) oacc[db] = Mfma32<E>::run(va[0][db][u], pop[0][u], oacc[db]);
+      ps = exponentials(1, sacc[1]);  // under P.V of sub-tile 0
+      __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+      }
+      if (!settled && beyond(ps)) {
+        asm volatile("" ::: "memory");  // K is read again, not kept
+        sacc[1] = scores(1);
+        settle(1);
+        ps = exponentials(1, sacc[1]);
+      }
+      lsum += ps;
+#pragma unroll
+      for (int db = 0; db < NDBV; ++db)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) oacc[db] = Mfma32<E>::run(va[1][db][u], pop[1][u], oacc[db]);
+      continue;
     }
-    if (SUB == 1) __builtin_amdgcn_sched_barrier(0);
-
     const bool full = tb + STEP <= s1 && (!CAUSAL || tb + STEP - 1 <= wk.causal_off + 32 * qb);
     float x[SUB][16];
     if (full) {
@@ -884,6 +1043,7 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   }
 
   PH_TL(8);
+  if (SUMS) mtrue = m;  // any reference serves a part's (m, l), and the true maximum is not known
   if constexpr (TQ == 1) {
     // one token group: nothing to fold across waves
     const float Lall = lsum + __shfl_xor(lsum, 32, kWave);
@@ -1204,7 +1364,7 @@ __global__ __launch_bounds__(64) void prefill_tiles_kernel(const int32_t* q_cu, 
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
 // SPLIT: the tile's visible tokens are cut into a.n_splits runs, this workgroup takes run `split` and writes an
 // (O, m, l) part for fold_parts_kernel instead of the output row.
-template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
+template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false, bool SUMS = false>
 __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const PrefillTile& pt, int split, char* smem) {
   constexpr int QB = 8 / TQ, NDB = 4 / TQ, QT = 32 * QB;
   // 64-wide heads: workgroup x is head x = half (x & 1) of pair x >> 1, whose K/V rows are one 128-wide row
@@ -1244,7 +1404,8 @@ __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const Prefil
   float16_t of[NDB];
   float m, l;
   // the prefill loop is bound by instruction issue: the pre-scaled query saves it one multiply-add per score
-  attn_tile8<E, true, TQ, NoMid, SUB, HALF, true>(wk, a.kc, a.vc, a.row_stride, head, a.scale_log2e, smem, of, m, l);
+  attn_tile8<E, true, TQ, NoMid, SUB, HALF, true, SUMS>(wk, a.kc, a.vc, a.row_stride, head, a.scale_log2e, smem, of, m,
+                                                        l);
   if (q < nq) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const int64_t pr = SPLIT ? ((int64_t)split * a.num_tokens + cq0 + q0 + q) * a.H + blockIdx.x : 0;
@@ -1284,14 +1445,14 @@ __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const Prefil
 // covers the tile rows from a.tile_row0 on (more rows than a grid's y extent holds take several launches; a loop
 // over rows inside the kernel cost the common single-launch case 6 %), grid.z the splits
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
-template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
+template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false, bool SUMS = false>
 __global__ __launch_bounds__(512) void prefill_mfma8_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   PH_TL(0);
   if ((int)blockIdx.x >= a.H) return;
   PrefillTile pt;
   if (!find_prefill_tile(a, a.tile_row0 + (int)blockIdx.y, 32 * (8 / TQ), pt)) return;
-  prefill_tile8<E, TQ, SUB, HALF, SPLIT>(a, pt, blockIdx.z, smem);
+  prefill_tile8<E, TQ, SUB, HALF, SPLIT, SUMS>(a, pt, blockIdx.z, smem);
   PH_TL(11);
 }
 
@@ -1329,7 +1490,7 @@ static int launch_prefix_t(const PrefixArgs& a, int num_groups, int max_group_re
 
 constexpr int64_t kMaxGridY = 65535;  // grid extent in y and z
 
-template <typename E, int TQ, int SUB, bool HALF, bool SPLIT>
+template <typename E, int TQ, int SUB, bool HALF, bool SPLIT, bool SUMS = false>
 static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
   constexpr int QT = 32 * (8 / TQ);  // queries per workgroup tile
   if (a.tile_cu) {
@@ -1337,7 +1498,7 @@ static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
     const int rc = launch_status();
     if (rc != PH_OK) return rc;
   }
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>),
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT, SUMS>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, kTile8Lds);
   const int hx = (a.H + 7) / 8 * 8;  // keeps head == linear id mod 8 for every tile row
   const int64_t max_tiles = (a.num_tokens - a.num_chunks) / QT + a.num_chunks;  // >= sum of ceil(n_c / QT), n_c >= 1
@@ -1345,7 +1506,7 @@ static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
     PrefillArgs part = a;
     part.tile_row0 = (int)row0;
     const int64_t rows = max_tiles - row0 < kMaxGridY ? max_tiles - row0 : kMaxGridY;
-    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>), dim3(hx, (unsigned)rows, SPLIT ? a.n_splits : 1),
+    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT, SUMS>), dim3(hx, (unsigned)rows, SPLIT ? a.n_splits : 1),
                        dim3(512), kTile8Lds, st, part);
   }
   return launch_status();
@@ -1360,6 +1521,14 @@ static int launch_prefill_sq(const PrefillArgs& a, hipStream_t st) {
 template <typename E>
 static int launch_prefill_t(const PrefillArgs& a, int tile_q, hipStream_t st) {
   if (tile_q == 256 && a.pair) return launch_prefill_sq<E, 1, 2, true>(a, st);
+  // The first step of a tile and those on its diagonal multiply their scores twice in the form without maxima, so tiles of
+  // few steps keep the other one.  In us, without / with, by the tokens a query sees on average: 3 chunks of 600 over 40
+  // (340) 39.7 / 41.2; 2 of 200 to 740 (240) 22.9 / 23.5; 4 of 400 to 1200 over 776 (1180) 123 / 127; 16 of 400 to 600
+  // over 1000 (1250) 286 / 290; 13 of 200 to 1900 over 989 (1510) 502 / 498; 16 of 64 to 1024 over 2048 (2340) 545 / 535;
+  // one of 8000 (4000) 679 / 655.
+  constexpr int kLongContext = 2048;
+  if (tile_q == 256 && a.n_splits <= 1 && a.mean_visible >= kLongContext)
+    return launch_prefill_tq<E, 1, 2, false, false, true>(a, st);
   if (tile_q == 256) return launch_prefill_sq<E, 1, 2>(a, st);  // 64-token steps (measured 4 % faster)
   if (tile_q == 128) return launch_prefill_sq<E, 2, 1>(a, st);
   return launch_prefill_sq<E, 4, 1>(a, st);

@@ -416,3 +416,63 @@ def test_prefill_in_parts_replays_from_a_captured_graph(dev, warm):
         if parts > 1:
             assert torch.equal(out, eager), f"replay {rep} differs from the eager result"
         torch.testing.assert_close(out.float(), eager.float(), **TOL[torch.bfloat16])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rises", [
+    {0: 0.0},                                                # one level throughout
+    {0: 0.0, 64: 13.0, 128: 26.0, 192: 39.0},                # past the limit at every step, in its first 32 tokens
+    {0: 0.0, 96: 13.0, 160: 26.0, 288: 39.0},                # in its second 32 tokens
+    {0: 0.0, 64: 11.0, 96: 13.5, 128: 9.0, 353: 25.0},       # within the limit, then past it; a single later token
+    {0: -200.0, 65: 200.0, 66: 0.0},                         # beyond what an fp32 exponential holds
+    {0: 40.0, 32: 0.0, 320: -90.0},                          # falling: the reference stays
+])
+def test_prefill_scores_that_outgrow_the_exponent_reference(dev, rises, dtype):
+    """256-query tiles over scores whose level (as a power of two) changes at the given tokens.  The oracle scales and
+    rounds the queries as the kernel does, so what is left is the rounding of the 16-bit probabilities and outputs."""
+    from parrotserve_amd import kernels
+
+    T, parent, H, D = 300, 2000, 40, 128  # a query sees 2150 tokens on average
+    n = parent + T
+    assert prefill_plan([T] * 12, [n] * 12, H, D, dtype) == (256, 1)
+    g = torch.Generator().manual_seed(5)
+    sign = torch.where(torch.rand(D, generator=g) < 0.5, -1.0, 1.0)
+    q = (8.0 * sign).expand(T, H, D) + 0.05 * torch.randn(T, H, D, generator=g)
+    level = torch.zeros(n)
+    for at, value in sorted(rises.items()):
+        level[at:] = value
+    per_unit = 8.0 * D * D ** -0.5 * 1.4426950408889634      # exponent per unit of a key along `sign`
+    k = (level / per_unit)[:, None, None] * sign + 0.1 * torch.randn(n, H, D, generator=g)
+    q, k, v = q.to(dtype), k.to(dtype), torch.randn(n, H, D, generator=g).to(dtype)
+    scaled = (q.float() * (D ** -0.5 * 1.4426950408889634)).to(dtype).double().transpose(0, 1)
+    s = scaled @ k.double().permute(1, 2, 0).contiguous() * 0.6931471805599453
+    s.masked_fill_(torch.arange(n)[None, None, :] > parent + torch.arange(T)[None, :, None], -float("inf"))
+    ref = (torch.softmax(s, dim=-1) @ v.double().transpose(0, 1)).transpose(0, 1)
+    slots = list(range(n))
+    tables = kernels.PrefillTables.build([T] * 12, [slots] * 12, dev)
+    out = kernels.prefill_attention(q.repeat(12, 1, 1).to(dev), k.to(dev), v.to(dev), tables).cpu().double()
+    for c in range(12):
+        torch.testing.assert_close(out[c * T:(c + 1) * T], ref, **TOL[dtype])
+
+
+@pytest.mark.parametrize("bad", ["key nan", "key inf", "query nan", "value nan"])
+def test_prefill_whole_tiles_keep_non_finite_values(dev, bad):
+    """The same in one part per tile of 256 queries: NaN where plain fp32 attention has it, the others untouched."""
+    from parrotserve_amd import kernels
+
+    T, parent, H, D, head = 300, 2000, 40, 128, 1
+    n = parent + T
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(m, H, D, generator=g).half() for m in (T, n, n))
+    what, value = bad.split()
+    {"key": k, "value": v, "query": q}[what][T // 2 if what == "query" else 100, head, 5] = float(value)
+    qf, kf, vf = (x.float().transpose(0, 1).contiguous() for x in (q, k, v))
+    s = (qf @ kf.transpose(1, 2).contiguous()) * D ** -0.5
+    s.masked_fill_(torch.arange(n)[None, None, :] > parent + torch.arange(T)[None, :, None], -float("inf"))
+    ref = (torch.softmax(s, dim=-1) @ vf).transpose(0, 1)
+    assert prefill_plan([T] * 12, [n] * 12, H, D, torch.float16) == (256, 1)
+    tables = kernels.PrefillTables.build([T] * 12, [list(range(n))] * 12, dev)
+    out = kernels.prefill_attention(q.repeat(12, 1, 1).to(dev), k.to(dev), v.to(dev), tables).cpu().float()[:T]
+    assert ref.isnan().any() and out[ref.isnan()].isnan().all()
+    others = torch.arange(H) != head
+    torch.testing.assert_close(out[:, others], ref[:, others], **TOL[torch.float16])
