@@ -292,14 +292,6 @@ __device__ __forceinline__ void divide(float (&x)[N], float T, float r, bool by_
     for (int j = 0; j < N; ++j) x[j] = div_by<E>(x[j], T, r);
   }
 }
-// e^x: 2^n 2^f with n + f = x log2(e), the product carried in two floats; to the bit what expf returns (every float from
-// -110 to 1000 compared), two instructions shorter: nothing but +infinity needs the overflow case.
-__device__ __forceinline__ float exp_of(float x) {
-  constexpr float kHi = 0x1.715476p+0f, kLo = 0x1.4ae0bep-26f;  // log2(e)
-  const float hi = x * kHi, lo = __builtin_fmaf(x, kLo, __builtin_fmaf(x, kHi, -hi)), n = __builtin_rintf(hi);
-  const float y = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((hi - n) + lo), (int)n);
-  return x < -0x1.9d1da0p+6f ? 0.f : y;  // (an x of -infinity, too)
-}
 
 // Histograms of the mass over the bit pattern of e: 32 bins per power of two, then 8 bits inside the bin the mass
 // crosses its target in, then, where that finer bin holds more than one value, the last 10 bits.  Values of one coarse
@@ -421,7 +413,7 @@ __device__ __forceinline__ void find_in_level(SampHist& hist, const mass_t* leve
 // the cumulative sum of the draw -- take one batched reduction over the rounds to find the round in which the
 // count / the sum crosses, and one scan over the lanes inside that round.
 // Bound by vector issue on one compute unit per row and by a chain of ten reductions over the workgroup.  64 rows of
-// 32,000 logits, top-p 0.9, fp16 / fp32: 15.7 / 14.2 us.  It was 24.6 / 58 us with one round's load awaited before the
+// 32,000 logits, top-p 0.9, fp16 / fp32: 16.0 / 14.6 us.  It was 24.6 / 58 us with one round's load awaited before the
 // next was requested, reductions through LDS shuffles, the top-p cut always from three levels, equal values counted lane
 // by lane, the uniform number fetched at the draw, and fp32 rows in scratch memory; by bisection alone 37.7 us.  About
 // 31 thousand cycles now: load 5.3, quotients and maximum 3.2, exponentials and coarse bins 9.5, cut 8.2, draw 5.4.
@@ -593,18 +585,12 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
     for (int i = 0; i < kSampWaves; ++i) m = fmaxf(m, sh.red[par][i]);
     par ^= 1;
     if (!(m > -INFINITY && m < INFINITY)) m = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if (k >= rounds) break;
-#pragma unroll
-      for (int j = 0; j < N; ++j) e[k][j] = e[k][j] == INFINITY ? 1000.f : e[k][j];  // the same exponential
-    }
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     if (k >= rounds) break;
 #pragma unroll
-    for (int j = 0; j < N; ++j) e[k][j] = exp_of(e[k][j] - m);
+    for (int j = 0; j < N; ++j) e[k][j] = expf(e[k][j] - m);
     if (!by_bins) continue;
     // the most likely token has e == 1, every e is in [0, 1]
     // where all lanes hold the same value, one of them adds for all (rows of 16-bit logits like that are bisected)

@@ -262,6 +262,26 @@ def test_rows_without_a_finite_mass_take_the_general_rule(dtype):
     assert torch.equal(kernels.sample_top_p(x, temps, tops, u), kernels.sample_top_p(buf[:, 1:V + 1], temps, tops, u))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("value", [1e3, 1e10, 2.3e38, 2.4e38, 3e38, -3e38])
+def test_huge_logits_beside_an_infinite_one_take_the_general_rule(dtype, value):
+    """A row that holds +inf keeps its logits as they are (no maximum to subtract): the exponential of the largest finite
+    ones is +inf, not NaN, and the same token comes out as from the kernel for rows off the 16-byte grid."""
+    V = 2000
+    x = torch.full((4, V), -200.0)
+    x[:, 3], x[:, 1900] = float("inf"), value
+    x[1, 5] = float("nan")
+    x = x.to(DT[dtype]).cuda()
+    buf = torch.zeros(4, V + 8, dtype=x.dtype, device="cuda")
+    buf[:, 1:V + 1] = x
+    u = torch.tensor([0.5, 0.5, 0.0, 0.9]).cuda()
+    for temps, tops in ((None, None), (torch.full((4,), 0.7), torch.tensor([0.9, 0.5, 1.0, 0.3]))):
+        args = [t if t is None else t.cuda() for t in (temps, tops)]
+        ids = kernels.sample_top_p(x, *args, u)
+        assert torch.equal(ids, kernels.sample_top_p(buf[:, 1:V + 1], *args, u))
+        assert ids[0] == (1900 if value > 0 else 3)  # no running sum passes an infinite goal: the last token with mass
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("V", [4000, 32000])
 def test_rows_of_few_distinct_values(dtype, V):
