@@ -91,7 +91,11 @@ bool number(PyObject* o, double& v) {
   if (PyFloat_CheckExact(o)) v = PyFloat_AS_DOUBLE(o);
   else if (PyLong_CheckExact(o)) v = PyLong_AsDouble(o);
   else return false;
-  return !(v == -1.0 && PyErr_Occurred());
+  if (v == -1.0 && PyErr_Occurred()) {  // beyond a double: the Python body's to refuse
+    PyErr_Clear();
+    return false;
+  }
+  return true;
 }
 
 bool whole(PyObject* o, int64_t& v) {

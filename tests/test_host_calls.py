@@ -162,3 +162,19 @@ def test_an_error_of_the_library_is_the_wrappers(dev):
     _both(lambda: [kernels.fused_add_rms_norm(x, x.clone(), w, 1e-6)])
     with pytest.raises(RuntimeError, match="fused_add_rms_norm: unsupported data type"):
         kernels.fused_add_rms_norm(x, x.clone(), w, 1e-6)
+
+
+@pytest.mark.gpu
+def test_a_whole_number_beyond_a_double_is_refused_as_by_python(dev):
+    """``float()`` of it raises OverflowError; the C++ form leaves the call to the body that says so."""
+    huge = 10 ** 400
+    x, w = torch.ones(4, 64, device=dev, dtype=torch.float16), torch.ones(64, device=dev, dtype=torch.float16)
+    q, kc, vc = (torch.ones(n, 2, 128, device=dev, dtype=torch.float16) for n in (2, 40, 40))
+    tables = kernels.DecodeTables.build([], [], [[1, 2, 3], [4, 5]], dev, num_heads=2)
+    pre = kernels.PrefillTables.build([2], [[1, 2, 3]], dev)
+    for call in (lambda: kernels.vllm_rms_norm(x, w, huge), lambda: kernels.rmsnorm_forward(x, w, -huge),
+                 lambda: kernels.fused_add_rms_norm(x, x.clone(), w, huge),
+                 lambda: kernels.decode_attention(q, kc, vc, tables, scale=huge),
+                 lambda: kernels.prefill_attention(q, kc, vc, pre, scale=huge)):
+        with pytest.raises(OverflowError):
+            call()
