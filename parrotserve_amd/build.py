@@ -4,14 +4,18 @@ Run ``python -m parrotserve_amd.build`` or call ``build()``; the shared library
 lands next to the sources' package (parrotserve_amd/libparrot_hip.so) so it
 travels with the tree.  ``python -m parrotserve_amd.build --timeline`` also links the
 profiling variant (libparrot_hip_timeline.so, what ``bench.py --timeline`` loads).  The C++ form of the wrappers'
-plain calls (csrc/host_calls.cpp, no device code) is built against torch by g++ into ``_host.so`` beside it.
+plain calls (csrc/host_calls.cpp, no device code) is built against torch into ``_host.so`` beside it, by g++ or the clang
+behind hipcc; it needs the interpreter's headers, and the package runs without it (kernels._load_host).
 """
 from __future__ import annotations
 
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from typing import List
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
@@ -53,21 +57,32 @@ def _compile(src: str, obj_dir: str, timeline: bool = False) -> str:
     return obj
 
 
-def _build_host() -> None:
-    """csrc/host_calls.cpp, a CPython module over torch's C++ interface."""
-    import sysconfig
+def _host_compiler() -> List[str]:
+    """$CXX, g++, or where neither is there the clang behind hipcc, as a plain C++ compiler."""
+    cxx = os.environ.get("CXX") or shutil.which("g++")
+    return [cxx] if cxx else [HIPCC, "-x", "c++"]
 
+
+def _build_host() -> bool:
+    """csrc/host_calls.cpp, a CPython module over torch's C++ interface.  False: this interpreter's headers are not
+    installed; the package then runs without the module, and none of an earlier build is left to be loaded."""
     import torch
 
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        if os.path.exists(HOST_LIB_PATH):
+            os.remove(HOST_LIB_PATH)
+        return False
     root = os.path.dirname(torch.__file__)
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+    cmd = [*_host_compiler(), "-O2", "-std=c++17", "-fPIC", "-shared",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"), "-isystem",
+           "-I" + include, "-isystem", os.path.join(root, "include"), "-isystem",
            os.path.join(root, "include", "torch", "csrc", "api", "include"), os.path.join(CSRC, "host_calls.cpp"),
            "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", HOST_LIB_PATH]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"the build of host_calls.cpp failed:\n{r.stdout}\n{r.stderr}")
+    return True
 
 
 def build(verbose: bool = True, timeline: bool = False) -> str:
@@ -77,7 +92,8 @@ def build(verbose: bool = True, timeline: bool = False) -> str:
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as ex:
         host = ex.submit(_build_host)
         objs = list(ex.map(lambda s: _compile(s, obj_dir), SOURCES))
-        host.result()
+        if not host.result() and verbose:
+            print("no Python.h: _host.so is not built, the wrappers run in Python")
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

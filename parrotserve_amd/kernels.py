@@ -16,6 +16,7 @@ import collections
 import ctypes
 import dataclasses
 import functools
+import warnings
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -141,13 +142,25 @@ def _workspace(nbytes: int, device: torch.device, least: Optional[int] = None) -
 _host = None  # the C++ form of the plain calls (csrc/host_calls.cpp), bound at the first call
 
 
+class _TakesNothing:
+    """In place of ``_host.so`` where it is not built for this interpreter and this torch: every call is the Python body's."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _load_host():
     """Loads ``_host.so`` and gives it the library's addresses and what this module keeps.  Its functions return
     ``None`` for a call that is not of the plain form; the body behind such a call here decides about it."""
     global _host
-    from . import _host as host
-
     lib = _lib.load()
+    try:
+        from . import _host as host
+    except ImportError as e:
+        warnings.warn(f"parrotserve_amd/_host.so does not load ({e}): the wrappers run in Python, 4 to 8 us a call slower. "
+                      "Build it with `python -m parrotserve_amd.build`.", RuntimeWarning, stacklevel=3)
+        _host = _TakesNothing()
+        return _host
     host.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _lib.SIGNATURES},
               dict(check=check, raw_stream=_raw_stream or (lambda device: torch.cuda.current_stream().cuda_stream),
                    raw_device=_raw_device, capturing=torch.cuda.is_current_stream_capturing, workspaces=_workspaces,

@@ -1,21 +1,18 @@
 """The C++ form of the wrappers' plain calls (csrc/host_calls.cpp) against the Python bodies behind it: the same results
 to the bit where it takes a call, the Python body's own decision where it does not."""
 import contextlib
+import sys
 
 import pytest
 import torch
 
-from parrotserve_amd import kernels, mem
-
-
-class _TakesNothing:
-    def __getattr__(self, name):
-        return lambda *args: None
+import parrotserve_amd
+from parrotserve_amd import build, kernels, mem
 
 
 @contextlib.contextmanager
 def _python_only():
-    host, kernels._host = kernels._host, _TakesNothing()
+    host, kernels._host = kernels._host, kernels._TakesNothing()
     try:
         yield
     finally:
@@ -43,6 +40,32 @@ def test_what_is_not_plain_is_left_to_python():
                  lambda: kernels.fused_add_rms_norm(x, x, w, 1e-6)):
         with pytest.raises(RuntimeError, match="CPU tensor"):
             call()
+
+
+def test_without_the_module_the_python_bodies_serve(monkeypatch):
+    """_host.so is bound to one interpreter and one torch; where it does not load, a warning names the build command and
+    every call is the Python body's, as it was before there was such a module."""
+    monkeypatch.setattr(kernels, "_host", None)
+    monkeypatch.delattr(parrotserve_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "parrotserve_amd._host", None)  # the import fails
+    x, w = torch.zeros(2, 8, dtype=torch.float16), torch.zeros(8, dtype=torch.float16)
+    with pytest.warns(RuntimeWarning, match="python -m parrotserve_amd.build"):
+        with pytest.raises(RuntimeError, match="CPU tensor"):
+            kernels.vllm_rms_norm(x, w, 1e-6)
+    assert kernels._host.decode_attention(x, x, x, None, None, None, 0) is None
+    with pytest.raises(RuntimeError, match="CPU tensor"):
+        kernels.silu_mul(x, x)
+
+
+def test_the_module_is_built_without_gcc_and_left_out_without_headers(monkeypatch, tmp_path):
+    monkeypatch.delenv("CXX", raising=False)
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    assert build._host_compiler() == [build.HIPCC, "-x", "c++"]
+    stale = tmp_path / "_host.so"
+    stale.write_bytes(b"of an earlier build")
+    monkeypatch.setattr(build, "HOST_LIB_PATH", str(stale))
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build._build_host() is False and not stale.exists()
 
 
 def _both(call):
