@@ -1167,7 +1167,6 @@ extern "C" int ph_prefill_attention(void* out, const void* q, const void* k_cach
     const PrefillPlan pp =
         plan_prefill(num_tokens, num_chunks, num_heads, head_dim, max_kv_len, ctx_slots_count, workspace_bytes);
     pa.n_splits = pp.splits;
-    pa.mean_visible = (ctx_slots_count - num_tokens / 2) / num_chunks;
     if (pp.splits > 1) {
       pa.opart = (float*)workspace;
       pa.ml = (float*)((char*)workspace + round_up((int64_t)pp.splits * T * H * D * 4, 256));

@@ -152,7 +152,6 @@ struct PrefillArgs {
   int n_splits;              // > 1: every tile's visible tokens are cut into this many parts,
   float* opart;              //      [n_splits][num_tokens][H] rows of head_dim (paired: 64) floats
   float* ml;                 //      and (m, l) each, folded by fold_parts_kernel
-  int64_t mean_visible;      // tokens a query sees, on average over the call (an estimate: it chooses a kernel)
 };
 
 // The parts of a split prefill and where their fold goes (16-bit elements).

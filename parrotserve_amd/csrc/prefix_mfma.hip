@@ -576,9 +576,9 @@ __device__ __forceinline__ void attn_tile8(const TileWork& wk, const uint16_t* _
   // sub-tile's scores to run under the exponentials of the other's, and P.V of the one under the exponentials of the
   // other (the maximum of both stood between them before).
   // 8192 tokens, 40 heads: 684 -> 666 us, 4 % fewer cycles at a clock 1 % lower; 16 chunks over 2048 tokens 545 -> 536.
-  // (256 requests over 8192 tokens 81.0 -> 80.9: the decode kernels, whose units are short, keep the maximum.)  Measured against this form and not kept: P.V behind both sub-tiles'
-  // exponentials (740), the two waves of a SIMD half a step apart with a barrier every half step (748 against 720 before
-  // and 702), one barrier for two steps (679 against 664).
+  // (256 requests over 8192 tokens 81.0 -> 80.9: the decode kernels, whose units are short, keep the maximum.)  Measured
+  // against this form and not kept: P.V behind both sub-tiles' exponentials (740), the two waves of a SIMD half a step
+  // apart with a barrier every half step (748 against 720 before and 702), one barrier for two steps (679 against 664).
   static_assert(!SUMS || (PRESC && SUB == 2 && TQ == 1), "the sums stand for a maximum in the pre-scaled 256-query form");
   constexpr uint32_t kSumLimitBits = 0x45800000u;  // 2^12, where a lane sums sixteen exponentials
   // HALF: a 64-wide head as half wk.pair_half (0 / 1) of a head pair -- only that half's two 32-dim blocks of the
@@ -1445,14 +1445,31 @@ __device__ __forceinline__ void prefill_tile8(const PrefillArgs& a, const Prefil
 // covers the tile rows from a.tile_row0 on (more rows than a grid's y extent holds take several launches; a loop
 // over rows inside the kernel cost the common single-launch case 6 %), grid.z the splits
 // HALF (64-wide heads, 256-query tiles): only this head's half of the pair's output is computed
-template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false, bool SUMS = false>
+//
+// A whole 256-query tile takes the form without maxima where all its queries see kSumsFrom tokens or more: the first
+// step and those on the diagonal multiply their scores twice in that form, so a tile of few steps is faster with the
+// maximum.  The tile decides, from its own chunk, because chunks of one call differ and the host does not know their
+// lengths (by the call's mean over chunks one Fill of 8192 tokens beside eight of 300 took 667 us in place of 648).
+// In us by where the line lies, 768 / 1024 / 1280 / 1536 / 1792 / 2048 tokens / nowhere (bf16): 16 chunks of 400 to 600
+// over 1000 306 / 303 / 302 / 310 / 307 / 312 / 310; 16 of 300 to 600 over 1500 344 / 347 / 343 / 345 / 351 / 354 / 355;
+// 8 of 1000 over 1200 257 / 260 / 259 / 260 / 259 / 263 / 264; one of 2048 59.6 / 59.4 / 59.4 / 59.2 / 59.0 / 60.6 / 60.6;
+// 4 of 400 to 1200 over 776 116.0 / 116.3 / 115.2 / 116.1 / 115.3 / 116.1 / 115.6; 3 of 600 over 40, with the line at 0,
+// 42.5 and 39.9 from 768 on.  (Runs differ by 0.5 to 1 %.)  Both loops in one kernel need the registers of the larger,
+// 256 and none spilled, and cost a call that takes one of them nothing that shows (115.2 / 115.6, 310 / 311, 619 / 619).
+constexpr int kSumsFrom = 1280;
+
+template <typename E, int TQ, int SUB, bool HALF = false, bool SPLIT = false>
 __global__ __launch_bounds__(512) void prefill_mfma8_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   PH_TL(0);
   if ((int)blockIdx.x >= a.H) return;
   PrefillTile pt;
   if (!find_prefill_tile(a, a.tile_row0 + (int)blockIdx.y, 32 * (8 / TQ), pt)) return;
-  prefill_tile8<E, TQ, SUB, HALF, SPLIT, SUMS>(a, pt, blockIdx.z, smem);
+  constexpr bool WHOLE256 = TQ == 1 && SUB == 2 && !HALF && !SPLIT;
+  if (WHOLE256 && pt.kvn - pt.n + 256 * pt.tile >= kSumsFrom)
+    prefill_tile8<E, TQ, SUB, HALF, SPLIT, WHOLE256>(a, pt, blockIdx.z, smem);
+  else
+    prefill_tile8<E, TQ, SUB, HALF, SPLIT, false>(a, pt, blockIdx.z, smem);
   PH_TL(11);
 }
 
@@ -1490,7 +1507,7 @@ static int launch_prefix_t(const PrefixArgs& a, int num_groups, int max_group_re
 
 constexpr int64_t kMaxGridY = 65535;  // grid extent in y and z
 
-template <typename E, int TQ, int SUB, bool HALF, bool SPLIT, bool SUMS = false>
+template <typename E, int TQ, int SUB, bool HALF, bool SPLIT>
 static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
   constexpr int QT = 32 * (8 / TQ);  // queries per workgroup tile
   if (a.tile_cu) {
@@ -1498,7 +1515,7 @@ static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
     const int rc = launch_status();
     if (rc != PH_OK) return rc;
   }
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT, SUMS>),
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, kTile8Lds);
   const int hx = (a.H + 7) / 8 * 8;  // keeps head == linear id mod 8 for every tile row
   const int64_t max_tiles = (a.num_tokens - a.num_chunks) / QT + a.num_chunks;  // >= sum of ceil(n_c / QT), n_c >= 1
@@ -1506,7 +1523,7 @@ static int launch_prefill_tq(const PrefillArgs& a, hipStream_t st) {
     PrefillArgs part = a;
     part.tile_row0 = (int)row0;
     const int64_t rows = max_tiles - row0 < kMaxGridY ? max_tiles - row0 : kMaxGridY;
-    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT, SUMS>), dim3(hx, (unsigned)rows, SPLIT ? a.n_splits : 1),
+    hipLaunchKernelGGL((prefill_mfma8_kernel<E, TQ, SUB, HALF, SPLIT>), dim3(hx, (unsigned)rows, SPLIT ? a.n_splits : 1),
                        dim3(512), kTile8Lds, st, part);
   }
   return launch_status();
@@ -1521,14 +1538,6 @@ static int launch_prefill_sq(const PrefillArgs& a, hipStream_t st) {
 template <typename E>
 static int launch_prefill_t(const PrefillArgs& a, int tile_q, hipStream_t st) {
   if (tile_q == 256 && a.pair) return launch_prefill_sq<E, 1, 2, true>(a, st);
-  // The first step of a tile and those on its diagonal multiply their scores twice in the form without maxima, so tiles of
-  // few steps keep the other one.  In us, without / with, by the tokens a query sees on average: 3 chunks of 600 over 40
-  // (340) 39.7 / 41.2; 2 of 200 to 740 (240) 22.9 / 23.5; 4 of 400 to 1200 over 776 (1180) 123 / 127; 16 of 400 to 600
-  // over 1000 (1250) 286 / 290; 13 of 200 to 1900 over 989 (1510) 502 / 498; 16 of 64 to 1024 over 2048 (2340) 545 / 535;
-  // one of 8000 (4000) 679 / 655.
-  constexpr int kLongContext = 2048;
-  if (tile_q == 256 && a.n_splits <= 1 && a.mean_visible >= kLongContext)
-    return launch_prefill_tq<E, 1, 2, false, false, true>(a, st);
   if (tile_q == 256) return launch_prefill_sq<E, 1, 2>(a, st);  // 64-token steps (measured 4 % faster)
   if (tile_q == 128) return launch_prefill_sq<E, 2, 1>(a, st);
   return launch_prefill_sq<E, 4, 1>(a, st);

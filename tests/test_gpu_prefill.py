@@ -1,6 +1,7 @@
 """GPU parity of prefill-with-parent-context (packed ragged chunks, bottom-right
 causal over scattered parent slots) against the CPU oracle."""
 import ctypes
+import dataclasses
 
 import pytest
 import torch
@@ -476,3 +477,43 @@ def test_prefill_whole_tiles_keep_non_finite_values(dev, bad):
     assert ref.isnan().any() and out[ref.isnan()].isnan().all()
     others = torch.arange(H) != head
     torch.testing.assert_close(out[:, others], ref[:, others], **TOL[torch.float16])
+
+
+def _random_prefill(dev, q_lens, parents, H=40, D=128):
+    from parrotserve_amd import kernels
+
+    g = torch.Generator().manual_seed(11)
+    ctx = [n + p for n, p in zip(q_lens, parents)]
+    q, k, v = (torch.randn(n, H, D, generator=g).half().to(dev) for n in (sum(q_lens), sum(ctx), sum(ctx)))
+    slots = torch.randperm(sum(ctx), generator=g).tolist()
+    lists = [slots[sum(ctx[:c]):sum(ctx[:c + 1])] for c in range(len(ctx))]
+    return q, k, v, lists, kernels.PrefillTables.build(q_lens, lists, dev)
+
+
+def test_a_longer_slot_list_does_not_change_the_kernel(dev):
+    """The slot list may be longer than the contexts (a buffer kept for the largest call): to the bit the same result."""
+    from parrotserve_amd import kernels
+
+    assert prefill_plan([600] * 3, [640] * 3, 40, 128, torch.float16) == (256, 1)
+    q, k, v, _, tables = _random_prefill(dev, [600] * 3, [40] * 3)
+    out = kernels.prefill_attention(q, k, v, tables)
+    room = torch.zeros(15000, dtype=torch.int32, device=dev)
+    longer = dataclasses.replace(tables, ctx_slots=torch.cat([tables.ctx_slots, room]))
+    assert torch.equal(kernels.prefill_attention(q, k, v, longer), out)
+
+
+def test_a_chunk_takes_the_kernel_form_of_its_own_length(dev):
+    """Chunks over long contexts beside more of them without any, and the other way round: to the bit what each gives in
+    a call of its own kind (the form of the tile loop follows from the tile, not from the call's mean)."""
+    from parrotserve_amd import kernels
+
+    long, short = [(300, 2000)] * 12, [(300, 0)] * 24
+    for chunks in (long, short, long + short):
+        q_lens = [n for n, _ in chunks]
+        assert prefill_plan(q_lens, [n + p for n, p in chunks], 40, 128, torch.float16) == (256, 1)
+    q, k, v, lists, tables = _random_prefill(dev, [300] * 36, [2000] * 12 + [0] * 24)
+    together = kernels.prefill_attention(q, k, v, tables)
+    for first, last in ((0, 12), (12, 36)):
+        part = kernels.PrefillTables.build([300] * (last - first), lists[first:last], dev)
+        rows = slice(300 * first, 300 * last)
+        assert torch.equal(kernels.prefill_attention(q[rows], k, v, part), together[rows])
