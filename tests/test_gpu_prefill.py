@@ -456,27 +456,63 @@ def test_prefill_scores_that_outgrow_the_exponent_reference(dev, rises, dtype):
         torch.testing.assert_close(out[c * T:(c + 1) * T], ref, **TOL[dtype])
 
 
-@pytest.mark.parametrize("bad", ["key nan", "key inf", "query nan", "value nan"])
-def test_prefill_whole_tiles_keep_non_finite_values(dev, bad):
-    """The same in one part per tile of 256 queries: NaN where plain fp32 attention has it, the others untouched."""
+@pytest.mark.parametrize("D,dtype", [(80, torch.float16), (96, torch.bfloat16), (112, torch.float16), (128, torch.float16),
+                                     (128, torch.bfloat16)])
+@pytest.mark.parametrize("rises", [
+    {0: 0.0, 1920: 13.0, 1952: 26.0, 1984: 39.0, 2016: 52.0},  # in the last whole steps of the waves whose diagonal follows
+    {0: 0.0, 1300: 12.5, 1345: 25.0, 1440: 38.0, 1499: 60.0},  # as far as the last token, across the tiles' forms
+    {0: 0.0, 1408: 50.0, 1409: 0.0, 2005: 30.0},               # one token far above all others, one inside the diagonal
+])
+def test_prefill_outgrown_references_in_unequal_chunks_and_short_heads(dev, rises, D, dtype):
+    """The same over chunks of different lengths and contexts, without a parent (tiles of both forms in one chunk), with a
+    tile of a few queries, and with heads shorter than the tile's 128 dims."""
+    from parrotserve_amd import kernels
+
+    q_lens, parents, H, heads = [300, 1500, 40, 777], [2000, 0, 2000, 1300], 40, [0, 17, 39]
+    ctx = [n + p for n, p in zip(q_lens, parents)]
+    assert prefill_plan(q_lens, ctx, H, D, dtype) == (256, 1)
+    g = torch.Generator().manual_seed(6)
+    sign = torch.where(torch.rand(D, generator=g) < 0.5, -1.0, 1.0)
+    q = ((8.0 * sign).expand(sum(q_lens), H, D) + 0.05 * torch.randn(sum(q_lens), H, D, generator=g)).to(dtype)
+    level = torch.zeros(max(ctx))
+    for at, value in sorted(rises.items()):
+        level[at:] = value
+    per_unit = 8.0 * D * D ** -0.5 * 1.4426950408889634
+    k = torch.cat([(level[:n] / per_unit)[:, None, None] * sign for n in ctx]) + 0.1 * torch.randn(sum(ctx), H, D, generator=g)
+    k, v = k.to(dtype), torch.randn(sum(ctx), H, D, generator=g).to(dtype)
+    tables = kernels.PrefillTables.build(q_lens, [list(range(sum(ctx[:c]), sum(ctx[:c + 1]))) for c in range(4)], dev)
+    out = kernels.prefill_attention(q.to(dev), k.to(dev), v.to(dev), tables).cpu()[:, heads].double()
+    scaled = (q[:, heads].float() * (D ** -0.5 * 1.4426950408889634)).to(dtype).double().transpose(0, 1)
+    for c, (n, p) in enumerate(zip(q_lens, parents)):
+        rows, keys = slice(sum(q_lens[:c]), sum(q_lens[:c + 1])), slice(sum(ctx[:c]), sum(ctx[:c + 1]))
+        s = scaled[:, rows] @ k[keys][:, heads].double().permute(1, 2, 0).contiguous() * 0.6931471805599453
+        s.masked_fill_(torch.arange(n + p)[None, None, :] > p + torch.arange(n)[None, :, None], -float("inf"))
+        ref = (torch.softmax(s, dim=-1) @ v[keys][:, heads].double().transpose(0, 1)).transpose(0, 1)
+        torch.testing.assert_close(out[rows], ref, **TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bad", ["key nan", "key inf", "query nan", "query inf", "value nan"])
+def test_prefill_whole_tiles_keep_non_finite_values(dev, bad, dtype):
+    """The same in one part per tile of 256 queries: NaN where plain fp32 attention has it and there alone, in the head
+    that holds it and in the others."""
     from parrotserve_amd import kernels
 
     T, parent, H, D, head = 300, 2000, 40, 128, 1
     n = parent + T
     g = torch.Generator().manual_seed(9)
-    q, k, v = (torch.randn(m, H, D, generator=g).half() for m in (T, n, n))
+    q, k, v = (torch.randn(m, H, D, generator=g).to(dtype) for m in (T, n, n))
     what, value = bad.split()
     {"key": k, "value": v, "query": q}[what][T // 2 if what == "query" else 100, head, 5] = float(value)
     qf, kf, vf = (x.float().transpose(0, 1).contiguous() for x in (q, k, v))
     s = (qf @ kf.transpose(1, 2).contiguous()) * D ** -0.5
     s.masked_fill_(torch.arange(n)[None, None, :] > parent + torch.arange(T)[None, :, None], -float("inf"))
     ref = (torch.softmax(s, dim=-1) @ vf).transpose(0, 1)
-    assert prefill_plan([T] * 12, [n] * 12, H, D, torch.float16) == (256, 1)
+    assert prefill_plan([T] * 12, [n] * 12, H, D, dtype) == (256, 1)
     tables = kernels.PrefillTables.build([T] * 12, [list(range(n))] * 12, dev)
     out = kernels.prefill_attention(q.repeat(12, 1, 1).to(dev), k.to(dev), v.to(dev), tables).cpu().float()[:T]
-    assert ref.isnan().any() and out[ref.isnan()].isnan().all()
-    others = torch.arange(H) != head
-    torch.testing.assert_close(out[:, others], ref[:, others], **TOL[torch.float16])
+    assert ref.isnan().any() and torch.equal(out.isnan(), ref.isnan())
+    torch.testing.assert_close(out, ref, equal_nan=True, **TOL[dtype])
 
 
 def _random_prefill(dev, q_lens, parents, H=40, D=128):

@@ -331,7 +331,8 @@ def test_row_lengths_around_the_rounds_and_forms_of_the_register_kernel(dtype, V
     """No whole chunk, a last chunk of one token and of all but one, a round that is full and one that holds a single
     chunk, the longest row of the 32-token form and the shortest of the other; rows start on the 16-byte grid whatever
     their length.  Values in steps of 1/4 (several equal ones at every cut, ranked over rounds and waves), and values so
-    close that the finer bin in question holds several, so that its last bits decide."""
+    close that the finer bin in question holds several, so that its last bits decide (in 32-bit rows: 16-bit rows this
+    close are bisected)."""
     B = 6
     pad = -V % 8 + 8
     x, temps, tops, u = _case(V, B, V, dtype, quantum=0.25)
@@ -341,3 +342,35 @@ def test_row_lengths_around_the_rounds_and_forms_of_the_register_kernel(dtype, V
     # than 2^-23 may share one, and the kernel ranks equal exponentials by id
     close = ((torch.rand(B, V, generator=g) * 1024).floor() * 2.0 ** -22).to(DT[dtype])
     _check(close, torch.ones(B), torch.tensor([0.9003, 0.3007, 0.6002] * 2), u, dtype, min_compared=0.3, stride_pad=pad)
+
+
+def _histogram_levels(x, p, chunk):
+    """What the register kernel's histograms meet on these rows, from fp32 exponentials: the share of equal and of nearly
+    equal values it would look at, and how many values the finer bin holds that the mass crosses `p` in."""
+    out = []
+    for row, top in zip(x.float().numpy(), p.numpy()):
+        first = row[::chunk][: len(row) // chunk // 64 * 64].reshape(-1, 64)
+        share = ((np.abs(first - first[:, :1]) < 0.011).sum() + 2 * (first == first[:, :1]).sum()) / first.size
+        e = np.sort(np.exp(row - row.max()))[::-1]
+        at = np.searchsorted(np.cumsum(e, dtype=np.float64), top * e.sum(dtype=np.float64))
+        bins = e.view(np.uint32) >> 10
+        out.append((share, len(np.unique(e[bins == bins[min(at, len(e) - 1)]]))))
+    return out
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("V", [8191, 32000, 32769])
+def test_last_bits_of_the_cut_in_16_bit_rows(dtype, V):
+    """16-bit rows that go through the histograms and whose cut falls among values so close that the finer bin holds
+    several: the first token of every 16-byte chunk, which is where the kernel looks for few distinct values, spreads over
+    31 units, the others lie in steps of 2^-22 (fp16) and 2^-20 (bf16) one unit below the maximum."""
+    B, step = 6, 2.0 ** (-22 if dtype == "f16" else -20)
+    g = torch.Generator().manual_seed(V)
+    x = (torch.rand(B, V, generator=g) * 128).floor() * step
+    x[:, ::8] = torch.rand(B, x[:, ::8].shape[1], generator=g) * 31 - 30
+    x[:, 0] = 1.0
+    x = x.to(DT[dtype])
+    tops = torch.tensor([0.9003, 0.3007, 0.6002] * 2)
+    for share, values in _histogram_levels(x, tops, 8):
+        assert share < 0.5 and values > 1
+    _check(x, torch.ones(B), tops, torch.rand(B, generator=g), dtype, min_compared=0.3, stride_pad=-V % 8 + 8)

@@ -1,5 +1,5 @@
-"""The C++ form of the wrappers' plain calls (csrc/host_calls.cpp) against the Python bodies behind it: the same results
-to the bit where it takes a call, the Python body's own decision where it does not."""
+"""The C++ form of the wrappers' plain calls (csrc/host_calls.cpp) against the Python bodies behind it: which calls it
+takes, the same results to the bit where it does, the Python body's own decision where it does not."""
 import contextlib
 import sys
 
@@ -68,15 +68,44 @@ def test_the_module_is_built_without_gcc_and_left_out_without_headers(monkeypatc
     assert build._build_host() is False and not stale.exists()
 
 
-def _both(call):
-    """The call's outputs (or the class of what it raised) with the C++ form and without."""
+class _Recorder:
+    """The C++ form with a note of every call: taken (it returned a result or raised), or left to Python (None)."""
+
+    def __init__(self, host):
+        self.host, self.taken = host, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.taken.append(True)
+            out = getattr(self.host, name)(*args)
+            self.taken[-1] = out is not None
+            return out
+        return call
+
+
+@contextlib.contextmanager
+def _recording():
+    host = kernels._host or kernels._load_host()
+    assert host.__name__ == "parrotserve_amd._host"
+    kernels._host = _Recorder(host)
+    try:
+        yield kernels._host
+    finally:
+        kernels._host = host
+
+
+def _both(call, takes):
+    """The call's outputs (or the class of what it raised) with the C++ form and without; ``takes``: the C++ form takes
+    the call, and does not leave it to Python."""
     seen = []
-    for ctx in (contextlib.nullcontext(), _python_only()):
-        with ctx:
+    for ctx in (_recording(), _python_only()):
+        with ctx as recorder:
             try:
                 out = call()
             except Exception as e:  # noqa: BLE001 -- what is compared is the class
                 out = type(e)
+            if recorder:
+                assert recorder.taken == [takes]
         seen.append(out)
     a, b = seen
     if isinstance(a, type) or isinstance(b, type):
@@ -112,19 +141,20 @@ def test_rows_through_both(dev, form):
         w = f(w)
     t, p, u = (torch.full((40,), v, device=dev) for v in (0.8, 0.9, 0.37))
     n = f(x).shape[0]
-    _both(lambda: [kernels.vllm_rms_norm(f(x), w, 1e-6)])
-    _both(lambda: [kernels.rmsnorm_forward(f(x), w, 1)])
-    _both(lambda: [kernels.silu_mul(f(x), f(up))])
-    _both(lambda: [kernels.silu_mul(f(x), up)])
-    _both(lambda: [kernels.sample_top_p(f(x), t[:n], p[:n], u[:n])])
-    _both(lambda: [kernels.sample_top_p(f(x), None, None, u)])
+    plain = form in ("plain", "columns", "one_row", "float", "grad")
+    _both(lambda: [kernels.vllm_rms_norm(f(x), w, 1e-6)], plain)
+    _both(lambda: [kernels.rmsnorm_forward(f(x), w, 1)], plain)
+    _both(lambda: [kernels.silu_mul(f(x), f(up))], plain)
+    _both(lambda: [kernels.silu_mul(f(x), up)], plain and form not in ("one_row", "float"))
+    _both(lambda: [kernels.sample_top_p(f(x), t[:n], p[:n], u[:n])], plain)
+    _both(lambda: [kernels.sample_top_p(f(x), None, None, u)], plain and form != "one_row")
 
     def add():
         res = f(r.clone())
         return [kernels.fused_add_rms_norm(f(x), res, w, 1e-6), res.detach()]
 
     if form != "grad":  # (a leaf that takes a gradient is refused by neither and written by both)
-        _both(add)
+        _both(add, plain)
 
 
 @pytest.mark.gpu
@@ -146,7 +176,7 @@ def test_rope_through_both(dev, form):
                                slots[:5] if form == "short_slots" else slots)
         return [q.contiguous(), k.contiguous(), kc, vc]
 
-    _both(call)
+    _both(call, form in ("plain", "chunks", "int64_slots"))
 
 
 @pytest.mark.gpu
@@ -170,19 +200,20 @@ def test_attention_through_both(dev, form):
     heads = {} if G == H else dict(head_mapping=torch.arange(G, dtype=torch.int32, device=dev).repeat_interleave(H // G),
                                    kv_group=H // G)
     scale = 0.05 if form == "scale" else None
-    _both(lambda: [kernels.decode_attention(q, kc, vc, tables, scale=scale, **heads)])
+    plain = not form.startswith("wrong")
+    _both(lambda: [kernels.decode_attention(q, kc, vc, tables, scale=scale, **heads)], plain)
     if form == "grouped":
         return
     new = [4, 1]
     pre = kernels.PrefillTables.build(new, [slots[:60], slots[60:61]], dev)
-    _both(lambda: [kernels.prefill_attention(q, kc, vc, pre, scale=scale)])
+    _both(lambda: [kernels.prefill_attention(q, kc, vc, pre, scale=scale)], plain)
 
 
 @pytest.mark.gpu
 def test_an_error_of_the_library_is_the_wrappers(dev):
     x = torch.zeros(4, 12, device=dev, dtype=torch.float32)  # no norm-and-add of 32-bit elements
     w = torch.zeros(12, device=dev, dtype=torch.float32)
-    _both(lambda: [kernels.fused_add_rms_norm(x, x.clone(), w, 1e-6)])
+    _both(lambda: [kernels.fused_add_rms_norm(x, x.clone(), w, 1e-6)], True)
     with pytest.raises(RuntimeError, match="fused_add_rms_norm: unsupported data type"):
         kernels.fused_add_rms_norm(x, x.clone(), w, 1e-6)
 
