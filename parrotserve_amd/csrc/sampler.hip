@@ -734,7 +734,17 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
       thr = e_hi;
       if (!(e_lo >= e_hi)) {
         uint32_t lo = to_key<SH>(-INFINITY), hi = to_key<SH>(m);
-        g_hi = 0.f;
+        if (e_lo > 0x1p-100f) {
+          // between the logits of the two values the looks leave, to within what expf (of a number that is not subnormal),
+          // logf and their sums can be off: 2e-7 of every term.  From the type's whole range such rows took 1 to 5 %
+          // longer than without the looks.  64 rows of 32,000 fp16 logits, whole range / between: nearly flat about zero,
+          // where most patterns lie, 38.3 / 37.6 us, four values 38.7 / 38.0, normal logits cut off above zero 36.4 / 29.7.
+          const float a = logf(e_lo), slack = 1e-6f * (1.f + __builtin_fabsf(m) - a);
+          lo = max(lo, to_key<SH>(m + a - slack));
+          hi = min(hi, to_key<SH>(m + logf(e_hi) + slack) + 1);
+        } else {
+          g_hi = 0.f;
+        }
         while (lo < hi) {  // lo, hi and g are the same in every lane
           const uint32_t mid = lo + ((hi - lo) >> 1);
           const float cut = expf(from_key<SH>(mid) - m);

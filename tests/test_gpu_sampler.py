@@ -374,3 +374,23 @@ def test_last_bits_of_the_cut_in_16_bit_rows(dtype, V):
     for share, values in _histogram_levels(x, tops, 8):
         assert share < 0.5 and values > 1
     _check(x, torch.ones(B), tops, torch.rand(B, generator=g), dtype, min_compared=0.3, stride_pad=-V % 8 + 8)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("at", [0.0, 1e-3, 0.9, 50.0, -300.0, 2000.0, 6e4])
+def test_rows_bisected_between_the_values_two_looks_leave(dtype, at):
+    """16-bit rows of so few distinct values, or so close ones, that their cut is bisected, and of more than the two looks
+    at halfway cuts resolve: neighbouring values of the type around small, large and negative logits (subnormal
+    exponentials among them), and nearly flat rows across zero."""
+    V, B = 4000, 12
+    g = torch.Generator().manual_seed(int(abs(at)) + 41)
+    top = torch.tensor(at).to(DT[dtype])
+    bits = top.view(torch.int16).to(torch.int32)
+    steps = (torch.rand(B // 2, V, generator=g) * torch.tensor([4.0, 5.0, 4.0, 5.0, 4.0, 5.0])[:, None]).floor()
+    near = (bits - steps if at >= 0 else bits + steps).to(torch.int16).view(DT[dtype]).float()
+    if at == 0.0:
+        near = steps * -(2.0 ** -10)
+    x = torch.cat([near, at + torch.randn(B // 2, V, generator=g) * 4e-3]).to(DT[dtype])
+    tops = torch.tensor([0.9003, 0.3007, 0.6002, 0.9701])[torch.arange(B) % 4]
+    temps = torch.tensor([1.0, 1.0, 0.7 if at < 6e4 else 1.0])[torch.arange(B) % 3]
+    _check(x, temps, tops, torch.rand(B, generator=g), dtype, min_compared=0.5)
