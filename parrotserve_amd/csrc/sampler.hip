@@ -416,7 +416,8 @@ __device__ __forceinline__ void find_in_level(SampHist& hist, const mass_t* leve
 // 32,000 logits, top-p 0.9, fp16 / fp32: 16.0 / 14.6 us.  It was 24.6 / 58 us with one round's load awaited before the
 // next was requested, reductions through LDS shuffles, the top-p cut always from three levels, equal values counted lane
 // by lane, the uniform number fetched at the draw, and fp32 rows in scratch memory; by bisection alone 37.7 us.  About
-// 31 thousand cycles now: load 5.3, quotients and maximum 3.2, exponentials and coarse bins 9.5, cut 8.2, draw 5.4.
+// 29 thousand cycles in fp16, read between the phases, whose loads and LDS adds may end in the next one: request 2.4,
+// quotients and maximum 5.7, exponentials and coarse bins 4.1, cut 11.3, draw 5.6.
 // FLOATS: tokens a lane holds, 32 or kSampRegFloats: the passes are unrolled over them (rows of up to 32,768 tokens
 // fetch three fifths of the instructions).
 constexpr int kSampRegFloats = 56;
@@ -535,11 +536,11 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(const SampArg
   // Adds of a wave to one address are taken one lane after the other, so a row of few distinct values (equal logits, a
   // high temperature) makes the histograms slow.  Every wave compares one token per chunk with lane 0's: the share in its
   // bin (by distance, half a bin's width) and twice the share of its value.  From one half on the row goes to the
-  // bisection, whose time hardly depends on the values.  64 rows of 32,000 fp16 logits, histograms and bisection: all
-  // equal 120 and 15.4 us, two values at random 69 and 17.7, four 43.2 and 37.3, five 39.3 and 38.9, normal logits of
-  // deviation 0.005 43.4 and 38.3; eight values (share 0.38) 30.9 and 36.9, deviation 0.02 29.3 and 38.7, deviation 4 15.4
-  // and 34 (15.6 with the look).  32-bit logits take the histograms whatever they hold: all equal 99 us against 16, but
-  // from four values on 44 against 50, deviation 4 14.1 against 48.
+  // bisection.  64 rows of 32,000 fp16 logits, histograms and bisection: all equal 119 and 15.8 us, two values at random
+  // 68 and 17, four 43.8 and 38.0, five 37.4 and 36.9, normal logits of deviation 0.005 44.5 and 37.3; eight values (share
+  // 0.38) 30.7 and 37.2, deviation 0.02 29.1 and 37.1, deviation 4 15.8 and 35.2 (16.0 with the look).  32-bit logits take
+  // the histograms whatever they hold: all equal 99.6 us against 17, but from four values on 45 against 52, deviation 4
+  // 14.6 against 48.
   constexpr bool kLooks = Logit<E>::kBytes == 2;
   constexpr float kNoMass = 41.5f;  // this far below the maximum a token is no mass (kHistLeast)
   if (kLooks && filter) {
